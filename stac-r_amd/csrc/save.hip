@@ -28,9 +28,11 @@ constexpr int kCandCap = 2048;               // candidates a workgroup keeps
 constexpr int kCandPer = kCandCap / kBlock;  // candidates a thread reads (consecutive)
 static_assert(kCandPer == 8, "one 16-byte vector of bf16 candidate values per thread");
 
+constexpr int kListCap = 4096;  // candidates a projection workgroup's list holds
+
 struct CandMeta {
     uint32_t cut;    // level-0 bin of the workgroup's cut
-    uint32_t count;  // candidates (more than kCandCap: the list overflowed and is not used)
+    uint32_t count;  // candidates (more than the list holds: it overflowed and is not used)
 };
 
 __device__ __forceinline__ void wg_rows(const SaveGeom &g, int64_t wg, int64_t &chunk, int64_t &row0,
@@ -960,7 +962,8 @@ __global__ __launch_bounds__(kBlock) void k_proj_hist_b(SaveGeom g, FastGeom fg,
     if (threadIdx.x < kCoarse) {  // the same counts in 64 bins of 32
         uint32_t sum = 0u;
 #pragma unroll 8
-        for (int b = 0; b < kBins / kCoarse; ++b) sum += s_hist[threadIdx.x * (kBins / kCoarse) + b];
+        for (int b = 0; b < kBins / kCoarse; ++b)
+            sum += s_hist[threadIdx.x * (kBins / kCoarse) + ((b + threadIdx.x) & (kBins / kCoarse - 1))];
         if (sum) atomicAdd(&coarse[(chunk * g.hcopies + copy) * kCoarse + threadIdx.x], sum);
     }
     if (threadIdx.x == 0) {
@@ -1196,7 +1199,7 @@ __global__ __launch_bounds__(NT) void k_proj_hist_w(SaveGeom g, int c_vec, const
     if (u < kCoarse) {
         uint32_t sum = 0u;
 #pragma unroll 8
-        for (int b = 0; b < kBins / kCoarse; ++b) sum += s_hist[u * (kBins / kCoarse) + b];
+        for (int b = 0; b < kBins / kCoarse; ++b) sum += s_hist[u * (kBins / kCoarse) + ((b + u) & (kBins / kCoarse - 1))];
         if (sum) atomicAdd(&coarse[(chunk * g.hcopies + copy) * kCoarse + u], sum);
     }
     if (u == 0) {
@@ -1703,7 +1706,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
 // at or above the cut where the workgroup's own count from the top reaches a quota (several times
 // its share of the chunk's k), in ascending flat order, with their residuals; the residual is not
 // stored.  The chunk's level-0 bin B0 is known after the pass.  A workgroup whose cut is at or
-// below B0, and whose candidates fit kCandCap, holds every element of bin B0 and above among its
+// below B0, and whose candidates fit its list, holds every element of bin B0 and above among its
 // candidates, so the level-1 pass and the emission work on those lists; any other workgroup
 // recomputes its residuals from X, C and the basis there (the same values, rarely needed).  The
 // selection is the same as the full passes'.
@@ -1726,6 +1729,38 @@ __device__ __forceinline__ uint32_t bf16_pair(float lo, float hi)
 // its bits 14..0 shifted up by 16, so its bin is bits 14..4 of the value.
 __device__ __forceinline__ uint32_t bin_lo(uint32_t w) { return __builtin_amdgcn_ubfe(w, 4, 11); }
 __device__ __forceinline__ uint32_t bin_hi(uint32_t w) { return __builtin_amdgcn_ubfe(w, 20, 11); }
+
+// A workgroup's cut, by one wave: the highest bin of its histogram where the count from the top reaches
+// the quota (bin 0 when it has fewer keys), from 64 sums of 32 bins and then the chosen 32 bins.
+__device__ __forceinline__ uint32_t list_cut(const uint32_t *__restrict__ s_hist, uint32_t quota)
+{
+    const int lane = threadIdx.x & 63;
+    constexpr int FB = kBins / kCoarse;
+    uint32_t suf = 0u;
+#pragma unroll 8
+    for (int b = 0; b < FB; ++b) suf += s_hist[lane * FB + ((b + lane) & (FB - 1))];  // (rotated: distinct banks)
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const uint32_t y = __shfl_down(suf, off, 64);
+        if (lane + off < 64) suf += y;
+    }
+    const uint64_t m = __ballot(suf >= quota);
+    uint32_t cut = 0u;
+    if (m != 0ull) {
+        const int cb = 63 - __clzll(m);
+        const uint32_t need1 = quota - (cb < 63 ? (uint32_t)__shfl((int)suf, cb + 1, 64) : 0u);
+        const int fl = lane & (FB - 1);
+        uint32_t sf = s_hist[cb * FB + fl];
+#pragma unroll
+        for (int off = 1; off < FB; off <<= 1) {
+            const uint32_t y = __shfl_down(sf, off, FB);
+            if (fl + off < FB) sf += y;
+        }
+        const uint64_t mf = __ballot(sf >= need1) & ((1ull << FB) - 1);
+        cut = (uint32_t)(cb * FB + (mf ? 63 - __clzll(mf) : 0));
+    }
+    return cut;
+}
 
 // Pass 1: as k_proj_hist_b (coefficients computed or loaded, level-0 histogram with its coarse
 // sums, max key), then the workgroup's cut and its candidates.
@@ -1831,33 +1866,8 @@ __global__ __launch_bounds__(kBlock) void k_proj_cand(SaveGeom g, FastGeom fg, c
     for (int off = 32; off > 0; off >>= 1) kmax = max(kmax, (uint32_t)__shfl_xor((int)kmax, off, 64));
     if (lane == 0) s_wmax[wave] = kmax;
     __syncthreads();
-    // the cut: the highest bin where the count from the top reaches the quota (bin 0 when the
-    // workgroup has fewer keys), from 64 sums of 32 bins and then the chosen 32 bins
     if (wave == 0) {
-        constexpr int FB = kBins / kCoarse;
-        uint32_t suf = 0u;
-#pragma unroll 8
-        for (int b = 0; b < FB; ++b) suf += s_hist[lane * FB + b];
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-            const uint32_t y = __shfl_down(suf, off, 64);
-            if (lane + off < 64) suf += y;
-        }
-        const uint64_t m = __ballot(suf >= quota);
-        uint32_t cut = 0u;
-        if (m != 0ull) {
-            const int cb = 63 - __clzll(m);
-            const uint32_t need1 = quota - (cb < 63 ? (uint32_t)__shfl((int)suf, cb + 1, 64) : 0u);
-            const int fl = lane & (FB - 1);
-            uint32_t sf = s_hist[cb * FB + fl];
-#pragma unroll
-            for (int off = 1; off < FB; off <<= 1) {
-                const uint32_t y = __shfl_down(sf, off, FB);
-                if (fl + off < FB) sf += y;
-            }
-            const uint64_t mf = __ballot(sf >= need1) & ((1ull << FB) - 1);
-            cut = (uint32_t)(cb * FB + (mf ? 63 - __clzll(mf) : 0));
-        }
+        const uint32_t cut = list_cut(s_hist, quota);
         if (lane == 0) s_cut = cut;
     }
     __syncthreads();
@@ -1885,8 +1895,8 @@ __global__ __launch_bounds__(kBlock) void k_proj_cand(SaveGeom g, FastGeom fg, c
         for (int i = 0; i < NB; ++i) s_wt[wave * NB + i] = incl[i];
     __syncthreads();
     uint32_t before_iter = 0u;
-    uint32_t *ci = cand_idx + (int64_t)blockIdx.x * kCandCap;
-    uint16_t *cv = cand_val + (int64_t)blockIdx.x * kCandCap;
+    uint32_t *ci = cand_idx + (int64_t)blockIdx.x * kListCap;
+    uint16_t *cv = cand_val + (int64_t)blockIdx.x * kListCap;
 #pragma unroll
     for (int i = 0; i < NB; ++i) {
         uint32_t waves_before = 0u, iter_total = 0u;
@@ -1905,7 +1915,7 @@ __global__ __launch_bounds__(kBlock) void k_proj_cand(SaveGeom g, FastGeom fg, c
                 uint32_t word = wd[0];
 #pragma unroll
                 for (int k = 1; k < 4; ++k) word = (e >> 1) == k ? wd[k] : word;
-                if (pos < (uint32_t)kCandCap) {
+                if (pos < (uint32_t)kListCap) {
                     ci[pos] = (uint32_t)(ld.rows[i] * g.d + col + e);
                     cv[pos] = (uint16_t)((word >> (16 * (e & 1))) & 0xffffu);
                 }
@@ -1922,7 +1932,8 @@ __global__ __launch_bounds__(kBlock) void k_proj_cand(SaveGeom g, FastGeom fg, c
     if (threadIdx.x < kCoarse) {
         uint32_t sum = 0u;
 #pragma unroll 8
-        for (int b = 0; b < kBins / kCoarse; ++b) sum += s_hist[threadIdx.x * (kBins / kCoarse) + b];
+        for (int b = 0; b < kBins / kCoarse; ++b)
+            sum += s_hist[threadIdx.x * (kBins / kCoarse) + ((b + threadIdx.x) & (kBins / kCoarse - 1))];
         if (sum) atomicAdd(&coarse[(chunk * g.hcopies + copy) * kCoarse + threadIdx.x], sum);
     }
     if (threadIdx.x == 0) {
@@ -1933,21 +1944,346 @@ __global__ __launch_bounds__(kBlock) void k_proj_cand(SaveGeom g, FastGeom fg, c
     }
 }
 
-// One vector's residual recomputed from X, C and the basis (the candidate passes' fallback, one
-// iteration at a time so that it does not set the kernels' register budget); false outside the
-// matrix or the workgroup's rows.
-template <int R>
-__device__ __forceinline__ bool cand_residual(const SaveGeom &g, const uint16_t *__restrict__ x,
-                                              const uint16_t *__restrict__ coeff, const float (&q)[8][R], int64_t row,
-                                              int64_t row_end, int64_t col, bool col_ok, float (&r)[8])
+// ------------------------------------------------------------------ candidate path (bf16, wide rows)
+// k_proj_hist_w's rows (its batch of NB = 64 / R rows a workgroup, its sums in the same order), with the
+// candidate lists of k_proj_cand in place of the stored residual: X is read once and nothing of its
+// size is written.  What bounds it is the vector unit (the v_dot2 projection, 8 an element at rank 16), so
+// the residual's fused-multiply-add chain runs on the matrix cores: v_mfma_f32_4x4x1 gives, for a
+// thread's column, sum_j c_j q_j of four rows as one chain over j, each step rounded as fmaf rounds it (the
+// same bits, NaNs included: checked on the GPU over 4 M chains of finite, subnormal, infinite and NaN
+// operands).
+template <int R, int MV, int NT>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(R == 8 && MV == 2 ? 3 : 4))) void k_proj_cand_w(SaveGeom g, const uint16_t *__restrict__ x,
+                                                    const float *__restrict__ qp, uint16_t *__restrict__ coeff,
+                                                    uint32_t *__restrict__ hist, uint32_t *__restrict__ maxkey,
+                                                    const uint16_t *__restrict__ coeff_in,
+                                                    uint32_t *__restrict__ coarse, float *__restrict__ y_out, int y_cols,
+                                                    float *__restrict__ epart, uint32_t quota,
+                                                    uint32_t *__restrict__ cand_idx, uint16_t *__restrict__ cand_val,
+                                                    CandMeta *__restrict__ meta)
 {
-    constexpr int DT = STACR_DTYPE_BF16;
-    const bool live = col_ok && row < row_end;
-    float xv[8], c[R];
-    unpack_raw<DT, 8>(load_raw<DT, 8>(x + row * g.d + col, live), xv);
-    load_coeff<DT, R>(coeff, row, g.rank, live, c);
-    batch_residual<DT, R, 8>(xv, c, q, r);
-    return live;
+    constexpr int DT = STACR_DTYPE_BF16, V = 8, NB = Batch<R>::NB, W = NT / 64;
+    constexpr int NG = NB / 4, E = V / NG;  // groups of four rows, and columns whose chains run together (8 chains)
+    static_assert(NB * R == 64 && NT % 64 == 0 && kBins % (4 * NT) == 0, "batch and block shape");
+    typedef float f32x4 __attribute__((ext_vector_type(4)));
+    typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+    __shared__ __align__(16) uint32_t s_hist[kBins];
+    __shared__ __align__(16) float s_part[W * 64];
+    __shared__ __align__(16) float s_c[64];
+    __shared__ uint32_t s_wmax[W];
+    __shared__ float s_ex[W];
+    __shared__ uint32_t s_wt[W * NB * MV];
+    __shared__ uint32_t s_cut;
+    int64_t chunk, row0, row_end;
+    wg_rows(g, blockIdx.x, chunk, row0, row_end);
+    if (row0 >= row_end) {  // a trailing workgroup with no rows (uniform): its energy partial is zero
+        if (epart && threadIdx.x < kEnergyStride) epart[(int64_t)blockIdx.x * kEnergyStride + threadIdx.x] = 0.f;
+        return;
+    }
+    const int u = threadIdx.x, lane = u & 63, wave = u >> 6;
+    const int n_rows = (int)(row_end - row0);  // (at most NB)
+    const uint32_t d = (uint32_t)g.d;
+    uint32_t col[MV], colc[MV];
+    bool col_ok[MV];
+#pragma unroll
+    for (int m = 0; m < MV; ++m) {
+        col[m] = (uint32_t)(m * NT + u) * V;
+        colc[m] = min(col[m], d - V);
+        col_ok[m] = col[m] < d;
+    }
+    // X: rows clamped into the workgroup's range and columns into the row, values outside zeroed
+    uint4 raw[NB][MV];
+#pragma unroll
+    for (int i = 0; i < NB; ++i) {
+        const uint16_t *src = x + (row0 + (i < n_rows ? i : 0)) * g.d;
+#pragma unroll
+        for (int m = 0; m < MV; ++m) raw[i][m] = *reinterpret_cast<const uint4 *>(src + colc[m]);
+    }
+    const uint16_t *qph = reinterpret_cast<const uint16_t *>(qp + 2 * g.d * R);  // [R][d], zero past the rank
+    for (int b = u; b < kBins / 4; b += NT) reinterpret_cast<uint4 *>(s_hist)[b] = make_uint4(0u, 0u, 0u, 0u);
+    if (coeff_in) {
+        if (u < 64) {
+            const int i = u / R, j = u % R;
+            s_c[u] = i < n_rows && j < g.rank ? Act<DT>::ld(coeff_in[(row0 + i) * g.rank + j]) : 0.f;
+        }
+        __syncthreads();
+    } else {
+        // (the sums of k_proj_hist_w: over a vector's pairs, then the vectors, then the lanes, then the waves)
+        // Basis words two columns at a time, the next two loaded while these are used: the scheduling
+        // barriers keep the compiler from loading every column's words at once (all of them would be
+        // MV * R * 4 registers, twice what this leaves for two workgroups a CU).
+        float acc[64];
+        constexpr int JC = 2;
+        uint4 qw[2][MV][JC];
+        auto load_q = [&](int j0, uint4 (&w)[MV][JC]) {
+#pragma unroll
+            for (int m = 0; m < MV; ++m)
+#pragma unroll
+                for (int j = 0; j < JC; ++j) w[m][j] = *reinterpret_cast<const uint4 *>(qph + (size_t)(j0 + j) * d + colc[m]);
+        };
+#pragma unroll
+        for (int i = 0; i < NB; ++i)
+            if (i >= n_rows) {  // (uniform) a row past the range adds zero
+#pragma unroll
+                for (int m = 0; m < MV; ++m) raw[i][m] = make_uint4(0u, 0u, 0u, 0u);
+            }
+#pragma unroll
+        for (int k = 0; k < 64; ++k) acc[k] = 0.f;
+        load_q(0, qw[0]);
+#pragma unroll
+        for (int j0 = 0; j0 < R; j0 += JC) {
+            uint4 (&w)[MV][JC] = qw[(j0 / JC) & 1];
+            if (j0 + JC < R) load_q(j0 + JC, qw[(j0 / JC + 1) & 1]);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int m = 0; m < MV; ++m) {
+                if (!col_ok[m]) continue;  // (a thread past the row adds nothing)
+#pragma unroll
+                for (int i = 0; i < NB; ++i)
+#pragma unroll
+                    for (int j = 0; j < JC; ++j) {
+                        float sum = acc[i * R + j0 + j];
+                        sum = dot2<DT>(raw[i][m].x, w[m][j].x, sum);
+                        sum = dot2<DT>(raw[i][m].y, w[m][j].y, sum);
+                        sum = dot2<DT>(raw[i][m].z, w[m][j].z, sum);
+                        sum = dot2<DT>(raw[i][m].w, w[m][j].w, sum);
+                        acc[i * R + j0 + j] = sum;
+                    }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        const float part = wave_reduce_scatter64(acc);
+        s_part[wave * 64 + lane] = part;
+        __syncthreads();
+        if (wave == 0) {
+            float tot = part;
+            for (int w = 1; w < W; ++w) tot += s_part[w * 64 + lane];
+            const int i = lane / R, j = lane % R;
+            const int64_t row = row0 + i;
+            if (y_out && j < y_cols && row < row_end) y_out[row * y_cols + j] = tot;
+            const float cv = j < g.rank ? Act<DT>::rnd(tot) : 0.f;  // (columns past the rank: Y only)
+            s_c[lane] = cv;
+            if (j < g.rank && row < row_end) coeff[row * g.rank + j] = Act<DT>::st(cv);
+        }
+        __syncthreads();
+    }
+    if (epart) {
+        // energies: sum of rnd(x^2) over this thread's elements, then over the workgroup in wave order
+        float ex = 0.f;
+#pragma unroll
+        for (int m = 0; m < MV; ++m)
+#pragma unroll
+            for (int i = 0; i < NB; ++i) {
+                if (i >= n_rows || !col_ok[m]) continue;
+                const uint32_t xw[4] = {raw[i][m].x, raw[i][m].y, raw[i][m].z, raw[i][m].w};
+#pragma unroll
+                for (int e = 0; e < V; ++e) {
+                    const float xe = Act<DT>::ld((uint16_t)((xw[e >> 1] >> (16 * (e & 1))) & 0xffffu));
+                    ex += Act<DT>::rnd(xe * xe);
+                }
+            }
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) ex += __shfl_xor(ex, off, 64);
+        if (lane == 0) s_ex[wave] = ex;
+        if (wave == 0) {  // C as saved: lane (i, j)
+            const float cv = s_c[lane];
+            float sc = Act<DT>::rnd(cv * cv), cj = cv * cv;
+#pragma unroll
+            for (int off = 32; off > 0; off >>= 1) sc += __shfl_xor(sc, off, 64);
+#pragma unroll
+            for (int off = 32; off >= R; off >>= 1) cj += __shfl_xor(cj, off, 64);  // over the rows i
+            float *ep = epart + (int64_t)blockIdx.x * kEnergyStride;
+            if (lane < g.rank) ep[2 + lane] = cj;
+            if (lane == 0) ep[1] = sc;
+        }
+        __syncthreads();
+        if (u == 0) {
+            float t = s_ex[0];
+            for (int w = 1; w < W; ++w) t += s_ex[w];
+            epart[(int64_t)blockIdx.x * kEnergyStride] = t;
+        }
+    }
+    // ---- residuals r = rnd(x - rnd(sum_j c_j q_j)), packed in place of X
+    // matrix operands: lane l gives c[4 gr + l % 4][j] of each group of rows and q_j of its own column; result
+    // register r of a lane is then row 4 gr + r of the lane's column
+    float cop[NG][R];
+#pragma unroll
+    for (int gr = 0; gr < NG; ++gr)
+#pragma unroll
+        for (int j = 0; j < R; j += 4) {
+            const float4 v = *reinterpret_cast<const float4 *>(s_c + (4 * gr + (lane & 3)) * R + j);
+            cop[gr][j] = v.x; cop[gr][j + 1] = v.y; cop[gr][j + 2] = v.z; cop[gr][j + 3] = v.w;
+        }
+    u16x2 kmax2 = {0, 0};
+#pragma unroll
+    for (int m = 0; m < MV; ++m) {
+#pragma unroll
+        for (int h = 0; h < V / E; ++h) {
+            f32x4 p[NG][E];
+#pragma unroll
+            for (int gr = 0; gr < NG; ++gr)
+#pragma unroll
+                for (int e = 0; e < E; ++e) p[gr][e] = f32x4{0.f, 0.f, 0.f, 0.f};
+            // (the basis words again, from L2, four columns at a time)
+            constexpr int JC = 4;
+            uint32_t w[2][JC][E / 2];
+            auto load_q = [&](int j0, uint32_t (&q)[JC][E / 2]) {
+#pragma unroll
+                for (int j = 0; j < JC; ++j) {
+                    const uint16_t *src = qph + (size_t)(j0 + j) * d + (colc[m] + h * E);
+                    if constexpr (E == 8) {
+                        const uint4 v = *reinterpret_cast<const uint4 *>(src);
+                        q[j][0] = v.x; q[j][1] = v.y; q[j][E / 2 - 2] = v.z; q[j][E / 2 - 1] = v.w;
+                    } else {
+                        const uint2 v = *reinterpret_cast<const uint2 *>(src);
+                        q[j][0] = v.x; q[j][1] = v.y;
+                    }
+                }
+            };
+            load_q(0, w[0]);
+#pragma unroll
+            for (int j0 = 0; j0 < R; j0 += JC) {
+                if (j0 + JC < R) load_q(j0 + JC, w[(j0 / JC + 1) & 1]);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int j = 0; j < JC; ++j) {
+#pragma unroll
+                    for (int e = 0; e < E; ++e) {
+                        const uint32_t we = w[(j0 / JC) & 1][j][e >> 1];
+                        const float qe = __uint_as_float(e & 1 ? we & 0xffff0000u : we << 16);
+#pragma unroll
+                        for (int gr = 0; gr < NG; ++gr)
+                            p[gr][e] = __builtin_amdgcn_mfma_f32_4x4x1f32(cop[gr][j0 + j], qe, p[gr][e], 0, 0, 0);
+                    }
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+            for (int i = 0; i < NB; ++i) {
+                uint32_t xw[4] = {raw[i][m].x, raw[i][m].y, raw[i][m].z, raw[i][m].w};
+#pragma unroll
+                for (int e = 0; e < E; e += 2) {
+                    const uint32_t pb = bf16_pair(p[i / 4][e][i % 4], p[i / 4][e + 1][i % 4]);
+                    const uint32_t xe = xw[h * (E / 2) + e / 2];
+                    xw[h * (E / 2) + e / 2] = bf16_pair(__uint_as_float(xe << 16) - __uint_as_float(pb << 16),
+                                                        __uint_as_float(xe & 0xffff0000u) - __uint_as_float(pb & 0xffff0000u));
+                }
+                raw[i][m] = make_uint4(xw[0], xw[1], xw[2], xw[3]);
+            }
+        }
+        if (!col_ok[m]) continue;
+#pragma unroll
+        for (int i = 0; i < NB; ++i) {
+            if (i >= n_rows) break;
+            const uint32_t w[4] = {raw[i][m].x, raw[i][m].y, raw[i][m].z, raw[i][m].w};
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                atomicAdd(&s_hist[bin_lo(w[k])], 1u);
+                atomicAdd(&s_hist[bin_hi(w[k])], 1u);
+                kmax2 = __builtin_elementwise_max(kmax2, __builtin_bit_cast(u16x2, w[k] & 0x7fff7fffu));
+            }
+        }
+    }
+    uint32_t kmax = (uint32_t)max(kmax2.x, kmax2.y) << 16;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) kmax = max(kmax, (uint32_t)__shfl_xor((int)kmax, off, 64));
+    if (lane == 0) s_wmax[wave] = kmax;
+    __syncthreads();
+    if (wave == 0) {
+        const uint32_t cut = list_cut(s_hist, quota);
+        if (lane == 0) s_cut = cut;
+    }
+    __syncthreads();
+    // ---- the candidates in ascending flat order: (row, vector, wave, lane, element)
+    const uint32_t cut = s_cut;
+    // A vector's 8-bit mask of elements in the cut's bin and above: |r|'s bits against the bin's lowest
+    // value, two at a time (a saturating difference is nonzero at or above it).
+    const unsigned short below = (unsigned short)((cut << 4) - 1u);  // (cut 0: every element)
+    const u16x2 below2 = {below, below}, one2 = {1, 1};
+    constexpr int NV = NB * MV;
+    uint32_t msk[NV];
+#pragma unroll
+    for (int i = 0; i < NB; ++i)
+#pragma unroll
+        for (int m = 0; m < MV; ++m) {
+            uint32_t k8 = 0u;
+            if (col_ok[m] && i < n_rows) {
+                const uint32_t w[4] = {raw[i][m].x, raw[i][m].y, raw[i][m].z, raw[i][m].w};
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    u16x2 t = __builtin_elementwise_sub_sat(__builtin_bit_cast(u16x2, w[k] & 0x7fff7fffu), below2);
+                    asm("" : "+v"(t));  // (kept packed: seen through, the two steps become single compares and selects)
+                    t = __builtin_elementwise_min(t, one2);
+                    k8 |= __builtin_bit_cast(uint32_t, t) << (2 * k);  // elements 2 k at bit 2 k, 2 k + 1 at 16 + 2 k
+                }
+                k8 = cut ? (k8 | (k8 >> 15)) & 0xffu : 0xffu;
+            }
+            msk[i * MV + m] = k8;
+        }
+    // their places: prefix sums over the lanes, two vectors' counts (at most 512 a wave) a word, then one
+    // wave's prefix over (row, vector, wave)
+    uint32_t at[NV];  // candidates of the wave's lower lanes in the same vector
+#pragma unroll
+    for (int v = 0; v < NV; v += 2) {
+        const uint32_t c0 = (uint32_t)__popc(msk[v]), c1 = v + 1 < NV ? (uint32_t)__popc(msk[v + 1 < NV ? v + 1 : v]) : 0u;
+        const uint32_t incl = wave_inclusive_scan(c0 | (c1 << 16));
+        at[v] = (incl & 0xffffu) - c0;
+        if (v + 1 < NV) at[v + 1 < NV ? v + 1 : v] = (incl >> 16) - c1;
+        if (lane == 63) {
+            s_wt[v * W + wave] = incl & 0xffffu;
+            if (v + 1 < NV) s_wt[(v + 1) * W + wave] = incl >> 16;
+        }
+    }
+    __syncthreads();
+    if (wave == 0) {
+        constexpr int N = W * NV;
+        uint32_t run = 0u;
+#pragma unroll
+        for (int k = 0; k < N; k += 64) {
+            const uint32_t t = k + lane < N ? s_wt[k + lane] : 0u;
+            const uint32_t incl = wave_inclusive_scan(t);
+            if (k + lane < N) s_wt[k + lane] = run + incl - t;
+            run += (uint32_t)__shfl((int)incl, 63, 64);
+        }
+        if (lane == 0) meta[blockIdx.x] = CandMeta{cut, run};
+    }
+    __syncthreads();
+    uint32_t *ci = cand_idx + (int64_t)blockIdx.x * kListCap;
+    uint16_t *cv = cand_val + (int64_t)blockIdx.x * kListCap;
+#pragma unroll
+    for (int i = 0; i < NB; ++i)
+#pragma unroll
+        for (int m = 0; m < MV; ++m) {
+            uint32_t pos = s_wt[(i * MV + m) * W + wave] + at[i * MV + m];
+            const uint32_t wd[4] = {raw[i][m].x, raw[i][m].y, raw[i][m].z, raw[i][m].w};
+            for (uint32_t k8 = msk[i * MV + m]; k8 != 0u; k8 &= k8 - 1u, ++pos) {
+                const int e = __builtin_ctz(k8);
+                uint32_t word = wd[0];
+#pragma unroll
+                for (int k = 1; k < 4; ++k) word = (e >> 1) == k ? wd[k] : word;
+                if (pos < (uint32_t)kListCap) {
+                    ci[pos] = (uint32_t)((row0 + i) * g.d) + col[m] + (uint32_t)e;
+                    cv[pos] = (uint16_t)((word >> (16 * (e & 1))) & 0xffffu);
+                }
+            }
+        }
+    // ---- this workgroup's copy of the chunk histogram and of the max key (as k_proj_hist_w)
+    const int copy = (int)(blockIdx.x % g.hcopies);
+    uint32_t *gh = hist + ((chunk * 3 + 0) * g.hcopies + copy) * kBins;
+    for (int b = u; b < kBins; b += NT)
+        if (s_hist[b]) atomicAdd(&gh[b], s_hist[b]);
+    if (u < kCoarse) {
+        uint32_t sum = 0u;
+#pragma unroll 8
+        for (int b = 0; b < kBins / kCoarse; ++b) sum += s_hist[u * (kBins / kCoarse) + ((b + u) & (kBins / kCoarse - 1))];
+        if (sum) atomicAdd(&coarse[(chunk * g.hcopies + copy) * kCoarse + u], sum);
+    }
+    if (u == 0) {
+        uint32_t mx = 0u;
+#pragma unroll
+        for (int w = 0; w < W; ++w) mx = max(mx, s_wmax[w]);
+        if (mx) atomicMax(maxkey + copy * kMaxKeyStride, mx);
+    }
 }
 
 // A thread's 8 consecutive candidate values (16 bytes), and their flat indices; entries at or past
@@ -1957,129 +2293,347 @@ struct CandVals {
     __device__ __forceinline__ uint32_t bits(int j) const { return (w[j >> 1] >> (16 * (j & 1))) & 0xffffu; }
 };
 
-// Level 1 (bf16, batched, candidates): the level-0 selection, then the histogram of key bits
-// 19..16 inside B0 and the per-workgroup records of k_refine_hist_b, from the candidates.
-template <int R, int HC>
-__global__ __launch_bounds__(kBlock) void k_refine_cand(SaveGeom g, FastGeom fg, const uint16_t *__restrict__ x,
-                                                        const float *__restrict__ qp, const uint16_t *__restrict__ coeff,
-                                                        uint32_t *__restrict__ hist, SelState *__restrict__ state,
-                                                        uint32_t k_full, uint32_t k_last, uint32_t *__restrict__ maxkey,
-                                                        uint32_t *__restrict__ fold, int64_t fold_stride,
-                                                        const uint32_t *__restrict__ coarse,
-                                                        const uint16_t *__restrict__ cand_val,
-                                                        const CandMeta *__restrict__ meta)
+// ------------------------------------------------------------------ the candidate lists' later passes
+// One wave per list (a projection workgroup's candidates, a few hundred): these passes are a chain of
+// dependent loads and a little arithmetic, so their time is that chain's latency times the rounds of
+// waves the lists take.  A wave a list instead of a workgroup puts every list of 8192 projection workgroups
+// on the chip at once and needs no barrier (8192 lists of about 880: level 1 90 -> 15 us, emission 102 -> 22 us; eight a workgroup 18 and 30 us).
+// A list that is not usable is recomputed by its whole workgroup.
+constexpr int kListWaves = 4;          // lists of a workgroup
+constexpr int kFewLists = 255;         // up to this many lists, a workgroup each: every list a compute unit (measured: 48
+                                       // lists 9.1 -> 8.0 us, but 512 lists 8.6 -> 9.7)
+constexpr int kListRound = 64 * 8;     // candidates a wave reads at once
+
+// A lane's 8 consecutive candidate values of round k (zeros past the list).
+__device__ __forceinline__ CandVals list_vals(const uint16_t *__restrict__ cand_val, int64_t list, int k, uint32_t n)
 {
-    constexpr int NB = Batch<R>::NB;
-    __shared__ uint32_t s_hist[kBins];
-    __shared__ uint32_t s_above[kWaves];
+    CandVals r;
+    uint4 v = make_uint4(0u, 0u, 0u, 0u);
+    const uint32_t e = (uint32_t)(k * kListRound + 8 * (threadIdx.x & 63));
+    if (e < n) v = *reinterpret_cast<const uint4 *>(cand_val + list * kListCap + e);
+    r.w[0] = v.x; r.w[1] = v.y; r.w[2] = v.z; r.w[3] = v.w;
+    return r;
+}
+
+// The residuals of 8 columns of a row, recomputed from X, the saved C and the basis (the fallback of a list
+// that is not usable): the projection pass's chain, one basis column at a time.
+__device__ __forceinline__ void list_residual(const SaveGeom &g, int R, const uint16_t *__restrict__ x,
+                                              const uint16_t *__restrict__ qph, const uint16_t *__restrict__ coeff,
+                                              int64_t row, int64_t col, float (&r)[8])
+{
+    float p[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) p[e] = 0.f;
+#pragma unroll 4  // (R is 4, 8, 16 or 32) four columns' words in flight
+    for (int j = 0; j < R; ++j) {
+        const uint4 v = *reinterpret_cast<const uint4 *>(qph + j * g.d + col);
+        const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+        const float c = j < g.rank ? bf16_bits_to_f(coeff[row * g.rank + j]) : 0.f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+            p[e] = fmaf(c, __uint_as_float(e & 1 ? w[e >> 1] & 0xffff0000u : w[e >> 1] << 16), p[e]);
+    }
+    float xv[8];
+    load_vec<STACR_DTYPE_BF16, 8>(x + row * g.d + col, xv);
+    using A = Act<STACR_DTYPE_BF16>;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) r[e] = A::rnd(xv[e] - A::rnd(p[e]));
+}
+
+// Level 1: the level-0 selection, then the 16 live bins of key bits 19..16 inside B0 (bf16: the bits below are
+// zero) and the records of k_refine_hist_b: cum[b] for b = 0..15, and cum[16], the count above B0.
+template <int HC, int LW>
+__global__ __launch_bounds__(64 * LW) void k_refine_lists(SaveGeom g, int R, int64_t n_lists,
+                                                                  const uint16_t *__restrict__ x,
+                                                                  const float *__restrict__ qp,
+                                                                  const uint16_t *__restrict__ coeff,
+                                                                  uint32_t *__restrict__ hist, SelState *__restrict__ state,
+                                                                  uint32_t k_full, uint32_t k_last,
+                                                                  uint32_t *__restrict__ maxkey, uint32_t *__restrict__ fold,
+                                                                  const uint32_t *__restrict__ coarse,
+                                                                  const uint16_t *__restrict__ cand_val,
+                                                                  const CandMeta *__restrict__ meta)
+{
+    __shared__ uint32_t s_cnt[LW][16];
+    __shared__ uint32_t s_above[LW];
+    __shared__ uint32_t s_redo[LW];  // the list's B0 + 1 when its workgroup recomputes it, else 0
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t list_raw = (int64_t)blockIdx.x * LW + wave;
+    const int64_t list = min(list_raw, n_lists - 1);
     int64_t chunk, row0, row_end;
-    wg_rows(g, blockIdx.x, chunk, row0, row_end);
-    const bool has_rows = row0 < row_end;
+    wg_rows(g, list, chunk, row0, row_end);
+    const bool in = list_raw < n_lists, has_rows = in && row0 < row_end;
     const SelState sp = prev_state(0, state, chunk, g.n_chunks, k_full, k_last);
     uint32_t cv[HC];
 #pragma unroll
-    for (int h = 0; h < HC; ++h) cv[h] = coarse[(chunk * HC + h) * kCoarse + (threadIdx.x & 63)];
-    const CandMeta mine = meta[has_rows ? blockIdx.x : 0];
-    // the candidate values go out before the selection's histogram words (only the list's used
-    // part: the threads past it read nothing)
-    CandVals vals;
-    {
-        uint4 v = make_uint4(0u, 0u, 0u, 0u);
-        if ((uint32_t)(kCandPer * threadIdx.x) < min(mine.count, (uint32_t)kCandCap))
-            v = *reinterpret_cast<const uint4 *>(cand_val + (int64_t)blockIdx.x * kCandCap + kCandPer * threadIdx.x);
-        vals.w[0] = v.x; vals.w[1] = v.y; vals.w[2] = v.z; vals.w[3] = v.w;
-    }
-    for (int b = threadIdx.x; b < kBins; b += kBlock) s_hist[b] = 0u;
+    for (int h = 0; h < HC; ++h) cv[h] = coarse[(chunk * HC + h) * kCoarse + lane];
+    const CandMeta mine = meta[has_rows ? list : 0];
+    const uint32_t n = has_rows ? min(mine.count, (uint32_t)kListCap) : 0u;
+    // the first two rounds go out before the selection's words
+    CandVals v0 = list_vals(cand_val, list, 0, n), v1 = list_vals(cand_val, list, 1, n);
+    if (lane < 16) s_cnt[wave][lane] = 0u;
     const SelState sel = select_level0<HC>(cv, hist + chunk * 3 * HC * kBins, sp);
-    if (blockIdx.x % g.wgs_per_chunk == 0 && threadIdx.x == 0) state[chunk * 3 + 0] = sel;
-    if (HC > 1 && blockIdx.x == 0 && threadIdx.x == 0) {  // fold the max key's copies into the first
+    if (in && list == chunk * g.wgs_per_chunk && lane == 0) state[chunk * 3 + 0] = sel;
+    if (HC > 1 && list_raw == 0 && lane == 0) {  // fold the max key's copies into the first
         uint32_t m = maxkey[0];
 #pragma unroll
         for (int c = 1; c < HC; ++c) m = max(m, maxkey[c * kMaxKeyStride]);
         maxkey[0] = m;
     }
-    if (!has_rows) {
-        if (threadIdx.x <= 16) fold[threadIdx.x * fold_stride + blockIdx.x] = 0u;
-        return;
-    }
     const uint32_t prefix = sel.prefix;  // B0
-    const bool valid = mine.count <= (uint32_t)kCandCap && mine.cut <= prefix;  // uniform
-    __syncthreads();  // s_hist is clear
+    const bool usable = !has_rows || (mine.count <= (uint32_t)kListCap && mine.cut <= prefix);  // (uniform in the wave)
+    if (lane == 0) s_redo[wave] = usable ? 0u : prefix + 1u;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the counters are clear before any lane adds
     uint32_t above = 0u;
-    if (valid) {
+    auto count = [&](uint32_t key, uint32_t b0, int l) {
+        if ((key >> kDigitShift[0]) == b0) atomicAdd(&s_cnt[l][(key >> 16) & 15u], 1u);
+        above += (key >> kDigitShift[0]) > b0;
+    };
+    if (usable) {
+        for (int k = 0; k * kListRound < (int)n; ++k) {
+            const CandVals v = v0;
+            v0 = v1;
+            v1 = list_vals(cand_val, list, k + 2, n);
 #pragma unroll
-        for (int j = 0; j < kCandPer; ++j) {
-            if (kCandPer * threadIdx.x + j >= mine.count) break;
-            const uint32_t key = bf16_key(vals.bits(j));
-            if ((key >> kDigitShift[0]) == prefix) atomicAdd(&s_hist[(key >> kDigitShift[1]) & (kDigitBins[1] - 1)], 1u);
-            above += (key >> kDigitShift[0]) > prefix;
+            for (int j = 0; j < 8; ++j)
+                if ((uint32_t)(k * kListRound + 8 * lane + j) < n) count(bf16_key(v.bits(j)), prefix, wave);
         }
-    } else {
-        const int slot = threadIdx.x >> g.log2L, u = threadIdx.x & (g.L - 1);
-        const int64_t col = (int64_t)u * 8, colc = min(col, g.d - 8);
-        const bool col_ok = col < g.d;
-        float q[8][R];
-        basis_issue<R, 8>(qp + g.d * R, g.d, colc, q);
-        basis_mask<R, 8>(col_ok, q);
-#pragma unroll 1
-        for (int i = 0; i < NB; ++i) {
+    }
+    above = (uint32_t)__shfl((int)wave_inclusive_scan(above), 63, 64);
+    if (lane == 0) s_above[wave] = above;
+    __syncthreads();
+    for (int l = 0; l < LW; ++l) {
+        if (s_redo[l] == 0u) continue;  // (uniform)
+        int64_t c2, r0, r1;
+        wg_rows(g, (int64_t)blockIdx.x * LW + l, c2, r0, r1);
+        above = 0u;
+        const int per_row = (int)(g.d / 8), n_vec = (int)(r1 - r0) * per_row;
+        for (int v = threadIdx.x; v < n_vec; v += 64 * LW) {
             float r[8];
-            if (!cand_residual<R>(g, x, coeff, q, row0 + (int64_t)i * g.rpi + slot, row_end, col, col_ok, r)) continue;
+            list_residual(g, R, x, reinterpret_cast<const uint16_t *>(qp + 2 * g.d * R), coeff, r0 + v / per_row,
+                          8 * (v % per_row), r);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) count(__float_as_uint(r[e]) & 0x7fffffffu, s_redo[l] - 1u, l);
+        }
+        if (above) atomicAdd(&s_above[l], above);
+    }
+    __syncthreads();
+    if (!in) return;
+    above = s_above[wave];
+    const uint32_t mine16 = lane < 16 ? s_cnt[wave][lane] : 0u;
+    uint32_t suf = mine16;
+#pragma unroll
+    for (int off = 1; off < 16; off <<= 1) {
+        const uint32_t y = __shfl_down(suf, off, 64);
+        if (lane + off < 16) suf += y;
+    }
+    if (lane <= 16) fold[lane * n_lists + list] = above + (lane < 16 ? suf : 0u);
+    if (mine16) atomicAdd(&hist[((chunk * 3 + 1) * HC + (int)(list % HC)) * kBins + (lane << 7)], mine16);
+}
+
+// Emission: the final selection and the list's offset and tie budget (the earlier lists' records), then its
+// survivors quantized and written in ascending flat order.  With a census the workgroup counts its lists' entries
+// per feature in LDS first: two 16-bit counts a word (features f and f + 2048; a feature has at most one entry
+// a row, so no half overflows), rows of at most 4096 features.
+template <int HC, int LW>
+__global__ __launch_bounds__(64 * LW) void k_emit_lists(
+    SaveGeom g, int R, int64_t n_lists, const uint16_t *__restrict__ x, const float *__restrict__ qp,
+    const uint16_t *__restrict__ coeff, SelState *__restrict__ state, uint32_t chunk_k,
+    const uint32_t *__restrict__ maxkey, OutSpec o, float *scale_out, int to_list, const uint32_t *__restrict__ hist,
+    const uint32_t *__restrict__ fold, const uint32_t *__restrict__ cand_idx, const uint16_t *__restrict__ cand_val,
+    const CandMeta *__restrict__ meta, uint32_t *__restrict__ census, uint32_t n_entries)
+{
+    constexpr int DT = STACR_DTYPE_BF16;
+    __shared__ uint32_t s_feat[kBins];
+    __shared__ uint32_t s_redo[LW], s_T[LW], s_off[LW], s_take[LW];
+    __shared__ uint32_t s_wt[LW];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t list_raw = (int64_t)blockIdx.x * LW + wave;
+    const int64_t list = min(list_raw, n_lists - 1);
+    int64_t chunk, row0, row_end;
+    wg_rows(g, list, chunk, row0, row_end);
+    const int64_t w = list - chunk * g.wgs_per_chunk, wg0 = chunk * g.wgs_per_chunk;
+    const bool live = list_raw < n_lists && row0 < row_end;  // (a trailing list with no rows writes nothing)
+    uint32_t hw[HC];
+    {
+        const uint32_t *h1 = hist + (chunk * 3 + 1) * HC * kBins + ((lane & 15) << 7);
+#pragma unroll
+        for (int c = 0; c < HC; ++c) hw[c] = h1[c * kBins];
+    }
+    const CandMeta mine = meta[live ? list : 0];
+    const uint32_t n = min(mine.count, (uint32_t)kListCap);
+    struct Round {
+        CandVals v;
+        uint32_t flat[8];
+    };
+    auto load_round = [&](int k) {
+        Round r;
+        r.v = list_vals(cand_val, list, k, n);
+        const uint32_t e = (uint32_t)(k * kListRound + 8 * lane);
+        uint4 f0 = make_uint4(0u, 0u, 0u, 0u), f1 = f0;
+        if (e < n) f0 = *reinterpret_cast<const uint4 *>(cand_idx + list * kListCap + e);
+        if (e + 4 < n) f1 = *reinterpret_cast<const uint4 *>(cand_idx + list * kListCap + e + 4);
+        r.flat[0] = f0.x; r.flat[1] = f0.y; r.flat[2] = f0.z; r.flat[3] = f0.w;
+        r.flat[4] = f1.x; r.flat[5] = f1.y; r.flat[6] = f1.z; r.flat[7] = f1.w;
+        return r;
+    };
+    Round cur = load_round(0);  // (before the selection's and the offsets' words)
+    SelState sel1;
+    const SelState st = fold_select<HC>(hw, state[chunk * 3 + 0], &sel1);
+    if (live && w == 0 && lane == 0) {
+        state[chunk * 3 + 1] = sel1;
+        state[chunk * 3 + 2] = st;
+    }
+    const uint32_t b1 = (st.prefix >> 16) & 15u;
+    const uint32_t *fhi = fold + (int64_t)(b1 + 1) * n_lists + wg0;
+    const uint32_t *flo = fold + (int64_t)b1 * n_lists + wg0;
+    const uint32_t mk = *maxkey;
+    const uint32_t T = st.prefix;
+    const float amax = Act<DT>::rnd(__uint_as_float(mk));
+    const float scale = o.bits ? quant_scale(mk, o.bits, amax) : 1.f;
+    if (!to_list && list_raw == 0 && lane == 0 && scale_out) *scale_out = scale;
+    const uint32_t cfeat = (uint32_t)g.d, dmask = (cfeat & (cfeat - 1)) == 0 ? cfeat - 1u : 0u;
+    const uint32_t cwords = min(cfeat, (uint32_t)kBins);
+    if (census) {
+        for (uint32_t f = threadIdx.x; f < cwords; f += 64 * LW) s_feat[f] = 0u;
+        __syncthreads();
+    }
+    auto put = [&](uint32_t pos, uint32_t fl, float rv) {
+        if (pos >= o.cap) {
+            // unreachable when the counts are consistent; never write out of bounds
+        } else if (to_list) {
+            o.list_rbits[pos] = __float_as_uint(rv);
+            o.list_idx[pos] = fl;
+        } else {
+            write_entry<DT>(o, pos, fl, rv, scale);
+        }
+        if (census) {
+            const uint32_t f = dmask ? fl & dmask : fl % cfeat;
+            atomicAdd(&s_feat[f & (kBins - 1)], f >= (uint32_t)kBins ? 0x10000u : 1u);
+        }
+    };
+    const bool usable = !live || (mine.count <= (uint32_t)kListCap && mine.cut <= (T >> kDigitShift[0]));  // (uniform in the wave)
+    if (lane == 0) s_redo[wave] = usable ? 0u : 1u;
+    if (live) {
+        WgOffset wo;
+        {
+            uint32_t gt = 0u, eq = 0u;
+#pragma unroll 4
+            for (int64_t v = lane; v < w; v += 64) {
+                const uint32_t hi = fhi[v], lo = flo[v];
+                gt += hi;
+                eq += lo - hi;
+            }
+            const uint32_t my_eq = flo[w] - fhi[w];
+            const uint32_t gt_before = (uint32_t)__shfl((int)wave_inclusive_scan(gt), 63, 64);
+            const uint32_t eq_before = (uint32_t)__shfl((int)wave_inclusive_scan(eq), 63, 64);
+            // (opaque: written as take = eq_before >= need ? 0 : ..., off = ... + min(need, eq_before), this
+            // compiler drops the min here, in its middle end, and later lists' offsets come out too large)
+            uint32_t eq_taken = min(st.need, eq_before);
+            asm volatile("" : "+v"(eq_taken));
+            wo = WgOffset{(uint32_t)chunk * chunk_k + gt_before + eq_taken, min(my_eq, st.need - eq_taken)};
+        }
+        uint32_t before = 0u;  // survivors of the earlier rounds: above T, and equal to it in the upper half
+        if (usable) {
+            for (int k = 0; k * kListRound < (int)n; ++k) {
+                const Round r = cur;
+                if ((k + 1) * kListRound < (int)n) cur = load_round(k + 1);
+                uint32_t m = 0u;  // bits 0..7 above T, 8..15 equal to it
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    const bool in = (uint32_t)(k * kListRound + 8 * lane + j) < n;
+                    const uint32_t key = bf16_key(r.v.bits(j));
+                    m |= in && key > T ? 1u << j : 0u;
+                    m |= in && key == T ? 0x100u << j : 0u;
+                }
+                const uint32_t c = (uint32_t)__popc(m & 0xffu) | ((uint32_t)__popc(m >> 8) << 16);
+                const uint32_t incl = wave_inclusive_scan(c);
+                const uint32_t ex = before + incl - c;
+                uint32_t gb = ex & 0xffffu, eb = ex >> 16;
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    const bool is_gt = (m >> j) & 1u, is_eq = (m >> (8 + j)) & 1u;
+                    if (is_gt || (is_eq && eb < wo.take)) put(wo.off + gb + min(eb, wo.take), r.flat[j], bf16_bits_to_f(r.v.bits(j)));
+                    gb += is_gt;
+                    eb += is_eq;
+                }
+                before += (uint32_t)__shfl((int)incl, 63, 64);
+            }
+        } else if (lane == 0) {
+            s_T[wave] = T;
+            s_off[wave] = wo.off;
+            s_take[wave] = wo.take;
+        }
+        if (census && lane == 0) {
+            uint32_t *bstart = census + (int64_t)kCensusCopies * cfeat;
+            if (row0 % kCensusRows == 0) bstart[row0 / kCensusRows] = wo.off;
+            if (list == 0) bstart[(g.rows + kCensusRows - 1) / kCensusRows] = n_entries;
+        }
+    }
+    __syncthreads();
+    for (int l = 0; l < LW; ++l) {
+        if (s_redo[l] == 0u) continue;  // (uniform)
+        int64_t c2, r0, r1;
+        wg_rows(g, (int64_t)blockIdx.x * LW + l, c2, r0, r1);
+        const uint32_t Tl = s_T[l], off = s_off[l], take = s_take[l];
+        const int per_row = (int)(g.d / 8), n_vec = (int)(r1 - r0) * per_row;
+        uint32_t gt_before = 0u, eq_before = 0u;
+        for (int v0 = 0; v0 < n_vec; v0 += 64 * LW) {
+            const int v = v0 + (int)threadIdx.x, vc = min(v, n_vec - 1);
+            const int64_t row = r0 + vc / per_row, col = 8 * (vc % per_row);
+            float r[8];
+            list_residual(g, R, x, reinterpret_cast<const uint16_t *>(qp + 2 * g.d * R), coeff, row, col, r);
+            uint32_t m = 0u;
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
                 const uint32_t key = __float_as_uint(r[e]) & 0x7fffffffu;
-                if ((key >> kDigitShift[0]) == prefix) atomicAdd(&s_hist[(key >> kDigitShift[1]) & (kDigitBins[1] - 1)], 1u);
-                above += (key >> kDigitShift[0]) > prefix;
+                m |= v < n_vec && key > Tl ? 1u << e : 0u;
+                m |= v < n_vec && key == Tl ? 0x100u << e : 0u;
             }
+            const uint32_t c = (uint32_t)__popc(m & 0xffu) | ((uint32_t)__popc(m >> 8) << 16);
+            uint32_t tot;
+            const uint32_t ex = block_exclusive_scan<64 * LW>(c, s_wt, &tot);  // (at most 4096 of each)
+            uint32_t gb = gt_before + (ex & 0xffffu), eb = eq_before + (ex >> 16);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const bool is_gt = (m >> e) & 1u, is_eq = (m >> (8 + e)) & 1u;
+                if (is_gt || (is_eq && eb < take)) put(off + gb + min(eb, take), (uint32_t)(row * g.d + col + e), r[e]);
+                gb += is_gt;
+                eb += is_eq;
+            }
+            gt_before += tot & 0xffffu;
+            eq_before += tot >> 16;
         }
     }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) above += (uint32_t)__shfl_xor((int)above, off, 64);
-    if ((threadIdx.x & 63) == 0) s_above[threadIdx.x >> 6] = above;
-    __syncthreads();
-    if (threadIdx.x <= 16) {  // cum[b] for b = threadIdx.x (16: above B0 only), as k_refine_hist_b
-        uint32_t c = 0u;
-#pragma unroll
-        for (int wv = 0; wv < kWaves; ++wv) c += s_above[wv];
-        for (int b = threadIdx.x; b < 16; ++b) c += s_hist[b << 7];
-        fold[threadIdx.x * fold_stride + blockIdx.x] = c;
+    if (census) {  // the entries per feature
+        __syncthreads();
+        uint32_t *counts = census + (int64_t)(blockIdx.x % kCensusCopies) * cfeat;
+        for (uint32_t f = threadIdx.x; f < cwords; f += 64 * LW) {
+            const uint32_t v = s_feat[f];
+            if (v & 0xffffu) atomicAdd(&counts[f], v & 0xffffu);
+            if (v >> 16) atomicAdd(&counts[f + kBins], v >> 16);
+        }
     }
-    uint32_t *gh = hist + ((chunk * 3 + 1) * HC + blockIdx.x % HC) * kBins;
-    for (int b = threadIdx.x; b < kDigitBins[1]; b += kBlock)
-        if (s_hist[b]) atomicAdd(&gh[b], s_hist[b]);
 }
 
-// The emission's fallback for a workgroup without a usable candidate list: its residuals
-// recomputed (RIN: read from the stored residual) one iteration at a time, survivors compacted in
-// the order of k_emit_b and handed to `put` (position, flat index, value).
-template <int R, bool RIN, typename Put>
-__device__ __forceinline__ void emit_cand_fallback(const SaveGeom &g, const FastGeom &fg, const uint16_t *__restrict__ x,
-                                                   const float *__restrict__ qp, const uint16_t *__restrict__ coeff,
-                                                   int64_t row0, int64_t row_end, uint32_t T, const WgOffset &wo,
-                                                   uint32_t *s_wt, Put &put)
+// The emission's fallback for a workgroup without a usable candidate list: its residuals read from the
+// stored residual one iteration at a time, survivors compacted in the order of k_emit_b and handed
+// to `put` (position, flat index, value).
+template <int NB, typename Put>
+__device__ __forceinline__ void emit_cand_fallback(const SaveGeom &g, const uint16_t *__restrict__ res, int64_t row0,
+                                                   int64_t row_end, uint32_t T, const WgOffset &wo, uint32_t *s_wt, Put &put)
 {
-    constexpr int NB = Batch<R>::NB;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int slot = threadIdx.x >> g.log2L, u = threadIdx.x & (g.L - 1);
-    const int64_t col = (int64_t)u * 8, colc = min(col, g.d - 8);
+    const int64_t col = (int64_t)u * 8;
     const bool col_ok = col < g.d;
-    float q[8][RIN ? 1 : R];
-    if constexpr (!RIN) {
-        basis_issue<R, 8>(qp + g.d * R, g.d, colc, q);
-        basis_mask<R, 8>(col_ok, q);
-    }
     uint32_t before_iter = 0u;  // survivors of the earlier iterations (all waves)
 #pragma unroll 1
     for (int i = 0; i < NB; ++i) {
         const int64_t row = row0 + (int64_t)i * g.rpi + slot;
         float r[8];
-        bool live;
-        if constexpr (RIN) {
-            live = col_ok && row < row_end;
-            unpack_raw<STACR_DTYPE_BF16, 8>(load_raw<STACR_DTYPE_BF16, 8>(x + row * g.d + col, live), r);
-        } else {
-            live = cand_residual<R>(g, x, coeff, q, row, row_end, col, col_ok, r);
-        }
+        const bool live = col_ok && row < row_end;
+        unpack_raw<STACR_DTYPE_BF16, 8>(load_raw<STACR_DTYPE_BF16, 8>(res + row * g.d + col, live), r);
         uint32_t m = 0u;
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
@@ -2118,13 +2672,12 @@ __device__ __forceinline__ void emit_cand_fallback(const SaveGeom &g, const Fast
     }
 }
 
-// Emission (bf16, batched, candidates): the final selection and the workgroup's offset and tie
-// budget as in k_emit_b, then its survivors from the candidate list (or, for a workgroup without a
-// usable list, from recomputed residuals) quantized and written in ascending flat order.
-template <int R, int HC, bool RIN = false>
+// Emission (bf16, lists of the level-1 pass over a stored residual): the final selection and the workgroup's
+// offset and tie budget as in k_emit_b, then its survivors from the candidate list (or, for a workgroup
+// without a usable list, from the stored residual) quantized and written in ascending flat order.
+template <int R, int HC>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) void k_emit_cand(
-    SaveGeom g, FastGeom fg, const uint16_t *__restrict__ x, const float *__restrict__ qp,
-    const uint16_t *__restrict__ coeff, SelState *__restrict__ state, uint32_t chunk_k,
+    SaveGeom g, const uint16_t *__restrict__ res, SelState *__restrict__ state, uint32_t chunk_k,
     const uint32_t *__restrict__ maxkey, OutSpec o, float *scale_out, int to_list, const uint32_t *__restrict__ hist,
     const uint32_t *__restrict__ fold, int64_t fold_stride, const uint32_t *__restrict__ cand_idx,
     const uint16_t *__restrict__ cand_val, const CandMeta *__restrict__ meta, uint32_t *__restrict__ census,
@@ -2239,7 +2792,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
             eb += is_eq;
         }
     } else {
-        emit_cand_fallback<R, RIN>(g, fg, x, qp, coeff, row0, row_end, T, wo, s_wt, put);
+        emit_cand_fallback<Batch<R>::NB>(g, res, row0, row_end, T, wo, s_wt, put);
     }
     if (census) {  // the entries per feature (copy w % 8) and, at a block's first row, its first entry
         __syncthreads();
@@ -2416,6 +2969,9 @@ struct Plan {
     SaveGeom gw;
     int mvw, ntw;
     int64_t n_wgs_w;
+    // (bf16 wide rows with a residual and a quota inside the list) the projection pass keeps the lists
+    // (k_proj_cand_w): no stored residual, and g is the projection pass's geometry
+    bool wcand;
     // bf16 on the batched path with a residual and not wide: the candidate passes (k_proj_cand,
     // k_refine_cand, k_emit_cand) with the workgroups' quota
     bool cand;
@@ -2526,26 +3082,33 @@ Plan make_plan_wide(const StacrSaveArgs &a)
     return pv.wide ? pv : p;
 }
 
-// The candidate passes take bf16 saves on the batched path (not wide rows) when a workgroup's
-// quota, four times its mean share of its chunk's k plus 64, fits half the candidate list: a
-// workgroup then needs more than four times its share above the chunk's level-0 bin before it
-// falls back to recomputing.
+// The candidate passes take bf16 saves on the batched path and wide rows when a workgroup's
+// quota, four times its mean share of its chunk's k plus 64, is at most 1024 (wide rows: six times, 2048:
+// half the list, as the cut's bin comes in whole): a workgroup then needs more than that many times
+// its share above the chunk's level-0 bin before its list is recomputed.
 Plan make_plan_base(const StacrSaveArgs &a)
 {
     Plan p = make_plan_wide(a);
     if (!p.fold || a.k_total <= 0) return p;
     p.cand_rin = true;  // (unless the projection pass keeps lists itself, below)
-    if (p.wide) return p;
-    const SaveGeom &g = p.g;
+    const SaveGeom &g = p.wide ? p.gw : p.g;
     const double wg_elems = (double)g.rows_per_wg * (double)g.d;
     const int64_t last_rows = g.rows - (g.n_chunks - 1) * g.chunk_rows;
     const double dens = hmax<double>((double)a.k_full / ((double)g.chunk_rows * (double)g.d),
                                      (double)a.k_last / ((double)last_rows * (double)g.d));
-    const double quota = 4.0 * dens * wg_elems + 64.0;
-    if (quota > kCandCap / 2) return p;
+    double quota = 4.0 * dens * wg_elems + 64.0;
+    // (a wide workgroup has few rows, whose shares differ more: half as much again)
+    if (p.wide) quota *= 1.5;
+    if (quota > (p.wide ? kListCap : kCandCap) / 2) return p;
     p.cand = true;
     p.cand_rin = false;
     p.quota = (uint32_t)quota;
+    if (p.wide) {
+        p.wcand = true;
+        p.gw.hcopies = p.gw.wgs_per_chunk >= 256 ? kHistCopies : 1;
+        p.g = p.gw;
+        p.n_wgs = p.n_wgs_w;
+    }
     return p;
 }
 
@@ -2560,7 +3123,7 @@ Plan make_plan(const StacrSaveArgs &a)
         Plan p = make_plan_base(ay);
         if (p.wide) {
             p.gw.rank = a.rank;
-            p.g.rank = a.rank < 8 ? a.rank : 8;
+            p.g.rank = p.wcand || a.rank < 8 ? a.rank : 8;
             p.yc = a.y_cols;
             return p;
         }
@@ -2599,7 +3162,7 @@ size_t layout(const StacrSaveArgs &a, const Plan &p, size_t *off)
     const bool rstore = p.fast && a.dtype != STACR_DTYPE_F32 && a.k_total > 0 && !p.cand;  // (wide rows: p.fast)
     take(WS_R, rstore ? (size_t)a.rows * a.feats * 2 : 0);  // the stored residual (16-bit types)
     const bool lists = p.cand || p.cand_rin;
-    const size_t nc = lists ? (size_t)p.n_wgs * kCandCap : 0;  // the candidate lists
+    const size_t nc = lists ? (size_t)p.n_wgs * (p.cand ? kListCap : kCandCap) : 0;  // the candidate lists
     take(WS_CIDX, nc * sizeof(uint32_t));
     take(WS_CVAL, nc * sizeof(uint16_t));
     take(WS_CMETA, lists ? (size_t)p.n_wgs * sizeof(CandMeta) : 0);
@@ -2645,6 +3208,42 @@ int launch_wide_pass1(const StacrSaveArgs &a, const Plan &p, const typename Act<
     return STACR_OK;
 }
 
+// The wide projection pass that keeps candidate lists (bf16, a residual wanted).
+int launch_wide_cand(const StacrSaveArgs &a, const Plan &p, const uint16_t *x, const float *qp, uint16_t *coeff,
+                     uint32_t *hist, uint32_t *maxkey, const uint16_t *coeff_in, uint32_t *coarse, uint32_t *cidx,
+                     uint16_t *cval, CandMeta *cmeta)
+{
+    float *y_out = a.y_out && !coeff_in ? a.y_out : nullptr;
+    hipStream_t s = a.stream;
+    const unsigned n = (unsigned)p.n_wgs_w;
+    bool done = false;
+    auto go = [&](auto r, auto mv, auto nt) {
+        constexpr int R = decltype(r)::value, MV = decltype(mv)::value, NT = decltype(nt)::value;
+        if (done || p.Rq != R || p.mvw != MV || p.ntw != NT) return;
+        done = true;
+        stacr_launch("k_proj_cand_w", s, [&] {
+            k_proj_cand_w<R, MV, NT><<<n, NT, 0, s>>>(p.gw, x, qp, coeff, hist, maxkey, coeff_in, coarse, y_out, p.yc,
+                                                      a.energy_part, p.quota, cidx, cval, cmeta);
+        });
+    };
+    using I1 = std::integral_constant<int, 1>;
+    using I2 = std::integral_constant<int, 2>;
+    using I8 = std::integral_constant<int, 8>;
+    using I16 = std::integral_constant<int, 16>;
+    using N256 = std::integral_constant<int, 256>;
+    using N512 = std::integral_constant<int, 512>;
+    go(I8{}, I2{}, N256{});
+    go(I8{}, I2{}, N512{});
+    go(I16{}, I1{}, N256{});
+    go(I16{}, I1{}, N512{});
+    go(I16{}, I2{}, N512{});
+    if (!done)
+        return stacr_fail(STACR_ERR_INVALID, "stacr_save: no wide projection kernel for rank %d, %d x %d", p.Rq, p.mvw, p.ntw);
+    if (y_out && a.y_written) *a.y_written = 1;
+    if (a.energy_part && a.energy_written) *a.energy_written = 1;
+    return STACR_OK;
+}
+
 template <int DT, int R, int V, bool QREG>
 int launch_typed(const StacrSaveArgs &a, const Plan &p, char *ws, const size_t *off)
 {
@@ -2661,6 +3260,8 @@ int launch_typed(const StacrSaveArgs &a, const Plan &p, char *ws, const size_t *
     WgCount *counts = carve<WgCount>(ws, off[WS_COUNTS]);
     const bool resid = a.k_total > 0;
     const int nwg = (int)p.n_wgs;
+    const bool few = p.n_wgs <= kFewLists;
+    const unsigned n_list_wgs = (unsigned)(few ? p.n_wgs : (p.n_wgs + kListWaves - 1) / kListWaves);
 
     // padded basis; histograms and max key (contiguous in the layout) cleared in the same launch
     const int64_t n_zero = resid ? (int64_t)((off[WS_MAXKEY] + (size_t)p.g.hcopies * kMaxKeyStride * sizeof(uint32_t) -
@@ -2671,7 +3272,7 @@ int launch_typed(const StacrSaveArgs &a, const Plan &p, char *ws, const size_t *
     const int64_t csegs = p.g.d > 0 && a.feats % p.g.d == 0 ? a.feats / p.g.d : 0;
     const bool census = a.census && (p.cand || p.cand_rin) && !p.trim && csegs >= 1 &&
                         (kCensusRows * csegs) % p.g.rows_per_wg == 0 && p.g.rows % csegs == 0 &&
-                        (csegs == 1 ? a.feats <= kBins : p.cand_rin && !p.cand && a.feats <= 2 * kBins);
+                        (csegs == 1 && !p.wcand ? a.feats <= kBins : (p.wcand || (p.cand_rin && !p.cand)) && a.feats <= 2 * kBins);
     const int64_t n_census = census ? (int64_t)kCensusCopies * a.feats : 0;
     stacr_launch("k_prep", s, [&] {
         k_prep<DT><<<grid_for(hmax<int64_t>(hmax<int64_t>(a.feats * p.Rq, n_zero), n_census)), kBlock, 0, s>>>(
@@ -2705,9 +3306,17 @@ int launch_typed(const StacrSaveArgs &a, const Plan &p, char *ws, const size_t *
     if (!coeff_in || resid) {
         if constexpr (kFastOk) {
             if (fast && p.wide) {
+                if constexpr (kCandOk) {
+                    if (p.wcand) {
+                        const int rc = launch_wide_cand(a, p, x, qp, coeff_out, hist, maxkey, coeff_in, coarse, cidx, cval, cmeta);
+                        if (rc) return rc;
+                    }
+                }
                 if constexpr (kRin) {
+                    if (!p.wcand) {
                     const int rc = launch_wide_pass1<DT>(a, p, x, qp, coeff_out, hist, maxkey, resid ? 1 : 0, coeff_in, rbuf, coarse);
                     if (rc) return rc;
+                    }
                 } else {
                     return stacr_fail(STACR_ERR_INVALID, "stacr_save: wide rows outside 16-bit activations");
                 }
@@ -2743,9 +3352,10 @@ int launch_typed(const StacrSaveArgs &a, const Plan &p, char *ws, const size_t *
                 using H1 = std::integral_constant<int, 1>;
                 auto refine_cand = [&](auto hc) {
                     if constexpr (kCandOk)
-                        stacr_launch("k_refine_cand", s, [&] {
-                            k_refine_cand<R, decltype(hc)::value><<<nwg, kBlock, 0, s>>>(
-                                p.g, fg, x, qp, coeff, hist, state, kf, kl, maxkey, fold, p.n_wgs, coarse, cval, cmeta);
+                        stacr_launch("k_refine_lists", s, [&] {
+                            const auto k = few ? k_refine_lists<decltype(hc)::value, 1> : k_refine_lists<decltype(hc)::value, kListWaves>;
+                            k<<<n_list_wgs, few ? 64 : 64 * kListWaves, 0, s>>>(p.g, p.Rq, p.n_wgs, x, qp, coeff, hist, state, kf, kl,
+                                                                               maxkey, fold, coarse, cval, cmeta);
                         });
                 };
                 auto refine_lists = [&](auto hc) {
@@ -2796,15 +3406,26 @@ int launch_typed(const StacrSaveArgs &a, const Plan &p, char *ws, const size_t *
         if constexpr (kCandOk) {
             uint32_t *cen = census ? a.census : nullptr;
             const uint32_t kt = (uint32_t)a.k_sum;  // the entries emitted (no trim: the chunks' k summed)
-            if (cand && hc8)
-                stacr_launch("k_emit_cand", s, [&] { k_emit_cand<R, kHistCopies><<<nwg, kBlock, 0, s>>>(p.g, fg, x, qp, coeff, state, kf, maxkey, o, a.scale, p.trim ? 1 : 0, hist, fold, p.n_wgs, cidx, cval, cmeta, cen, kt, (uint32_t)a.feats); });
-            else if (cand)
-                stacr_launch("k_emit_cand", s, [&] { k_emit_cand<R, 1><<<nwg, kBlock, 0, s>>>(p.g, fg, x, qp, coeff, state, kf, maxkey, o, a.scale, p.trim ? 1 : 0, hist, fold, p.n_wgs, cidx, cval, cmeta, cen, kt, (uint32_t)a.feats); });
+            auto emit = [&](auto hc) {
+                stacr_launch("k_emit_lists", s, [&] {
+                    const auto k = few ? k_emit_lists<decltype(hc)::value, 1> : k_emit_lists<decltype(hc)::value, kListWaves>;
+                    k<<<n_list_wgs, few ? 64 : 64 * kListWaves, 0, s>>>(p.g, p.Rq, p.n_wgs, x, qp, coeff, state, kf, maxkey, o, a.scale,
+                                                                        p.trim ? 1 : 0, hist, fold, cidx, cval, cmeta, cen, kt);
+                });
+            };
+            auto emit_rin = [&](auto hc) {
+                stacr_launch("k_emit_cand", s, [&] {
+                    k_emit_cand<R, decltype(hc)::value><<<nwg, kBlock, 0, s>>>(p.g, xin, state, kf, maxkey, o, a.scale, p.trim ? 1 : 0, hist,
+                                                                             fold, p.n_wgs, cidx, cval, cmeta, cen, kt, (uint32_t)a.feats);
+                });
+            };
+            using C8 = std::integral_constant<int, kHistCopies>;
+            using C1 = std::integral_constant<int, 1>;
+            if (cand && hc8) emit(C8{});
+            else if (cand) emit(C1{});
             if constexpr (kRin) {  // the lists of the level-1 pass; the fallback reads the stored residual
-                if (cand_rin && hc8)
-                    stacr_launch("k_emit_cand", s, [&] { k_emit_cand<R, kHistCopies, true><<<nwg, kBlock, 0, s>>>(p.g, fg, xin, qp, coeff, state, kf, maxkey, o, a.scale, p.trim ? 1 : 0, hist, fold, p.n_wgs, cidx, cval, cmeta, cen, kt, (uint32_t)a.feats); });
-                else if (cand_rin)
-                    stacr_launch("k_emit_cand", s, [&] { k_emit_cand<R, 1, true><<<nwg, kBlock, 0, s>>>(p.g, fg, xin, qp, coeff, state, kf, maxkey, o, a.scale, p.trim ? 1 : 0, hist, fold, p.n_wgs, cidx, cval, cmeta, cen, kt, (uint32_t)a.feats); });
+                if (cand_rin && hc8) emit_rin(C8{});
+                else if (cand_rin) emit_rin(C1{});
             }
             // (written only by an emission that ran: candidate lists from X, or from the stored
             // residual where this type and rank build that pass)

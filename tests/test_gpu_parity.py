@@ -11,6 +11,8 @@ Bars:
     accumulation term, and rel-L2 <= 4e-3 (a result rounded once to bf16 sits near 1.5e-3).
 All calls go through the C ABI (stacr_amd.kernels / the drop-in layer).
 """
+import contextlib
+
 import numpy as np
 import pytest
 import torch
@@ -65,6 +67,18 @@ def assert_rounded_once_bf16(got, exact, accum_abs=None, what="result"):
 
 def _np(t: torch.Tensor) -> np.ndarray:
     return t.detach().float().cpu().numpy()
+
+
+@contextlib.contextmanager
+def _kernel_names():
+    """The library kernels launched inside the block (a set, filled when it ends)."""
+    from stacr_amd import _lib
+
+    names = set()
+    with _lib.KernelTimer(max_launches=64) as timer:
+        yield names
+        torch.cuda.synchronize()
+    names.update(timer.results)
 
 
 def run_and_check_save(dev, rows, d, rank, dtype, mode, budget, chunk, bits, lognormal=False, seed=1234):
@@ -874,3 +888,25 @@ def test_weight_grad_census_refuses_a_census_too_small_for_the_problem(dev):
     small = census[: 8 * 512].clone()  # a census of a 512-feature layer
     with pytest.raises(ValueError, match="census has"):
         kernels.weight_grad(g, coeff, q, (idx, data, scale), 8, True, torch.bfloat16, census=small)
+
+
+@pytest.mark.parametrize("rows,d,rank,mode,budget,chunk,bits,lognormal", [
+    (5, 2064, 3, "global_topk", 0.003, 512, 8, False),     # two vectors past a thread a row, fewer rows than a batch
+    (33, 4096, 8, "chunk_topk", 0.005, 11, 0, True),       # chunks that batches of 8 rows do not divide: 1-row workgroups
+    (1030, 8128, 8, "chunk_topk", 0.005, 512, 4, False),   # the last vector's threads partly past the row, a trim
+    (7, 264, 16, "global_topk", 0.02, 512, 8, False),      # rank 16, a row of 33 vectors
+    (515, 6000, 13, "chunk_topk", 0.004, 100, 8, True),    # rank padded to 16, trailing workgroups without rows
+    (2052, 2048, 16, "global_topk", 0.005, 512, 8, True),  # histogram copies (513 workgroups), 4-list workgroups
+])
+def test_save_wide_candidate_lists_match_oracle(dev, rows, d, rank, mode, budget, chunk, bits, lognormal):
+    """bf16 rows of over 2048 features or rank 16: the projection pass forms the residual on the matrix cores
+    and keeps candidate lists.  Selection, codes and scale bit for bit against the oracle on the kernel's
+    coefficients, and the same on given coefficients."""
+    from stacr_amd import kernels
+
+    out = run_and_check_save(dev, rows, d, rank, "bf16", mode, budget, chunk, bits, lognormal)
+    idx, data, scale, coeff, xd, qd = out
+    with _kernel_names() as names:
+        _, i2, d2, s2 = kernels.save(xd, qd, mode=mode, budget=budget, chunk_rows=chunk, bits=bits, coeff=coeff)
+    assert "k_proj_cand_w" in names
+    assert torch.equal(i2, idx) and torch.equal(d2, data) and torch.equal(s2, scale)

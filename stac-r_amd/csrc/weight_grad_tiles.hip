@@ -33,8 +33,8 @@
 //     and at the end reduces the per-wave tiles over the waves (in wave order) and writes
 //     dW[o][f] = sum_j M[o][j] Q[f][j] + scale * (light sum + column sum).
 //   k_tile_wide   in place of k_tile_grad for problems with at least 256 workgroups of 32 outputs
-//     (the plan then selects no column features: every entry is a light record): one workgroup per
-//     (32 output features, part), the same three-buffer stream of G tiles and records, every entry
+//     (the plan then selects no column features: every entry is a light record, and orders a tile's
+//     records for the LDS banks): one workgroup per (32 or 64 output features, part), every entry
 //     summed on the matrix cores in chunks of 32 records (see the kernel).
 #include <type_traits>
 
@@ -100,7 +100,7 @@ struct TileArgs {
     int sparse;         // nnz > 0: the plan builds the entry structures
     int row_split;      // (no entries) workgroups over the rows of one o-slab; above 1 their M tiles go to mpart
     float *mpart;       // [o-slabs][row_split][256] the row ranges' M tiles (k_tile_lr_finish sums them)
-    int columns;        // the plan picks kNC column features per part (0: every entry is a light record)
+    int nj;             // 16-output tiles of a k_tile_wide workgroup (0: k_tile_grad)
     // division by d_in as a multiply-high and shifts (Granlund and Montgomery, "Division by invariant
     // integers using multiplication", 1994, figure 4.1): exact for every 32-bit dividend
     uint32_t div_m;
@@ -252,6 +252,22 @@ __global__ __launch_bounds__(kThreads) void k_tile_count(TileArgs a)
 }
 
 // ------------------------------------------------------------------ the plan
+// k_tile_wide's G tile in LDS: rows of nj x 32 bytes, 32 bytes of padding after each 1 KiB.  The place
+// of row t (of 512) in 32-byte units, and the row renumbered by class: the eight classes are the
+// places modulo 256 bytes, the LDS's width, so rows of different classes share no bank.  class_row is
+// class << 6 | the bits of t that the class does not fix.
+__device__ __forceinline__ uint32_t row_unit(int t, int nj)
+{
+    const uint32_t x = (uint32_t)(t * nj);
+    return x + (x >> 5);
+}
+
+__device__ __forceinline__ int class_row(int t, int nj)
+{
+    const int l = nj == 4 ? 3 : 4;  // log2 of the rows in 1 KiB
+    return (int)((row_unit(t, nj) & 7u) << 6) | (t >> (l + 3) << l) | (t & ((1 << l) - 1));
+}
+
 // Exclusive prefix sums of two values over the workgroup's threads in one exchange (two barriers);
 // the totals in *t0 and *t1.  s_tot2 holds 2 kWaves words.  Every thread must call it.
 __device__ __forceinline__ uint32_t block_exclusive_scan2(uint32_t v0, uint32_t v1, uint32_t *s_tot2, uint32_t *t0,
@@ -314,7 +330,8 @@ __device__ __forceinline__ int2 select_bin256(const uint32_t *__restrict__ h, ui
     return *res;
 }
 
-template <bool BT8>
+// WIDE: for k_tile_wide (no column features; its record order).
+template <bool BT8, bool WIDE>
 __global__ __launch_bounds__(kThreads) void k_tile_plan(TileArgs a)
 {
     using BE = typename std::conditional<BT8, uint8_t, uint16_t>::type;  // one column-operand element
@@ -324,8 +341,9 @@ __global__ __launch_bounds__(kThreads) void k_tile_plan(TileArgs a)
     __shared__ uint16_t s_pre[8 * kPartMax];     // light rows of feature f in words below 2 v, at v * kPartMax + f
     __shared__ uint32_t s_h[256];
     __shared__ int2 s_sel;
-    __shared__ __attribute__((aligned(16))) BE s_bt[kNC * kBtStride];  // the block's column entries [slot][t]
+    __shared__ __attribute__((aligned(16))) BE s_bt[WIDE ? 8 : kNC * kBtStride];  // the block's column entries [slot][t]
     __shared__ uint32_t s_tot[2 * kWaves];
+    __shared__ uint4 s_cls[WIDE ? kPartMax / 16 : 1];  // (k_tile_wide) records of each 16-feature tile by bank class, 16 bits each
 
     const int b = blockIdx.x, part = blockIdx.y, tid = threadIdx.x;
     // with entries, the workgroups past the last part pack the coefficient operands, in parallel
@@ -389,9 +407,9 @@ __global__ __launch_bounds__(kThreads) void k_tile_plan(TileArgs a)
         uint32_t cnt = 0;
 #pragma unroll
         for (int c = 0; c < kChunks; ++c) cnt += c < a.n_hist ? hv[c] : 0u;
-        cnt = tid < pw && a.columns ? (cnt < 0xffffu ? cnt : 0xffffu) : 0u;
+        cnt = tid < pw && !WIDE ? (cnt < 0xffffu ? cnt : 0xffffu) : 0u;
         s_slot[tid] = -1;
-        if (a.columns) {  // (uniform; without column features every entry is a light record)
+        if constexpr (!WIDE) {
             if (tid < 256) s_h[tid] = 0u;
             __syncthreads();
             {   // most features have fewer than 256 entries: bin 0 is added once per wave (a ballot
@@ -433,7 +451,7 @@ __global__ __launch_bounds__(kThreads) void k_tile_plan(TileArgs a)
 
         // ---- this block's entries: the column tile and the light bitmaps
         static_assert((kNC * kBtStride * sizeof(BE)) % 16 == 0, "the column tile clears in 16-byte words");
-        for (int i = tid; a.columns && i < (int)(kNC * kBtStride * sizeof(BE) / 16); i += kThreads)
+        for (int i = tid; !WIDE && i < (int)(kNC * kBtStride * sizeof(BE) / 16); i += kThreads)
             reinterpret_cast<uint4 *>(s_bt)[i] = make_uint4(0u, 0u, 0u, 0u);
         for (int i = tid; i < 16 * kPartMax / 4; i += kThreads)
             reinterpret_cast<uint4 *>(s_mask)[i] = make_uint4(0u, 0u, 0u, 0u);
@@ -462,7 +480,12 @@ __global__ __launch_bounds__(kThreads) void k_tile_plan(TileArgs a)
             before_part += f < 0;
             if (f < 0 || f >= pw) return;
             const int s = s_slot[f];
-            if (s >= 0) {
+            if constexpr (WIDE) {
+                const int tp = class_row(tl, a.nj);
+                atomicOr(&s_mask[(tp >> 5) * kPartMax + f], 1u << (tp & 31));
+                pko = (uint32_t)tl | ((uint32_t)f << 9);
+                v16 = to_g16(val[k], a.g_dt);
+            } else if (s >= 0) {
                 if constexpr (BT8) s_bt[s * kBtStride + tl] = (BE)(uint8_t)(int8_t)(int)val[k];
                 else s_bt[s * kBtStride + tl] = (BE)to_g16(val[k], a.g_dt);
             } else {
@@ -503,11 +526,30 @@ __global__ __launch_bounds__(kThreads) void k_tile_plan(TileArgs a)
         // light count of each feature; then, in one exchange, their offsets and the block's entries
         // in lower parts
         uint32_t lcnt = 0;
+        uint32_t ncls[4] = {0u, 0u, 0u, 0u};  // the feature's records of classes 2 i and 2 i + 1, 16 bits each
         if (tid < pw) {
 #pragma unroll
             for (int w = 0; w < 16; ++w) {
                 if (!(w & 1)) s_pre[(w >> 1) * kPartMax + tid] = (uint16_t)lcnt;
-                lcnt += __popc(s_mask[w * kPartMax + tid]);
+                const uint32_t bits = __popc(s_mask[w * kPartMax + tid]);
+                lcnt += bits;
+                ncls[w >> 2] += bits << (w & 2 ? 16 : 0);
+            }
+        }
+        if constexpr (WIDE) {
+            // s_pre becomes, per class, the records of the tile's lower features (a tile is a row of
+            // 16 lanes: a prefix sum by row shifts; at most 64 x 16 records a class)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                uint32_t x = ncls[i];
+                x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xf, 0xf, true);  // row_shr:1
+                x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xf, 0xf, true);  // row_shr:2
+                x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xf, 0xf, true);  // row_shr:4
+                x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xf, 0xf, true);  // row_shr:8
+                if ((tid & 15) == 15) reinterpret_cast<uint32_t *>(s_cls)[(tid >> 4) * 4 + i] = x;
+                x -= ncls[i];
+                s_pre[2 * i * kPartMax + tid] = (uint16_t)(x & 0xffffu);
+                s_pre[(2 * i + 1) * kPartMax + tid] = (uint16_t)(x >> 16);
             }
         }
         uint32_t n_light, all_before;
@@ -527,7 +569,25 @@ __global__ __launch_bounds__(kThreads) void k_tile_plan(TileArgs a)
         __syncthreads();
         // each light entry at its feature's offset + the feature's light entries in earlier rows
         // (blocks of at most kRounds rounds have them in registers already)
+        // (for k_tile_wide, at its tile's offset + its place in the tile: the tile's records by rank in
+        // their class, then by class, so that eight consecutive records are of eight classes)
         auto write_record = [&](int tl, int64_t f, uint32_t v16) {
+            if constexpr (WIDE) {
+                const int tp = class_row(tl, a.nj), w = tp >> 5;
+                const uint32_t v = (uint32_t)tp >> 6;
+                uint32_t r = s_pre[v * kPartMax + f] + __popc(s_mask[w * kPartMax + f] & ((1u << (tp & 31)) - 1u));
+                if (w & 1) r += __popc(s_mask[(w - 1) * kPartMax + f]);
+                const uint4 t = s_cls[f >> 4];
+                const uint32_t tw[4] = {t.x, t.y, t.z, t.w};
+                uint32_t pos = s_key[f & ~15];
+#pragma unroll
+                for (uint32_t i = 0; i < 4; ++i) {
+                    const uint32_t lo = tw[i] & 0xffffu, hi = tw[i] >> 16;
+                    pos += min(lo, r + (2 * i < v)) + min(hi, r + (2 * i + 1 < v));
+                }
+                reg[kOffWords + pos] = (uint32_t)(f & 15) | (row_unit(tl, a.nj) << 4) | (v16 << 16);
+                return;
+            }
             const int w = tl >> 5;
             uint32_t r = s_pre[(w >> 1) * kPartMax + f] + __popc(s_mask[w * kPartMax + f] & ((1u << (tl & 31)) - 1u));
             if (w & 1) r += __popc(s_mask[(w - 1) * kPartMax + f]);
@@ -559,7 +619,7 @@ __global__ __launch_bounds__(kThreads) void k_tile_plan(TileArgs a)
         // .. + 7 of column 16 i + l % 16, 8 elements
         using BV = typename std::conditional<BT8, uint2, uint4>::type;  // 8 elements
         BV *bt = static_cast<BV *>(a.bt) + ((int64_t)b * a.n_parts + part) * kNT * kWaves * 64;
-        for (int u = tid; a.columns && u < kNT * kWaves * 64; u += kThreads) {
+        for (int u = tid; !WIDE && u < kNT * kWaves * 64; u += kThreads) {
             const int l = u & 63, w = (u >> 6) & 15, i = u >> 10;
             bt[u] = *reinterpret_cast<const BV *>(s_bt + (16 * i + (l & 15)) * kBtStride + 32 * w + 8 * (l >> 4));
         }
@@ -1170,44 +1230,47 @@ __global__ __launch_bounds__(256) void k_tile_lr_finish(TileArgs a)
 }
 
 // ------------------------------------------------------------------ the wide streaming kernel
-// For problems large enough to fill the chip with 32-output slabs: one workgroup per (32 outputs,
-// part), every entry of the part a light record (the plan selects no column features).  Wave w
-// owns features 64 w .. 64 w + 63 of the part as four 16-feature tiles, whose records of a block
-// are contiguous (grouped by feature, then by row).  The wave takes each tile's records 32 at a
-// time as one chunk: the G rows of the 32 records, gathered by two transposing reads per 16
-// outputs, are the A operand; the records scatter their values into a zeroed [16 features][32
-// slots] LDS scratch at (feature in the tile, slot), the scratch read in operand order is the B
-// operand (cleared again after the read), and one v_mfma_f32_16x16x32 per 16 outputs adds
-// G[t_k][o] v_k to (o, feature).  So each wave's work is about its entry count / 32 + 4 matrix
-// instructions a block, whatever the spread of the entries over the features, and the sums have a
-// fixed order (chunks in record order, blocks in order).
-constexpr int kWOS = 32;         // outputs per workgroup
-constexpr int kWRecBuf = 3584;   // record words of a stream buffer
-constexpr int kWRecCap = kWRecBuf - 32;  // blocks with at most this many records read them from LDS
-                                         // (a chunk reads up to 31 words past its first record)
+// One workgroup per (16 NJ outputs, part), every entry of the part a light record (the plan selects
+// no column features).  Wave w owns the part's 16-feature tiles w, w + 16, w + 32 and w + 48, whose
+// records of a block are contiguous.  It takes each tile's records 32 at a time as one chunk: the G
+// rows of the 32 records, gathered by two transposing reads per 16 outputs, are the A operand; the
+// records scatter their values into a zeroed [16 features][32 slots] LDS scratch at (feature in the
+// tile, slot), the scratch read in operand order is the B operand (cleared again after the read),
+// and one v_mfma_f32_16x16x32 per 16 outputs adds G[t_k][o] v_k to (o, feature).  So each wave's
+// work is about its entry count / 32 + 2 chunks a block, whatever the spread of the entries over the
+// features, and the sums have a fixed order (chunks in record order, blocks in order).
+//
+// The LDS bounds it: 2 NJ gathers, one 16-byte read and two 2-byte stores a chunk.  A gather costs
+// 2.7 cycles when the eight rows that each half of the wave reads lie in different banks, 5.2 to
+// 6.9 for rows at random and 16 where they share them; the row padding and the plan's record order
+// (eight consecutive records of eight classes) make it the former, and more outputs a workgroup
+// spread the chunk's other 10 cycles.  The records go from memory to registers, a block ahead,
+// which leaves the LDS to two G tiles of 64 outputs.
+constexpr int kBsStride = 40;    // scratch elements a feature: 16 bytes past its 32 slots, so that 16 features'
+                                 // 16-byte reads fall in different banks
 
+template <int NJ>
 struct WideLds {
-    static constexpr size_t g = 0;                                  // [kTB][kWOS] G elements
-    static constexpr size_t rec = g + (size_t)kTB * kWOS * 2;       // [kWRecBuf] records
-    static constexpr size_t size = rec + (size_t)kWRecBuf * 4;      // 46 KiB
-    static_assert(size % 1024 == 0, "buffers start on 1 KiB boundaries");
-    static_assert(kWRecBuf % 256 == 0, "records are staged in 1 KiB copies");
-    static_assert(3 * size + kWaves * (1024 + 64) + kMaxBlocks * sizeof(TileHdr) <= 160 * 1024, "fits the CU's LDS");
-    static_assert(size >= (size_t)kWaves * 2 * 256 * 4, "every wave's two coefficient tiles fit a buffer");
-    static_assert(size >= (size_t)kPartMax * 16 * 2, "the part's Q rows fit a buffer");
+    static constexpr int copies = kTB * NJ * 32 / 1024;      // 1 KiB copies of a G tile
+    static constexpr int per_wave = copies / kWaves;         // NJ
+    static constexpr size_t pitch = 1024 + 32;               // LDS bytes from one copy to the next
+    static constexpr size_t g = copies * pitch;              // bytes of a G tile
+    static constexpr size_t total = 2 * g + (size_t)kWaves * (16 * kBsStride * 2 + 64) + kMaxBlocks * sizeof(TileHdr);
+    static_assert(total <= 160 * 1024, "fits the CU's LDS");
+    static_assert(g >= (size_t)kWaves * NJ * 256 * 4, "every wave's coefficient tiles fit a buffer");
+    static_assert(kTB * NJ + (kTB * NJ >> 5) <= 4096, "a row's place in 12 bits of a record");
 };
 
-template <int DT>
+template <int DT, int NJ>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_tile_wide(TileArgs a)
 {
-    using L = WideLds;
-    __shared__ __attribute__((aligned(1024))) unsigned char lds0[L::size];
-    __shared__ __attribute__((aligned(1024))) unsigned char lds1[L::size];
-    __shared__ __attribute__((aligned(1024))) unsigned char lds2[L::size];
-    __shared__ __attribute__((aligned(16))) uint16_t s_bs[kWaves * 512];  // per wave [16 features][32 slots]
+    using L = WideLds<NJ>;
+    __shared__ __attribute__((aligned(1024))) unsigned char lds0[L::g];
+    __shared__ __attribute__((aligned(1024))) unsigned char lds1[L::g];
+    __shared__ __attribute__((aligned(16))) uint16_t s_bs[kWaves * 16 * kBsStride];
     __shared__ uint16_t s_spare[kWaves * 32];  // per wave, a word each for the lanes whose stores go nowhere
     __shared__ TileHdr s_hdr[kMaxBlocks];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n = lane & 15, grp = lane >> 4;
 
     // workgroup -> (o-slab, part), consecutive logical ids on one XCD (as k_tile_grad)
@@ -1215,74 +1278,68 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4))
     int logical = blockIdx.x;
     if (nwg % 8 == 0) logical = (blockIdx.x % 8) * (nwg / 8) + blockIdx.x / 8;
     const int part = logical % a.n_parts;
-    const int64_t o0 = (int64_t)(logical / a.n_parts) * kWOS;
+    const int64_t o0 = (int64_t)(logical / a.n_parts) * (16 * NJ);
     const int64_t plo = (int64_t)part * a.part_w;
     const int pw = (int)(a.d_in - plo < a.part_w ? a.d_in - plo : a.part_w);
     const int nb = a.n_blocks;
 
     for (int b = tid; b < nb; b += kThreads) s_hdr[b] = a.hdr[b * a.n_parts + part];
-    uint16_t *bs = s_bs + wave * 512;
-    reinterpret_cast<uint4 *>(bs)[lane] = make_uint4(0u, 0u, 0u, 0u);  // 1 KiB: the scratch starts zero
+    for (int i = tid; i < kWaves * 16 * kBsStride / 8; i += kThreads)
+        reinterpret_cast<uint4 *>(s_bs)[i] = make_uint4(0u, 0u, 0u, 0u);  // the scratch starts zero
     __syncthreads();
 
     const uint32_t row_bytes = (uint32_t)a.d_out * 2;
-    const uint32_t g_lane_row = (uint32_t)tid >> 2;                        // + 256 for the second copy
-    const uint32_t g_lane_col = (uint32_t)o0 * 2 + 16u * (uint32_t)(tid & 3);
-    const uint32_t rec_lane = (256u * wave + 4u * lane) * 4;
     const uint32_t cp_lane = ((wave * 4u + grp) * a.ncol + n) * 16;
     const bool has_c = n < a.ncol;
     const uint32_t regions = (uint32_t)nb * (uint32_t)a.n_parts;
     const __amdgpu_buffer_rsrc_t r_cp = make_rsrc(a.cp, (uint64_t)nb * kTB * a.ncol * 2);
     const __amdgpu_buffer_rsrc_t r_light = make_rsrc(a.light, record_words(a.nnz, regions) * 4);
 
-    // A block with more records than a buffer stages runs as several windows of kWRecCap records
-    // over the same G tile ("steps"): step = (block, window), in order.  A step's state in scalar
-    // registers: its block, window, record region and count.
-    struct Step {
-        int blk;
-        uint32_t w, base, count;
-    };
-    auto windows = [&](uint32_t count) { return count <= (uint32_t)kWRecCap ? 1u : (count + kWRecCap - 1) / kWRecCap; };
-    auto step_at = [&](int blk, uint32_t w) {
-        const int b = blk < nb ? blk : nb - 1;
-        return Step{blk, w, (uint32_t)__builtin_amdgcn_readfirstlane(s_hdr[b].light_base),
-                    (uint32_t)__builtin_amdgcn_readfirstlane(s_hdr[b].light_count)};
-    };
-    auto next_step = [&](const Step &st) {
-        return st.w + 1 < windows(st.count) ? Step{st.blk, st.w + 1, st.base, st.count} : step_at(st.blk + 1, 0u);
-    };
-    // the step's records (window w: records [w kWRecCap, ..), the 1 KiB chunks it has) into buffer B
-    auto issue_records = [&](const Step &st, unsigned char *B) {
-        const uint32_t first = st.w * (uint32_t)kWRecCap;
-        const uint32_t left = st.count - first;
-#pragma unroll
-        for (int h = 0; h < kWRecBuf / 256; h += kWaves) {
-            const int c = h + wave;
-            if (c < kWRecBuf / 256 && 256u * (uint32_t)c < left)
-                copy16(r_light, B + L::rec + (size_t)c * 1024, rec_lane + (uint32_t)h * 1024,
-                       (st.base + kOffWords + first) * 4);
-        }
-    };
-    // block `blk`'s G tile [512 rows][32 outputs] into buffer B: two 16-byte copies a lane
-    auto issue_g = [&](int blk, unsigned char *B) {
-        const uint32_t rows_here = (uint32_t)(a.rows - (int64_t)blk * kTB) < (uint32_t)kTB
-                                       ? (uint32_t)(a.rows - (int64_t)blk * kTB) : (uint32_t)kTB;
+    // copy h of this wave's NJ of block `blk`'s G tile [512 rows][16 NJ outputs] into buffer B
+    constexpr int kRows = 32 / NJ, kPieces = 64 / kRows;  // rows of a 1 KiB copy, 16-byte pieces of a row
+    auto issue_g = [&](int blk, int h, unsigned char *B) {
+        const uint32_t left = (uint32_t)(a.rows - (int64_t)blk * kTB < kTB ? a.rows - (int64_t)blk * kTB : kTB);
         const __amdgpu_buffer_rsrc_t r_g =
-            make_rsrc(static_cast<const char *>(a.g) + (size_t)blk * kTB * row_bytes, (uint64_t)rows_here * row_bytes);
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const uint32_t row = g_lane_row + 256u * h;
-            const uint32_t r = row < rows_here - 1 ? row : rows_here - 1;
-            copy16(r_g, B + L::g + (size_t)h * 16384 + (size_t)wave * 1024, r * row_bytes + g_lane_col, 0u);
-        }
+            make_rsrc(static_cast<const char *>(a.g) + (size_t)blk * kTB * row_bytes, (uint64_t)left * row_bytes);
+        const int c = h * kWaves + wave;
+        const uint32_t row = (uint32_t)(c * kRows + lane / kPieces);
+        const uint32_t r = row < left - 1 ? row : left - 1;
+        copy16(r_g, B + (size_t)c * L::pitch, r * row_bytes + (uint32_t)o0 * 2 + 16u * (uint32_t)(lane % kPieces), 0u);
     };
-    // this wave's tile bounds of the step's block: lane i <= 4 loads the offset of feature
-    // 64 w + 16 i (the part's end past pw), clamped to the block's records
-    auto load_bounds = [&](const Step &st) {
-        const int f = 64 * wave + 16 * (lane < 5 ? lane : 4);
-        const uint32_t fo = (uint32_t)(f < pw ? f : pw);
-        const uint32_t v = __builtin_amdgcn_raw_buffer_load_b32(r_light, (int)(fo * 4), (int)(st.base * 4), 0);
-        return v < st.count ? v : st.count;
+
+    // the wave's records of a block: its tiles' ranges [l[i], h[i])
+    struct Block {
+        uint32_t first;  // the region's first record, in words of the array
+        uint32_t l[4], h[4];
+    };
+    // lane 2 i + e <= 7 loads the offset of feature 16 (w + 16 i + e) (the part's end past pw)
+    auto load_bounds = [&](int blk, const TileHdr *__restrict__ hdr) {
+        const int b = blk < nb ? blk : nb - 1;
+        const int f = 16 * (wave + 16 * ((lane >> 1) & 3) + (lane & 1));
+        const uint32_t base = (uint32_t)__builtin_amdgcn_readfirstlane(hdr[b].light_base);
+        return (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(r_light, (f < pw ? f : pw) * 4, (int)(base * 4), 0);
+    };
+    auto block_of = [&](int blk, uint32_t v, const TileHdr *__restrict__ hdr) {
+        const int b = blk < nb ? blk : nb - 1;
+        Block k;
+        const uint32_t count = (uint32_t)__builtin_amdgcn_readfirstlane(hdr[b].light_count);
+        k.first = (uint32_t)__builtin_amdgcn_readfirstlane(hdr[b].light_base) + kOffWords;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t lo = __builtin_amdgcn_readlane(v, 2 * i), hi = __builtin_amdgcn_readlane(v, 2 * i + 1);
+            k.h[i] = hi < count ? hi : count;
+            k.l[i] = lo < k.h[i] ? lo : k.h[i];
+        }
+        return k;
+    };
+    // The records come 64 at a time, a pair of chunks: lane 16 g + 4 q + 2 p + h of a load holds, for
+    // its chunk p, the record of slot 8 g + 4 h + q.  So the quad's lanes 2 p and 2 p + 1 hold slots
+    // k1 = 8 g + q and k1 + 4, whose rows this lane's transposing reads need, and the slots of one
+    // read's half wave (g, g + 1; q) are eight consecutive records.
+    const uint32_t slot = 8u * grp + 4u * (lane & 1) + ((lane >> 2) & 3);
+    const uint32_t my = 16u * (grp >> 1) + 8u * (lane & 1) + 4u * (grp & 1) + ((lane >> 2) & 3) + 16u * (lane & 2);
+    auto load_records = [&](uint32_t word) {
+        return (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(r_light, (int)(my * 4), (int)(word * 4), 0);
     };
     auto load_c = [&](int blk) {
         uint4 c = make_uint4(0u, 0u, 0u, 0u);
@@ -1290,214 +1347,189 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4))
         return c;
     };
 
-    f32x4 acc_m[2], acc[4][2];
+    f32x4 acc_m[NJ], acc[4][NJ];
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
+    for (int j = 0; j < NJ; ++j) {
         acc_m[j] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int i = 0; i < 4; ++i) acc[i][j] = acc_m[j];
     }
-
-    // Each chunk is up to 32 consecutive records of one of the wave's four tiles (a tile's records
-    // are grouped by feature, the tiles' ranges follow each other).  Lane 16 g + 4 q + h (h = 0, 1) holds the record
-    // of slot 8 g + 4 h + q (lanes with h = 2, 3 repeat h = 0, 1): so the quad's first two lanes
-    // hold slots k1 = 8 g + q and k1 + 4, the rows this lane's transposing reads need, and
-    // every slot < 32 is held once by a lane with h < 2, which scatters its value.
-    const uint32_t my = 8u * grp + 4u * (lane & 1) + ((lane >> 2) & 3);  // the slot this lane holds
-    const bool scatters = (lane & 2) == 0;
+    uint32_t pr[4][2];    // the first two pairs of each of the wave's tiles, loaded a block ahead
+    uint4 cop;            // the wave's coefficient operand, loaded a block ahead
     uint16_t *spare = s_spare + wave * 32 + 2 * (lane >> 2) + (lane & 1);
-    // the scratch row of feature f keeps its four 16-byte slot groups rotated by rot(f): a 16-byte
-    // read is served eight lanes a cycle over 32 banks, and (f & 1, rot(f)) differ across each eight
-    // consecutive features (a rotation by f's bits 2..3 alone gave every read two cycles of conflicts)
-    // rot(f) = f2 | (f1 ^ f2 ^ f3) << 1, two bits a feature of the constant
-    auto rot = [](uint32_t f) { return (0xf50a5fa0u >> (2u * f)) & 3u; };
-    const uint16_t *bsrd_lane = s_bs + wave * 512 + n * 32 + 8 * (grp ^ rot((uint32_t)n));
-    const uint32_t ga_lane = (n & 3) * 4;
+    const uint32_t row_lane = (n & 3) * 8;  // this lane's bytes of a gathered row
 
-    // the step in buffer B: (window 0) M = G^T [C | 1] over the wave's 32 rows, then the wave's
-    // records of the window as chunks
-    auto run_step = [&](const Step &st, const unsigned char *B, uint4 cop, uint32_t bnd) {
-        const uint16_t *gt = reinterpret_cast<const uint16_t *>(B + L::g);
-        if (st.w == 0) {
-            const int kk = 32 * wave + 8 * grp;
-            const uint16_t *pa = gt + (kk + (n >> 2)) * kWOS + (n & 3) * 4;
+    uint32_t bnd;         // the tile bounds of the block after the next one
+    // block blk in buffer B, while block blk + 1 is copied into buffer B2: M = G^T [C | 1] over the
+    // wave's 32 rows, then the wave's records c; returns the next block's.  (Every LDS access is
+    // through a restrict parameter, or the compiler would make it wait for the copies in flight.)
+    auto run_block = [&](int blk, const Block &c, const unsigned char *__restrict__ B, unsigned char *__restrict__ B2,
+                         uint16_t *__restrict__ bs, const TileHdr *__restrict__ hdr) {
+        const Block x = block_of(blk + 1, bnd, hdr);
+        bnd = load_bounds(blk + 2, hdr);
+        {
+            const int t = 32 * wave + 8 * grp + (n >> 2);
+            const unsigned char *p1 = B + 32 * row_unit(t, NJ) + row_lane, *p2 = B + 32 * row_unit(t + 4, NJ) + row_lane;
 #pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                const uint2 lo = lds_tr16(pa + 16 * j), hi = lds_tr16(pa + 16 * j + 4 * kWOS);
+            for (int j = 0; j < NJ; ++j) {
+                const uint2 lo = lds_tr16(reinterpret_cast<const uint16_t *>(p1 + 32 * j));
+                const uint2 hi = lds_tr16(reinterpret_cast<const uint16_t *>(p2 + 32 * j));
                 acc_m[j] = mfma16<DT>(make_uint4(lo.x, lo.y, hi.x, hi.y), cop, acc_m[j]);
             }
         }
-        const uint32_t *recs = reinterpret_cast<const uint32_t *>(B + L::rec);
-        // tile i spans records [b_i, b_i+1) of the block (every value here is wave-uniform)
-        const uint32_t b0 = __builtin_amdgcn_readlane(bnd, 0);
-        uint32_t b1 = __builtin_amdgcn_readlane(bnd, 1), b2 = __builtin_amdgcn_readlane(bnd, 2);
-        uint32_t b3 = __builtin_amdgcn_readlane(bnd, 3), b4 = __builtin_amdgcn_readlane(bnd, 4);
-        b1 = b1 > b0 ? b1 : b0;
-        b2 = b2 > b1 ? b2 : b1;
-        b3 = b3 > b2 ? b3 : b2;
-        b4 = b4 > b3 ? b4 : b3;
-        const uint32_t bb[5] = {b0, b1, b2, b3, b4};
-        // the window's records [w0, w1) staged from recs[0]; this wave's part of them [lo, hi)
-        const uint32_t w0 = st.w * (uint32_t)kWRecCap;
-        const uint32_t w1 = st.count - w0 < (uint32_t)kWRecCap ? st.count : w0 + kWRecCap;
-        uint16_t *bs = s_bs + wave * 512;
-        const uint16_t *ga = gt + ga_lane;
-        // this wave's records in the window
-        const uint32_t lo = b0 > w0 ? b0 : w0, hi0 = b4 < w1 ? b4 : w1, hi = hi0 > lo ? hi0 : lo;
-        // one chunk of tile i at records [e0, e0 + 32) (slots at or past t_hi hold whatever follows:
-        // the next tile's records or a stale word of the buffer; their lanes store zero, and the G
-        // row they address is in the tile, t & 511): A = the G rows of slots k1 (.. + 3 over the
-        // group) and k1 + 4, per 16 outputs; B = the tile's values at (feature in the tile, slot) of
-        // the zeroed scratch (rows of 32 slots, the four 16-byte groups of a row rotated by rot(f)),
-        // cleared again after the read; one product per 16 outputs.  Every lane stores unconditionally: a lane past
-        // t_hi stores zero at its own slot, which no other lane of the chunk writes and which is
-        // zero already, and the lanes that repeat another's record store into their spare word.
-        auto chunk = [&](f32x4 (&ac)[2], uint32_t rec, uint32_t e0, uint32_t t_hi) {
-            const uint32_t r1 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)rec, 0x00, 0xf, 0xf, false);
-            const uint32_t r2 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)rec, 0x55, 0xf, 0xf, false);
-            const uint16_t *p1 = ga + (r1 & 511u) * kWOS;
-            const uint16_t *p2 = ga + (r2 & 511u) * kWOS;
-            const uint2 lo0 = lds_tr16(p1), hi0 = lds_tr16(p2);
-            const uint2 lo1 = lds_tr16(p1 + 16), hi1 = lds_tr16(p2 + 16);
-            const uint4 a0 = make_uint4(lo0.x, lo0.y, hi0.x, hi0.y), a1 = make_uint4(lo1.x, lo1.y, hi1.x, hi1.y);
-            const uint32_t fo = (rec >> 9) & 15u;
-            uint16_t *slot = scatters ? bs + fo * 32 + 8 * ((my >> 3) ^ rot(fo)) + (my & 7) : spare;
-            const uint16_t v = e0 + my < t_hi ? (uint16_t)(rec >> 16) : (uint16_t)0;
+        cop = load_c(blk + 1);
+        if (blk + 1 < nb) {
+#pragma unroll
+            for (int h = 0; h < L::per_wave; ++h) issue_g(blk + 1, h, B2);
+        }
+        // one chunk: A = the G rows of slots k1 (.. + 3 over the group) and k1 + 4, per 16 outputs;
+        // B = the values at (feature in the tile, slot) of the zeroed scratch, cleared again after the
+        // read; one product per 16 outputs.  Every lane stores unconditionally: a lane past the tile's
+        // records (its record zero) stores zero at its own slot, which no other lane of the chunk writes
+        // and which is zero already, and the other chunk's lanes store into their spare word.
+        auto chunk = [&](f32x4 (&ac)[NJ], uint32_t rec, auto second) {
+            constexpr int kQ = decltype(second)::value ? 0xaa : 0x00;  // quad_perm 2,2,2,2 or 0,0,0,0
+            const uint32_t r1 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)rec, kQ, 0xf, 0xf, false);
+            const uint32_t r2 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)rec, kQ + 0x55, 0xf, 0xf, false);
+            const unsigned char *p1 = B + (row_lane + ((r1 & 0xfff0u) << 1));
+            const unsigned char *p2 = B + (row_lane + ((r2 & 0xfff0u) << 1));
+            uint16_t *sl = bs + (rec & 15u) * kBsStride + slot;
+            sl = ((lane & 2) != 0) == decltype(second)::value ? sl : spare;
             // The lanes exchange values through the scratch: wavefront-scope fences keep the
             // compiler from moving one lane's store across another lane's load (a wave's LDS
             // operations are performed in order, so they cost no wait).
-            *slot = v;
+            *sl = (uint16_t)(rec >> 16);
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-            const uint4 bop = *reinterpret_cast<const uint4 *>(bsrd_lane);
+            const uint4 bop = *reinterpret_cast<const uint4 *>(bs + n * kBsStride + 8 * grp);
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-            *slot = 0;
+            *sl = 0;
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-            ac[0] = mfma16<DT>(a0, bop, ac[0]);
-            ac[1] = mfma16<DT>(a1, bop, ac[1]);
-        };
-        // tile by tile, the tile's records of the window [max(b_i, lo), min(b_i+1, hi)) in chunks,
-        // each chunk's record read before the previous one runs.  The chunks follow each other in
-        // record order (a tile's first record is where the previous tile's ended), so the next
-        // start is always e0 + 32 or the tile's end; its index, at most hi - w0 + 31 <= kWRecCap +
-        // 31, is inside the buffer.
-        if (lo < hi) {
-            uint32_t nx = recs[lo - w0 + my];
+            uint4 av[NJ];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const uint32_t t_lo = bb[i] > lo ? bb[i] : lo;
-                const uint32_t t_hi = bb[i + 1] < hi ? bb[i + 1] : hi;
-                for (uint32_t e0 = t_lo; e0 < t_hi; e0 += 32) {
-                    const uint32_t cur = nx;
-                    nx = recs[(e0 + 32 < t_hi ? e0 + 32 : t_hi) - w0 + my];
-                    chunk(acc[i], cur, e0, t_hi);
-                }
+            for (int j = 0; j < NJ; ++j) {
+                const uint2 lo = lds_tr16(reinterpret_cast<const uint16_t *>(p1 + 32 * j));
+                const uint2 hi = lds_tr16(reinterpret_cast<const uint16_t *>(p2 + 32 * j));
+                av[j] = make_uint4(lo.x, lo.y, hi.x, hi.y);
+            }
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) ac[j] = mfma16<DT>(av[j], bop, ac[j]);
+        };
+        auto pair = [&](f32x4 (&ac)[NJ], uint32_t rec, uint32_t left) {  // (left: the tile's records from the pair's first on)
+            rec = my < left ? rec : 0u;
+            chunk(ac, rec, std::false_type());
+            if (left > 32) chunk(ac, rec, std::true_type());
+        };
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t left = c.h[i] - c.l[i];
+            if (left > 0) pair(acc[i], pr[i][0], left);
+            if (left > 64) pair(acc[i], pr[i][1], left - 64);
+            pr[i][0] = load_records(x.first + x.l[i]);
+            pr[i][1] = load_records(x.first + x.l[i] + 64);
+        }
+        // tiles with more pairs than are loaded ahead
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            if (c.h[i] - c.l[i] > 128) {
+                uint32_t e = c.l[i] + 128, r = load_records(c.first + e);
+                do {
+                    const uint32_t r_here = r;
+                    r = load_records(c.first + e + 64);
+                    pair(acc[i], r_here, c.h[i] - e);
+                    e += 64;
+                } while (e < c.h[i]);
+                // (the last load is not used: landed here, or the compiler waits for it where its
+                // register is next written, in every block)
+                __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
             }
         }
+        // the copies have landed: the eight record loads above are younger
+        __builtin_amdgcn_s_waitcnt(0x0078);  // vmcnt(8) lgkmcnt(0)
+        return x;
     };
 
-    // ---- the stream: step v runs in buffer v % 3 while step v + 2 is copied into buffer
-    // (v + 2) % 3; the operands (C, tile bounds) of step v + 1 are loaded into registers.  (The
-    // states of steps v, v + 1 and v + 2 are carried in scalar registers; a step past the last
-    // repeats the last block's copies into a buffer nothing reads any more.)
-    int n_steps = 0;
-    for (int b = 0; b < nb; ++b) n_steps += (int)windows((uint32_t)__builtin_amdgcn_readfirstlane(s_hdr[b].light_count));
-    Step s0 = step_at(0, 0u);
-    Step s1 = next_step(s0);
-    Step s2 = next_step(s1);
-    uint4 cop = load_c(0);
-    uint32_t bnd = load_bounds(s0);
-    issue_records(s0, lds0);
-    issue_g(0, lds0);
-    if (n_steps > 1) {
-        issue_records(s1, lds1);
-        issue_g(s1.blk < nb ? s1.blk : nb - 1, lds1);
+    // ---- the stream: block v runs in buffer v % 2 while block v + 1 is copied into the other; the
+    // operands of block v + 1 and the tile bounds of block v + 2 are loaded into registers
+    Block cur = block_of(0, load_bounds(0, s_hdr), s_hdr);
+    bnd = load_bounds(1, s_hdr);
+    cop = load_c(0);
+#pragma unroll
+    for (int h = 0; h < L::per_wave; ++h) issue_g(0, h, lds0);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        pr[i][0] = load_records(cur.first + cur.l[i]);
+        pr[i][1] = load_records(cur.first + cur.l[i] + 64);
     }
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
-    auto step = [&](int v, const unsigned char *__restrict__ B, unsigned char *__restrict__ B2) {
-        const uint4 c_here = cop;
-        const uint32_t b_here = bnd;
-        cop = load_c(s1.blk);
-        bnd = load_bounds(s1);
-        if (v + 2 < n_steps) issue_records(s2, B2);
-        run_step(s0, B, c_here, b_here);
-        issue_g(s2.blk < nb ? s2.blk : nb - 1, B2);
-        const Step s3 = next_step(s2);
-        __builtin_amdgcn_s_waitcnt(0x0072);  // vmcnt(2) lgkmcnt(0): only the two G copies stay in flight
+    for (int v = 0; v < nb; ++v) {
+        cur = run_block(v, cur, v & 1 ? lds1 : lds0, v & 1 ? lds0 : lds1, s_bs + wave * 16 * kBsStride, s_hdr);
         asm volatile("s_barrier" ::: "memory");
-        s0 = s1;
-        s1 = s2;
-        s2 = s3;
-    };
-    int cb = 0;
-    for (int v = 0; v + 1 < n_steps; ++v, cb = cb == 2 ? 0 : cb + 1) {
-        unsigned char *B = cb == 0 ? lds0 : cb == 1 ? lds1 : lds2;
-        unsigned char *B2 = cb == 0 ? lds2 : cb == 1 ? lds0 : lds1;
-        step(v, B, B2);
     }
-    run_step(s0, cb == 0 ? lds0 : cb == 1 ? lds1 : lds2, cop, bnd);
 
     const float scale = a.bits ? *a.scale : 1.f;
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
 
-    // ---- M over the waves, in wave order: every wave's two tiles staged in lds0, sums in lds2;
-    // the part's Q rows (16-bit) in lds1
+    // ---- M over the waves, in wave order: every wave's tiles staged in lds0, sums in lds1
     float *stage = reinterpret_cast<float *>(lds0);
-    float *fin = reinterpret_cast<float *>(lds2);  // [2][16 o][16 j]
-    uint16_t *sq = reinterpret_cast<uint16_t *>(lds1);
+    float *fin = reinterpret_cast<float *>(lds1);  // [NJ][16 o][16 j]
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+    for (int j = 0; j < NJ; ++j)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) stage[(wave * 2 + j) * 256 + (4 * grp + r) * 16 + n] = acc_m[j][r];
-    const uint16_t *q = static_cast<const uint16_t *>(a.q);
-    for (int e = tid; e < pw * a.rank; e += kThreads) sq[e] = q[plo * a.rank + e];
+        for (int r = 0; r < 4; ++r) stage[(wave * NJ + j) * 256 + (4 * grp + r) * 16 + n] = acc_m[j][r];
     __syncthreads();
-    if (tid < 512) {
+    if (tid < 256 * NJ) {
         float sum = 0.f;
-        for (int w = 0; w < kWaves; ++w) sum += stage[(w * 2 + (tid >> 8)) * 256 + (tid & 255)];
+        for (int w = 0; w < kWaves; ++w) sum += stage[(w * NJ + (tid >> 8)) * 256 + (tid & 255)];
         fin[tid] = sum;
     }
     __syncthreads();
 
     // ---- dW: lane (n, grp) of wave w holds, per tile i and o-tile j, outputs 16 j + 4 grp .. + 3 of
-    // feature 64 w + 16 i + n
+    // feature 16 (w + 16 i) + n
+    const uint16_t *q = static_cast<const uint16_t *>(a.q);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        const int fl = 64 * wave + 16 * i + n;
+        const int fl = 16 * (wave + 16 * i) + n;
         if (fl >= pw) continue;
         const int64_t f = plo + fl;
+        float out[NJ][4];
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            float out[4];
+        for (int j = 0; j < NJ; ++j)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) out[r] = scale * acc[i][j][r];
-            for (int c = 0; c < a.rank; ++c) {
-                const float qc = g16_to_f<DT>(sq[fl * a.rank + c]);
+            for (int r = 0; r < 4; ++r) out[j][r] = scale * acc[i][j][r];
+        for (int c = 0; c < a.rank; ++c) {
+            const float qc = g16_to_f<DT>(q[f * a.rank + c]);
 #pragma unroll
-                for (int r = 0; r < 4; ++r) out[r] = fmaf(fin[j * 256 + (4 * grp + r) * 16 + c], qc, out[r]);
-            }
+            for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) out[j][r] = fmaf(fin[j * 256 + (4 * grp + r) * 16 + c], qc, out[j][r]);
+        }
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
             const int64_t o = o0 + 16 * j + 4 * grp;
             if (a.transposed) {  // Conv1D: dW is d_in x d_out, four consecutive outputs
                 if (a.dw_dt == STACR_DTYPE_F32) {
                     *reinterpret_cast<float4 *>(static_cast<float *>(a.dw) + f * a.d_out + o) =
-                        make_float4(out[0], out[1], out[2], out[3]);
+                        make_float4(out[j][0], out[j][1], out[j][2], out[j][3]);
                 } else {
                     const bool bf = a.dw_dt == STACR_DTYPE_BF16;
                     uint32_t wv[2];
 #pragma unroll
                     for (int k = 0; k < 2; ++k)
-                        wv[k] = bf ? (f_to_bf16_bits(out[2 * k]) | (f_to_bf16_bits(out[2 * k + 1]) << 16))
-                                   : (f_to_f16_bits(out[2 * k]) | (f_to_f16_bits(out[2 * k + 1]) << 16));
+                        wv[k] = bf ? (f_to_bf16_bits(out[j][2 * k]) | (f_to_bf16_bits(out[j][2 * k + 1]) << 16))
+                                   : (f_to_f16_bits(out[j][2 * k]) | (f_to_f16_bits(out[j][2 * k + 1]) << 16));
                     *reinterpret_cast<uint2 *>(static_cast<uint16_t *>(a.dw) + f * a.d_out + o) = make_uint2(wv[0], wv[1]);
                 }
             } else {  // nn.Linear: dW is d_out x d_in
 #pragma unroll
-                for (int r = 0; r < 4; ++r) store_any(a.dw, a.dw_dt, (o + r) * a.d_in + f, out[r]);
+                for (int r = 0; r < 4; ++r) store_any(a.dw, a.dw_dt, (o + r) * a.d_in + f, out[j][r]);
             }
         }
     }
-    if (a.dbias && part == 0 && tid < kWOS) store_any(a.dbias, a.db_dt, o0 + tid, fin[(tid >> 4) * 256 + (tid & 15) * 16 + a.bias_col]);
+    if (a.dbias && part == 0 && tid < 16 * NJ)
+        store_any(a.dbias, a.db_dt, o0 + tid, fin[(tid >> 4) * 256 + (tid & 15) * 16 + a.bias_col]);
 }
 
 }  // namespace
@@ -1509,12 +1541,16 @@ struct TileGeom {
     int n_blocks, n_parts, part_w, ncol, bias_col;
     int gb;  // bytes of a G / C element
     bool sparse, bt8;
-    bool wide;  // k_tile_wide (every entry a light record, no column operands) in place of k_tile_grad
+    int nj;     // 16-output tiles of a k_tile_wide workgroup (every entry a light record); 0: k_tile_grad
     int row_split;  // (no entries) k_tile_grad workgroups over the rows of one o-slab
 };
 
-// Workgroups of the wide kernel that make it the better choice: at least one per CU (256) with
-// 32-output slabs.  Below that the 16-output kernel's twice as many workgroups fill the chip better.
+// Workgroups of 32 outputs that make the wide kernel the better choice: one per CU.  Below that the
+// 16-output kernel's column features win where a few features hold most entries (at 128 workgroups,
+// 8192 rows, 1 % kept: 41 against 69 us with lognormal features, but 66 against 55 with Gaussian
+// ones, which the host cannot tell apart).  A second round of workgroups costs more than 64 outputs a
+// workgroup do (8192 rows of 1024 features, 1 % kept, 32 against 64 outputs: d_out 8192 78 and
+// 104 us, 12288 144 and 108, 16384 161 and 117).
 constexpr int kWideMinWgs = 256;
 
 bool tile_geom(const StacrGradArgs &a, TileGeom *g)
@@ -1540,7 +1576,8 @@ bool tile_geom(const StacrGradArgs &a, TileGeom *g)
     g->gb = f32 ? 4 : 2;
     g->sparse = a.nnz > 0;
     g->bt8 = a.bits != 0;
-    g->wide = g->sparse && !f32 && a.d_out % kWOS == 0 && (a.d_out / kWOS) * g->n_parts >= kWideMinWgs;
+    const int64_t wide = g->sparse && !f32 && a.d_out % 32 == 0 ? a.d_out / 32 * g->n_parts : 0;
+    g->nj = wide < kWideMinWgs ? 0 : a.d_out % 64 || wide == kWideMinWgs ? 2 : 4;
     // without entries a workgroup's results are its M tile alone, so the rows of each o-slab are
     // split (at least two blocks a workgroup) until the launch fills the chip evenly; the tiles are
     // summed in a fixed order by k_tile_lr_finish
@@ -1563,7 +1600,7 @@ size_t tile_layout(int64_t nnz, int64_t d_in, int64_t d_out, const TileGeom &g, 
     take(TW_HIST, g.sparse ? (size_t)kChunks * d_in * 4 : 0);
     take(TW_BSTART, g.sparse ? ((size_t)g.n_blocks + 1) * 4 : 0);
     take(TW_CP, (size_t)g.n_blocks * kTB * g.ncol * g.gb);
-    take(TW_BT, g.sparse && !g.wide ? bt_bytes : 0);
+    take(TW_BT, g.sparse && !g.nj ? bt_bytes : 0);
     take(TW_LIGHT, g.sparse ? (size_t)record_words(nnz, regions) * 4 : 0);
     take(TW_HDR, g.sparse ? regions * sizeof(TileHdr) : 0);
     take(TW_COLMAP, g.sparse ? (size_t)g.n_parts * kNC * 4 : 0);
@@ -1583,6 +1620,17 @@ int launch_tile_grad_dt(const TileArgs &t, const TileGeom &g, int nwg, hipStream
 {
     if (!g.sparse) return launch_tile_grad<DT, false, true>(t, nwg, s);
     return g.bt8 ? launch_tile_grad<DT, true, true>(t, nwg, s) : launch_tile_grad<DT, true, false>(t, nwg, s);
+}
+
+template <int DT>
+int launch_tile_wide(const TileArgs &t, const TileGeom &g, hipStream_t s)
+{
+    const int nwg = (int)(t.d_out / (16 * g.nj)) * g.n_parts;
+    stacr_launch("k_tile_wide", s, [&] {
+        if (g.nj == 4) k_tile_wide<DT, 4><<<nwg, kThreads, 0, s>>>(t);
+        else k_tile_wide<DT, 2><<<nwg, kThreads, 0, s>>>(t);
+    });
+    return stacr_hip_check(hipGetLastError(), "weight_grad wide matrix-core kernel");
 }
 
 }  // namespace
@@ -1612,7 +1660,7 @@ size_t stacr_tiles_ws_bound(int64_t rows, int64_t d_out, int64_t d_in, int64_t n
     g.gb = 4;       // fp32 coefficient operands
     g.sparse = nnz > 0;
     g.bt8 = false;  // the wider column-operand form
-    g.wide = false;  // (with column operands: the larger layout)
+    g.nj = 0;        // (with column operands: the larger layout)
     g.row_split = nnz > 0 ? 1 : kMaxRowSplit;  // (the most M tiles)
     size_t off[TW_N];
     return tile_layout(nnz, d_in, d_out, g, off);
@@ -1670,7 +1718,7 @@ int stacr_tiles_launch(const StacrGradArgs &a)
     t.sparse = g.sparse ? 1 : 0;
     t.row_split = g.row_split;
     t.mpart = reinterpret_cast<float *>(ws + off[TW_MPART]);
-    t.columns = g.wide ? 0 : 1;
+    t.nj = g.nj;
     div_magic((uint32_t)a.d_in, &t.div_m, &t.div_s1, &t.div_s2);
     hipStream_t s = a.stream;
     int rc;
@@ -1680,18 +1728,16 @@ int stacr_tiles_launch(const StacrGradArgs &a)
         if (rc) return rc;
     }
     const dim3 pgrid((unsigned)g.n_blocks, g.sparse ? (unsigned)g.n_parts + 1u : 1u);
-    if (g.bt8) stacr_launch("k_tile_plan", s, [&] { k_tile_plan<true><<<pgrid, kThreads, 0, s>>>(t); });
-    else stacr_launch("k_tile_plan", s, [&] { k_tile_plan<false><<<pgrid, kThreads, 0, s>>>(t); });
+    stacr_launch("k_tile_plan", s, [&] {
+        if (g.nj) k_tile_plan<true, true><<<pgrid, kThreads, 0, s>>>(t);
+        else if (g.bt8) k_tile_plan<true, false><<<pgrid, kThreads, 0, s>>>(t);
+        else k_tile_plan<false, false><<<pgrid, kThreads, 0, s>>>(t);
+    });
     rc = stacr_hip_check(hipGetLastError(), "weight_grad plan");
     if (rc) return rc;
-    if (g.wide) {
-        const int nw = (int)(a.d_out / kWOS) * g.n_parts;
-        if (a.dtype == STACR_DTYPE_BF16)
-            stacr_launch("k_tile_wide", s, [&] { k_tile_wide<STACR_DTYPE_BF16><<<nw, kThreads, 0, s>>>(t); });
-        else
-            stacr_launch("k_tile_wide", s, [&] { k_tile_wide<STACR_DTYPE_F16><<<nw, kThreads, 0, s>>>(t); });
-        return stacr_hip_check(hipGetLastError(), "weight_grad wide matrix-core kernel");
-    }
+    if (g.nj)
+        return a.dtype == STACR_DTYPE_BF16 ? launch_tile_wide<STACR_DTYPE_BF16>(t, g, s)
+                                           : launch_tile_wide<STACR_DTYPE_F16>(t, g, s);
     const int nwg = (int)(a.d_out / kOS) * g.n_parts * g.row_split;
     if (a.dtype == STACR_DTYPE_F32) return launch_tile_grad<STACR_DTYPE_F32, true, true>(t, nwg, s);
     rc = a.dtype == STACR_DTYPE_BF16 ? launch_tile_grad_dt<STACR_DTYPE_BF16>(t, g, nwg, s)

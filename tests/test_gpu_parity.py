@@ -910,3 +910,40 @@ def test_save_wide_candidate_lists_match_oracle(dev, rows, d, rank, mode, budget
         _, i2, d2, s2 = kernels.save(xd, qd, mode=mode, budget=budget, chunk_rows=chunk, bits=bits, coeff=coeff)
     assert "k_proj_cand_w" in names
     assert torch.equal(i2, idx) and torch.equal(d2, data) and torch.equal(s2, scale)
+
+
+@pytest.mark.parametrize("rows,d_in,d_out,rank,dtype,transposed,bits", [
+    (513, 1000, 16384, 8, "bf16", False, 8),    # 64 outputs a workgroup; a one-row block, a partial feature tile
+    (1100, 1025, 8192, 15, "bf16", True, 0),    # 64 outputs; two parts, each ending in a tile of one feature
+    (1536, 1024, 8224, 5, "f16", False, 4),     # d_out not a multiple of 64: 32 outputs a workgroup
+    (700, 777, 8192, 3, "f16", True, 8),        # exactly 256 workgroups of 32 outputs
+])
+def test_weight_grad_wide_tiles_at_their_edges(dev, rows, d_in, d_out, rank, dtype, transposed, bits):
+    """The wide kernel's two slab widths, with features whose tile holds more records a block than are loaded
+    ahead and rows whose records fall in one bank class."""
+    from stacr_amd import kernels
+
+    announce("grad wide edges", rows, d_in, d_out, rank, dtype, transposed, bits)
+    x = make_activation(rows, d_in)
+    x[::8] *= 8.0
+    x[:, 40] *= 40.0
+    x[:, 768:776] *= 10.0
+    x = x.to(dev, DT[dtype])
+    q = make_basis(d_in, rank).to(dev, DT[dtype])
+    g = make_grad(rows, d_out).to(dev, DT[dtype])
+    coeff, idx, data, scale = kernels.save(x, q, mode="global_topk", budget=0.02, chunk_rows=512, bits=bits)
+    with _kernel_names() as names:
+        dw, db = kernels.weight_grad(g, coeff, q, (idx, data, scale), bits, transposed, DT[dtype], DT[dtype])
+    assert "k_tile_wide" in names
+    oidx = idx.cpu().numpy().astype(np.int64)
+    tiles = np.bincount((oidx // d_in // 512) * 1024 + oidx % d_in // 16)
+    assert tiles.max() > 128
+    raw = data.cpu().numpy() if bits else None
+    ovals = (_np(data) if bits == 0 else
+             orc.dequantize(raw.view(np.int8) if bits == 8 else raw, np.float32(scale.item()), bits, oidx.size))
+    odw, odb = orc.weight_grad(_np(g), _np(coeff), _np(q), oidx, ovals, d_in)
+    got = _np(dw).T if transposed else _np(dw)
+    assert rel_l2(got, odw) <= TOL[dtype]
+    assert rel_l2(_np(db), odb) <= TOL[dtype]
+    if dtype == "bf16":
+        assert_rounded_once_bf16(got, odw, what="dW")

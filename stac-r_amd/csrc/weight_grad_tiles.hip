@@ -36,6 +36,8 @@
 //     (the plan then selects no column features: every entry is a light record, and orders a tile's
 //     records for the LDS banks): one workgroup per (32 or 64 output features, part), every entry
 //     summed on the matrix cores in chunks of 32 records (see the kernel).
+//   k_lr_stream, k_lr_finish   in place of k_tile_grad without entries, for wide d_out and many rows:
+//     M = G^T [C | 1] from whole lines of G, then dW = M Q^T.
 #include <type_traits>
 
 #include "internal.h"
@@ -58,6 +60,10 @@ constexpr int kBatch = 8;            // entries per thread whose loads the count
 constexpr int kRounds = 3;           // rounds of kBatch entries a thread the plan keeps in registers between its passes
 constexpr int kMaxRowSplit = 8;     // (no entries) workgroups over the rows of one o-slab, at most
 constexpr int kSplitTargetWgs = 1024;  // rows are split until this many workgroups: two rounds of two a CU
+constexpr int kLrOuts = 128;           // outputs of a k_lr_stream workgroup: whole 256-byte pieces of G's rows
+constexpr int kLrThreads = 512;
+constexpr int kLrTargetWgs = 512;      // rows are split until this many: two a CU, which are all resident
+constexpr int kLrMinWgs = 256;         // fewer leave CUs idle, and k_tile_grad's 16-output slabs fill the chip better
 
 static_assert(kThreads == 2 * kTB, "two G tile rows per lane pair: one 16-byte copy per lane");
 static_assert(kTB == kCensusRows, "a save's entry census gives the first entry of every block");
@@ -1229,6 +1235,158 @@ __global__ __launch_bounds__(256) void k_tile_lr_finish(TileArgs a)
     store_dw_row(a, i, o0, out);
 }
 
+// ------------------------------------------------------------------ the stream without entries
+// M = Gᵀ[C | 1] over a row range, for 128 outputs a workgroup.  Without entries nothing else needs G,
+// so it goes from memory to registers and the LDS is left to the reduction.  HBM bounds it: a wave
+// reads 32 rows by 256 bytes at a time (lane l: rows 8 (l / 16) .. + 7, outputs 8 (l % 16) .. + 7, so
+// 16 lanes read two whole lines of a row; k_tile_grad's 32-byte pieces stop at 3.5 TB/s), the next
+// 32 rows in flight while these are multiplied.  A lane's 8 rows by 8 outputs are transposed by 32
+// v_perm into the A operands of eight products: product m has output 8 r + m in row r.  The waves'
+// tiles are summed in wave order, the row ranges' by the finish.  8192 rows, d_out 5120: 18.0 us,
+// 4.7 TB/s of G (k_tile_grad 23.8 us).
+template <int DT>
+__global__ __launch_bounds__(kLrThreads) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_lr_stream(TileArgs a)
+{
+    constexpr int kWv = kLrThreads / 64;
+    constexpr int kWaveTile = kLrOuts * 16 + kLrOuts / 32 * 16;  // 16 words of padding every 32 outputs: no bank conflicts
+    __shared__ __attribute__((aligned(16))) float s_t[kWv * kWaveTile];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, n = lane & 15, grp = lane >> 4;
+    const int groups = (int)(a.d_out / kLrOuts);
+    const int split = blockIdx.x / groups, group = blockIdx.x % groups;
+    const int bb = (int)((int64_t)split * a.n_blocks / a.row_split);
+    const int nb = (int)((int64_t)(split + 1) * a.n_blocks / a.row_split) - bb;
+    const int steps = nb * (kTB / 32 / kWv);  // this wave's: 32-row pieces wave, wave + 8, .. of the range (even)
+    const int64_t last = a.rows - 1;
+    const uint16_t *g = static_cast<const uint16_t *>(a.g) + (int64_t)group * kLrOuts + 8 * n;
+    const uint16_t *cp = static_cast<const uint16_t *>(a.cp);
+    const int nc = n < a.ncol ? n : a.ncol - 1;
+
+    struct Piece {
+        uint4 g[8], c;
+    };
+    // (pieces past the range repeat its last one: loads without a branch.  Rows past the end repeat the
+    // last row, their operands are zero)
+    auto load = [&](int st, Piece &r) {
+        const int64_t piece = (int64_t)bb * (kTB / 32) + (st < steps ? st : steps - 1) * kWv + wave;
+        const int64_t row = piece * 32 + 8 * grp;
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            r.g[i] = *reinterpret_cast<const uint4 *>(g + (row + i < last ? row + i : last) * a.d_out);
+        r.c = *reinterpret_cast<const uint4 *>(cp + ((piece * 4 + grp) * a.ncol + nc) * 8);
+    };
+    f32x4 acc[8];
+#pragma unroll
+    for (int m = 0; m < 8; ++m) acc[m] = f32x4{0.f, 0.f, 0.f, 0.f};
+    auto multiply = [&](const Piece &r) {
+        const uint4 c = n < a.ncol ? r.c : make_uint4(0u, 0u, 0u, 0u);
+        uint32_t w[8][4];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) w[i][0] = r.g[i].x, w[i][1] = r.g[i].y, w[i][2] = r.g[i].z, w[i][3] = r.g[i].w;
+#pragma unroll
+        for (int m = 0; m < 8; ++m) {
+            const uint32_t sel = m & 1 ? 0x07060302u : 0x05040100u;  // the high or the low halves of two rows' words
+            const uint4 av = make_uint4(__builtin_amdgcn_perm(w[1][m >> 1], w[0][m >> 1], sel),
+                                        __builtin_amdgcn_perm(w[3][m >> 1], w[2][m >> 1], sel),
+                                        __builtin_amdgcn_perm(w[5][m >> 1], w[4][m >> 1], sel),
+                                        __builtin_amdgcn_perm(w[7][m >> 1], w[6][m >> 1], sel));
+            acc[m] = mfma16<DT>(av, c, acc[m]);
+        }
+    };
+    Piece p0, p1;
+    load(0, p0);
+    for (int st = 0; st < steps; st += 2) {
+        load(st + 1, p1);
+        multiply(p0);
+        load(st + 2, p0);
+        multiply(p1);
+    }
+    // tile row 4 grp + q of product m is output 8 (4 grp + q) + m, which lies in the grp-th 32 outputs
+    float *t = s_t + wave * kWaveTile + grp * 16 + n;
+#pragma unroll
+    for (int m = 0; m < 8; ++m)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) t[(8 * (4 * grp + q) + m) * 16] = acc[m][q];
+    __syncthreads();
+    const int e = 4 * tid, o = e >> 4;  // four of output o's 16 columns
+    static_assert(4 * kLrThreads == kLrOuts * 16, "four values a thread");
+    float4 sum = *reinterpret_cast<const float4 *>(s_t + e + (o >> 5) * 16);
+#pragma unroll
+    for (int w = 1; w < kWv; ++w) {
+        const float4 v = *reinterpret_cast<const float4 *>(s_t + w * kWaveTile + e + (o >> 5) * 16);
+        sum.x += v.x, sum.y += v.y, sum.z += v.z, sum.w += v.w;
+    }
+    const int64_t slab = (int64_t)group * (kLrOuts / kOS) + (o >> 4);
+    *reinterpret_cast<float4 *>(a.mpart + (slab * a.row_split + split) * 256 + (e & 255)) = sum;
+}
+
+// k_tile_lr_finish for a Conv1D dW (d_in x d_out): one workgroup per (128 outputs, 128 features), so
+// that 16 lanes write 256 consecutive bytes of a dW row where the 16-output form writes 32.  The same
+// sums in the same order.  1280 x 5120: 16.0 -> 7.9 us.
+template <int DT>
+__global__ __launch_bounds__(kLrThreads) void k_lr_finish(TileArgs a)
+{
+    constexpr int kF = 128;                // features a workgroup
+    constexpr int kMs = kLrOuts + 4;       // M's LDS stride: [column][output]
+    __shared__ __attribute__((aligned(16))) float s_m[16 * kMs];
+    __shared__ float s_q[kF * 16];
+    const int tid = threadIdx.x;
+    const int groups = (int)(a.d_out / kLrOuts);
+    const int64_t group = blockIdx.x % groups, chunk = blockIdx.x / groups, o0 = group * kLrOuts, f0 = chunk * kF;
+    const int nf = a.d_in - f0 < kF ? (int)(a.d_in - f0) : kF;
+    const uint16_t *q = static_cast<const uint16_t *>(a.q) + f0 * a.rank;
+    for (int e = tid; e < nf * a.rank; e += kLrThreads) s_q[e] = g16_to_f<DT>(q[e]);
+    // M: four of an output's columns a thread, the row ranges' tiles in order
+    const int e = 4 * tid, o = e >> 4, j0 = e & 15;
+    const float *mp = a.mpart + (group * (kLrOuts / kOS) + (o >> 4)) * a.row_split * 256 + (e & 255);
+    float4 v[kMaxRowSplit];
+#pragma unroll
+    for (int r = 0; r < kMaxRowSplit; ++r)
+        v[r] = *reinterpret_cast<const float4 *>(mp + (r < a.row_split ? r : a.row_split - 1) * 256);
+    float4 m = v[0];
+#pragma unroll
+    for (int r = 1; r < kMaxRowSplit; ++r)
+        if (r < a.row_split) m.x += v[r].x, m.y += v[r].y, m.z += v[r].z, m.w += v[r].w;
+    s_m[(j0 + 0) * kMs + o] = m.x;
+    s_m[(j0 + 1) * kMs + o] = m.y;
+    s_m[(j0 + 2) * kMs + o] = m.z;
+    s_m[(j0 + 3) * kMs + o] = m.w;
+    __syncthreads();
+    if (chunk == 0 && a.dbias && tid < kLrOuts) store_any(a.dbias, a.db_dt, o0 + tid, s_m[a.bias_col * kMs + tid]);
+    // outputs 8 og .. + 7 of features fr, fr + 32, fr + 64 and fr + 96 (past the last: its row again, not stored)
+    const int og = tid & 15, fr = tid >> 4;
+    float out[4][8] = {};
+    for (int j = 0; j < a.rank; ++j) {
+        float mv[8];
+        *reinterpret_cast<float4 *>(mv) = *reinterpret_cast<const float4 *>(s_m + j * kMs + 8 * og);
+        *reinterpret_cast<float4 *>(mv + 4) = *reinterpret_cast<const float4 *>(s_m + j * kMs + 8 * og + 4);
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+            const int f = fr + 32 * p < nf ? fr + 32 * p : nf - 1;
+            const float qj = s_q[f * a.rank + j];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) out[p][k] = fmaf(mv[k], qj, out[p][k]);
+        }
+    }
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+        if (fr + 32 * p >= nf) break;
+        const int64_t at = (f0 + fr + 32 * p) * a.d_out + o0 + 8 * og;
+        if (a.dw_dt == STACR_DTYPE_F32) {
+            float4 *dst = reinterpret_cast<float4 *>(static_cast<float *>(a.dw) + at);
+            dst[0] = make_float4(out[p][0], out[p][1], out[p][2], out[p][3]);
+            dst[1] = make_float4(out[p][4], out[p][5], out[p][6], out[p][7]);
+        } else {
+            const bool bf = a.dw_dt == STACR_DTYPE_BF16;
+            uint32_t wv[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                wv[k] = bf ? (f_to_bf16_bits(out[p][2 * k]) | (f_to_bf16_bits(out[p][2 * k + 1]) << 16))
+                           : (f_to_f16_bits(out[p][2 * k]) | (f_to_f16_bits(out[p][2 * k + 1]) << 16));
+            *reinterpret_cast<uint4 *>(static_cast<uint16_t *>(a.dw) + at) = make_uint4(wv[0], wv[1], wv[2], wv[3]);
+        }
+    }
+}
+
 // ------------------------------------------------------------------ the wide streaming kernel
 // One workgroup per (16 NJ outputs, part), every entry of the part a light record (the plan selects
 // no column features).  Wave w owns the part's 16-feature tiles w, w + 16, w + 32 and w + 48, whose
@@ -1542,7 +1700,8 @@ struct TileGeom {
     int gb;  // bytes of a G / C element
     bool sparse, bt8;
     int nj;     // 16-output tiles of a k_tile_wide workgroup (every entry a light record); 0: k_tile_grad
-    int row_split;  // (no entries) k_tile_grad workgroups over the rows of one o-slab
+    int row_split;  // (no entries) workgroups over the rows of one o-slab
+    bool lr;        // (no entries) k_lr_stream takes the rows of 128 outputs a workgroup
 };
 
 // Workgroups of 32 outputs that make the wide kernel the better choice: one per CU.  Below that the
@@ -1585,6 +1744,13 @@ bool tile_geom(const StacrGradArgs &a, TileGeom *g)
     while (!g->sparse && g->row_split < kMaxRowSplit && (a.d_out / kOS) * g->row_split < kSplitTargetWgs &&
            g->n_blocks >= 4 * g->row_split)
         g->row_split *= 2;
+    // k_lr_stream reads G in whole lines, where its 128-output workgroups still fill the chip
+    int lr_split = 1;
+    while (!g->sparse && lr_split < kMaxRowSplit && a.d_out / kLrOuts * lr_split < kLrTargetWgs &&
+           g->n_blocks >= 4 * lr_split)
+        lr_split *= 2;
+    g->lr = lr_split > 1 && a.rank > 0 && a.d_out % kLrOuts == 0 && a.d_out / kLrOuts * lr_split >= kLrMinWgs;
+    if (g->lr) g->row_split = lr_split;
     return true;
 }
 
@@ -1633,6 +1799,27 @@ int launch_tile_wide(const TileArgs &t, const TileGeom &g, hipStream_t s)
     return stacr_hip_check(hipGetLastError(), "weight_grad wide matrix-core kernel");
 }
 
+template <int DT>
+int launch_lr_finish(const TileArgs &t, hipStream_t s)
+{
+    const unsigned grid = (unsigned)((t.d_out / kOS) * ((t.d_in + 255) / 256));
+    stacr_launch("k_tile_lr_finish", s, [&] { k_tile_lr_finish<DT><<<grid, 256, 0, s>>>(t); });
+    return stacr_hip_check(hipGetLastError(), "weight_grad row-split finish");
+}
+
+// The stream without entries, and (Conv1D) its finish.
+template <int DT>
+int launch_lr(const TileArgs &t, hipStream_t s)
+{
+    const unsigned groups = (unsigned)(t.d_out / kLrOuts);
+    stacr_launch("k_lr_stream", s, [&] { k_lr_stream<DT><<<groups * t.row_split, kLrThreads, 0, s>>>(t); });
+    const int rc = stacr_hip_check(hipGetLastError(), "weight_grad low-rank stream");
+    if (rc || !t.transposed) return rc;
+    const unsigned grid = groups * (unsigned)((t.d_in + 127) / 128);
+    stacr_launch("k_lr_finish", s, [&] { k_lr_finish<DT><<<grid, kLrThreads, 0, s>>>(t); });
+    return stacr_hip_check(hipGetLastError(), "weight_grad low-rank finish");
+}
+
 }  // namespace
 
 bool stacr_tiles_eligible(const StacrGradArgs &a)
@@ -1662,6 +1849,7 @@ size_t stacr_tiles_ws_bound(int64_t rows, int64_t d_out, int64_t d_in, int64_t n
     g.bt8 = false;  // the wider column-operand form
     g.nj = 0;        // (with column operands: the larger layout)
     g.row_split = nnz > 0 ? 1 : kMaxRowSplit;  // (the most M tiles)
+    g.lr = false;
     size_t off[TW_N];
     return tile_layout(nnz, d_in, d_out, g, off);
 }
@@ -1738,15 +1926,17 @@ int stacr_tiles_launch(const StacrGradArgs &a)
     if (g.nj)
         return a.dtype == STACR_DTYPE_BF16 ? launch_tile_wide<STACR_DTYPE_BF16>(t, g, s)
                                            : launch_tile_wide<STACR_DTYPE_F16>(t, g, s);
+    if (g.lr) {
+        rc = a.dtype == STACR_DTYPE_BF16 ? launch_lr<STACR_DTYPE_BF16>(t, s) : launch_lr<STACR_DTYPE_F16>(t, s);
+        if (rc || a.transposed) return rc;
+        return a.dtype == STACR_DTYPE_BF16 ? launch_lr_finish<STACR_DTYPE_BF16>(t, s)
+                                           : launch_lr_finish<STACR_DTYPE_F16>(t, s);
+    }
     const int nwg = (int)(a.d_out / kOS) * g.n_parts * g.row_split;
     if (a.dtype == STACR_DTYPE_F32) return launch_tile_grad<STACR_DTYPE_F32, true, true>(t, nwg, s);
     rc = a.dtype == STACR_DTYPE_BF16 ? launch_tile_grad_dt<STACR_DTYPE_BF16>(t, g, nwg, s)
                                      : launch_tile_grad_dt<STACR_DTYPE_F16>(t, g, nwg, s);
     if (rc || g.row_split == 1) return rc;
-    const unsigned fgrid = (unsigned)((a.d_out / kOS) * ((a.d_in + 255) / 256));
-    if (a.dtype == STACR_DTYPE_BF16)
-        stacr_launch("k_tile_lr_finish", s, [&] { k_tile_lr_finish<STACR_DTYPE_BF16><<<fgrid, 256, 0, s>>>(t); });
-    else
-        stacr_launch("k_tile_lr_finish", s, [&] { k_tile_lr_finish<STACR_DTYPE_F16><<<fgrid, 256, 0, s>>>(t); });
-    return stacr_hip_check(hipGetLastError(), "weight_grad row-split finish");
+    return a.dtype == STACR_DTYPE_BF16 ? launch_lr_finish<STACR_DTYPE_BF16>(t, s)
+                                       : launch_lr_finish<STACR_DTYPE_F16>(t, s);
 }

@@ -346,6 +346,12 @@ GRAD_CASES = [
     # (3 + 3, the last one partial) over 25 slabs (no XCD remap), 2100 rows 5 blocks (2 + 3)
     ("turbo_split_ragged_bf16_conv1d", 2900, 300, 400, 5, "bf16", True, 8, "chunk_topk", 0.0, False),
     ("turbo_split_ragged_f16", 2100, 130, 160, 7, "f16", False, 8, "chunk_topk", 0.0, False),
+    # the 128-output stream: 7700 rows are 16 blocks (eight ranges, the last with 20 rows in its last
+    # block) over 32 groups and feature chunks of 128 + 1; 4100 rows 9 blocks (2 + 2 + 2 + 3), rank 15
+    # and the bias column filling the operand, in either layout
+    ("turbo_stream_bf16_conv1d", 7700, 129, 4096, 5, "bf16", True, 8, "chunk_topk", 0.0, False),
+    ("turbo_stream_f16_conv1d_rank15", 4100, 300, 8192, 15, "f16", True, 8, "chunk_topk", 0.0, False),
+    ("turbo_stream_f16_rank15", 4100, 200, 8192, 15, "f16", False, 8, "chunk_topk", 0.0, False),
     ("cfg3_cfc_bf16_conv1d", 2048, 1024, 4096, 8, "bf16", True, 8, "global_topk", 0.005, False),
     ("fp32_bits0", 512, 256, 384, 4, "f32", False, 0, "chunk_topk", 0.02, False),
     ("fp32_bits4_conv1d_rank5", 1100, 300, 160, 5, "f32", True, 4, "chunk_topk", 0.02, True),

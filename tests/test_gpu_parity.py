@@ -400,6 +400,31 @@ def test_weight_grad_matches_oracle(dev, case):
         assert_rounded_once_bf16(_np(db), odb, what="dbias")
 
 
+@pytest.mark.parametrize("index_dtype", [torch.int32, torch.int64])
+@pytest.mark.parametrize("spans", [((700, 1),), ((600, 40), (1500, 25)), ((0, 64), (511, 65), (2047, 1)),
+                                   ((512, 1), (1024, 4160), (2040, 5))], ids=str)
+def test_wide_block_starts_without_census(dev, spans, index_dtype):
+    """Blocks without entries, entries on a block's first and last row, and counts at the edges of the
+    64-probe search (1, 64, 65, above 65 * 64): the starts are found from the entries alone."""
+    from stacr_amd import kernels
+
+    announce("wide block starts", spans, index_dtype)
+    rows, d_in, d_out, rank = 2048, 2048, 8192, 4
+    rng = np.random.default_rng(5)
+    # n entries at random features of the rows from r on, at most 2048 a row
+    idx = np.unique(np.concatenate([r * d_in + rng.choice(d_in * (n // d_in + 1), n, replace=False) for r, n in spans]))
+    codes = rng.integers(-127, 128, idx.size).astype(np.int8)
+    scale = np.float32(0.01)
+    coeff = torch.randn(rows, rank).to(dev, torch.bfloat16)
+    q = make_basis(d_in, rank).to(dev, torch.bfloat16)
+    g = make_grad(rows, d_out).to(dev, torch.bfloat16)
+    residual = (torch.from_numpy(idx).to(dev, index_dtype), torch.from_numpy(codes).to(dev),
+                torch.tensor(scale, device=dev))
+    dw, _ = kernels.weight_grad(g, coeff, q, residual, 8, False, torch.bfloat16, torch.bfloat16)
+    odw, _ = orc.weight_grad(_np(g), _np(coeff), _np(q), idx, orc.dequantize(codes, scale, 8, idx.size), d_in)
+    assert_rounded_once_bf16(_np(dw), odw, what="dW")
+
+
 @pytest.mark.parametrize("dtype,budget,rank", [("bf16", 0.03, 8), ("f32", 0.03, 8), ("f16", 0.004, 16),
                                                ("bf16", 0.2, 4)])
 def test_weight_grad_heavy_features_and_many_rounds(dev, dtype, budget, rank):

@@ -63,7 +63,11 @@ constexpr int kSplitTargetWgs = 1024;  // rows are split until this many workgro
 constexpr int kLrOuts = 128;           // outputs of a k_lr_stream workgroup: whole 256-byte pieces of G's rows
 constexpr int kLrThreads = 512;
 constexpr int kLrTargetWgs = 512;      // rows are split until this many: two a CU, which are all resident
-constexpr int kLrMinWgs = 256;         // fewer leave CUs idle, and k_tile_grad's 16-output slabs fill the chip better
+// Fewer leave so many CUs idle that k_tile_grad's 16-output slabs are better.  d_in 1024, Conv1D dW, k_tile_grad
+// (and its finish) against k_lr_stream and k_lr_finish, plan included: 16 workgroups (2048 rows, d_out 1024) 12.5
+// and 13.6 us, 32 (4096 x 1024) 12.9 and 13.7, 48 (2048 x 3072) 16.9 and 14.1, 64 (4096 x 2048) 16.1 and 14.0,
+// 128 (8192 x 2048) 21.8 and 15.2, 256 (8192 x 4096) 32.9 and 22.1; nn.Linear dW at 48 17.3 and 16.7.
+constexpr int kLrMinWgs = 48;
 
 static_assert(kThreads == 2 * kTB, "two G tile rows per lane pair: one 16-byte copy per lane");
 static_assert(kTB == kCensusRows, "a save's entry census gives the first entry of every block");
@@ -259,8 +263,8 @@ __global__ __launch_bounds__(kThreads) void k_tile_count(TileArgs a)
 
 // The block starts alone, for k_tile_wide's plan, which selects no columns and so needs no counts: one
 // wave per start, 64 probes of the ascending entries at a time.  Each round is one load latency, and
-// ceil(log65 nnz) rounds are all there is.  32768 rows of 8192
-// features (1.3 M entries): 5.5 us, against 32 for the sixteen counting workgroups above; of 2048: 4.9 against 10.
+// ceil(log65 nnz) rounds are all there is.  32768 rows of 8192 features (1.3 M entries): 5.5 us, against
+// 32 for the sixteen counting workgroups above; of 2048 features 4.9 against 10.
 __global__ __launch_bounds__(64) void k_block_starts(TileArgs a)
 {
     const int b = blockIdx.x, lane = threadIdx.x;

@@ -351,6 +351,7 @@ GRAD_CASES = [
     # and the bias column filling the operand, in either layout
     ("turbo_stream_bf16_conv1d", 7700, 129, 4096, 5, "bf16", True, 8, "chunk_topk", 0.0, False),
     ("turbo_stream_f16_conv1d_rank15", 4100, 300, 8192, 15, "f16", True, 8, "chunk_topk", 0.0, False),
+    ("turbo_stream_two_ranges_bf16_conv1d", 2049, 255, 3072, 8, "bf16", True, 8, "chunk_topk", 0.0, False),
     ("turbo_stream_f16_rank15", 4100, 200, 8192, 15, "f16", False, 8, "chunk_topk", 0.0, False),
     ("cfg3_cfc_bf16_conv1d", 2048, 1024, 4096, 8, "bf16", True, 8, "global_topk", 0.005, False),
     ("fp32_bits0", 512, 256, 384, 4, "f32", False, 0, "chunk_topk", 0.02, False),

@@ -979,3 +979,67 @@ def test_weight_grad_wide_tiles_at_their_edges(dev, rows, d_in, d_out, rank, dty
     assert rel_l2(_np(db), odb) <= TOL[dtype]
     if dtype == "bf16":
         assert_rounded_once_bf16(got, odw, what="dW")
+
+
+def _check_save_against_oracle(xd, qd, mode, budget, chunk, bits, coeff=None):
+    """One bf16 save, its entries bit for bit against the oracle on the kernel's own coefficients; the
+    names of the kernels that ran."""
+    from stacr_amd import kernels
+
+    with _kernel_names() as names:
+        c, idx, data, scale = kernels.save(xd, qd, mode=mode, budget=budget, chunk_rows=chunk, bits=bits, coeff=coeff)
+    _, oidx, odata, oscale = orc.save(_np(xd), _np(qd), "bf16", mode, budget, chunk, bits, coeff=_np(c))
+    assert np.array_equal(idx.cpu().numpy().astype(np.int64), oidx)
+    if bits == 0:
+        assert np.array_equal(_np(data), odata)
+    else:
+        assert np.array_equal(data.cpu().numpy().view(np.int8 if bits == 8 else np.uint8), odata)
+        assert np.float32(scale.item()) == oscale
+    return names
+
+
+def _list_passes_us(xd, qd, mode="global_topk", budget=0.005):
+    """Time of a save's two list passes, the smallest of several."""
+    from stacr_amd import _lib, kernels
+
+    best = float("inf")
+    for _ in range(5):
+        with _lib.KernelTimer(max_launches=256) as timer:
+            for _ in range(4):
+                kernels.save(xd, qd, mode=mode, budget=budget, chunk_rows=512, bits=8)
+            torch.cuda.synchronize()
+        best = min(best, sum(timer.results[k][0] for k in ("k_refine_lists", "k_emit_lists")) / 4 * 1e3)
+    return best
+
+
+@pytest.mark.parametrize("rows,d,rank,mode,live", [
+    (1024, 1024, 8, "global_topk", 24),   # the last 8 of every 32 rows zero: part of a list, and whole lists
+    (2048, 1024, 8, "chunk_topk", 8),
+    (1024, 4096, 8, "global_topk", 24),
+    (1100, 2048, 16, "chunk_topk", 20),
+    (512, 1024, 8, "global_topk", 0),     # zeros only, but for one row: level-0 bin 0 holds the threshold
+    (512, 2048, 16, "global_topk", 0),
+])
+def test_save_with_rows_of_zeros_matches_oracle(dev, rows, d, rank, mode, live):
+    """Rows of zeros (padding) put whole rows of keys into the lowest bin."""
+    announce("save rows of zeros", rows, d, rank, mode, live)
+    x = make_activation(rows, d)
+    x[torch.arange(rows) % 32 >= live] = 0.0
+    if live == 0:
+        x[7] = make_activation(1, d)[0]
+        x[7, 3:] = 0.0
+    xd, qd = x.to(dev, torch.bfloat16), make_basis(d, rank).to(dev, torch.bfloat16)
+    assert "k_emit_lists" in _check_save_against_oracle(xd, qd, mode, 0.005, 512, 8)
+
+
+@pytest.mark.parametrize("rows,d,rank", [(512, 768, 8), (8192, 1024, 8), (8192, 4096, 8), (8192, 2048, 16)])
+def test_rows_of_zeros_leave_the_lists_usable(dev, rows, d, rank):
+    """The later passes read the candidate lists of padded batches too.  (A list that is not usable is
+    recomputed from X: these passes then took 5 to 15 times as long.)"""
+    announce("rows of zeros, list passes", rows, d, rank)
+    x = make_activation(rows, d).to(dev, torch.bfloat16)
+    qd = make_basis(d, rank).to(dev, torch.bfloat16)
+    whole = _list_passes_us(x, qd)
+    x.view(8, rows // 8, d)[:, rows * 3 // 32:] = 0.0  # eight sequences, the last quarter of each padding
+    padded = _list_passes_us(x, qd)
+    assert padded <= 2.5 * whole, f"{padded:.1f} us with a quarter of the rows zero, {whole:.1f} us without"

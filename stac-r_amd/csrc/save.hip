@@ -27,8 +27,9 @@ constexpr int kEmitStage = 1024;   // survivors a batched emission workgroup sta
 constexpr int kCandCap = 2048;               // candidates a workgroup keeps
 constexpr int kCandPer = kCandCap / kBlock;  // candidates a thread reads (consecutive)
 static_assert(kCandPer == 8, "one 16-byte vector of bf16 candidate values per thread");
+constexpr int kCandBytes = 6;                // a candidate: its flat index and its bf16 residual
 
-constexpr int kListCap = 4096;  // candidates a projection workgroup's list holds
+constexpr int kListMax = 4096;  // candidates a wide projection workgroup's list holds, at most (the plan's list_cap)
 
 struct CandMeta {
     uint32_t cut;    // level-0 bin of the workgroup's cut
@@ -1776,7 +1777,7 @@ __global__ __launch_bounds__(kBlock) void k_proj_cand(SaveGeom g, FastGeom fg, c
                                                       const float *__restrict__ qp, uint16_t *__restrict__ coeff,
                                                       uint32_t *__restrict__ hist, uint32_t *__restrict__ maxkey,
                                                       const uint16_t *__restrict__ coeff_in,
-                                                      uint32_t *__restrict__ coarse, uint32_t quota,
+                                                      uint32_t *__restrict__ coarse, uint32_t quota, uint32_t cap,
                                                       uint32_t *__restrict__ cand_idx, uint16_t *__restrict__ cand_val,
                                                       CandMeta *__restrict__ meta)
 {
@@ -1874,7 +1875,7 @@ __global__ __launch_bounds__(kBlock) void k_proj_cand(SaveGeom g, FastGeom fg, c
     if (lane == 0) s_wmax[wave] = kmax;
     __syncthreads();
     if (wave == 0) {
-        const uint32_t cut = list_cut(s_hist, quota, kListCap);
+        const uint32_t cut = list_cut(s_hist, quota, cap);
         if (lane == 0) s_cut = cut;
     }
     __syncthreads();
@@ -1902,8 +1903,8 @@ __global__ __launch_bounds__(kBlock) void k_proj_cand(SaveGeom g, FastGeom fg, c
         for (int i = 0; i < NB; ++i) s_wt[wave * NB + i] = incl[i];
     __syncthreads();
     uint32_t before_iter = 0u;
-    uint32_t *ci = cand_idx + (int64_t)blockIdx.x * kListCap;
-    uint16_t *cv = cand_val + (int64_t)blockIdx.x * kListCap;
+    uint32_t *ci = cand_idx + (int64_t)blockIdx.x * cap;
+    uint16_t *cv = cand_val + (int64_t)blockIdx.x * cap;
 #pragma unroll
     for (int i = 0; i < NB; ++i) {
         uint32_t waves_before = 0u, iter_total = 0u;
@@ -1922,7 +1923,7 @@ __global__ __launch_bounds__(kBlock) void k_proj_cand(SaveGeom g, FastGeom fg, c
                 uint32_t word = wd[0];
 #pragma unroll
                 for (int k = 1; k < 4; ++k) word = (e >> 1) == k ? wd[k] : word;
-                if (pos < (uint32_t)kListCap) {
+                if (pos < cap) {
                     ci[pos] = (uint32_t)(ld.rows[i] * g.d + col + e);
                     cv[pos] = (uint16_t)((word >> (16 * (e & 1))) & 0xffffu);
                 }
@@ -1965,7 +1966,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(R == 8 && MV
                                                     uint32_t *__restrict__ hist, uint32_t *__restrict__ maxkey,
                                                     const uint16_t *__restrict__ coeff_in,
                                                     uint32_t *__restrict__ coarse, float *__restrict__ y_out, int y_cols,
-                                                    float *__restrict__ epart, uint32_t quota,
+                                                    float *__restrict__ epart, uint32_t quota, uint32_t cap,
                                                     uint32_t *__restrict__ cand_idx, uint16_t *__restrict__ cand_val,
                                                     CandMeta *__restrict__ meta)
 {
@@ -2197,7 +2198,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(R == 8 && MV
     if (lane == 0) s_wmax[wave] = kmax;
     __syncthreads();
     if (wave == 0) {
-        const uint32_t cut = list_cut(s_hist, quota, kListCap);
+        const uint32_t cut = list_cut(s_hist, quota, cap);
         if (lane == 0) s_cut = cut;
     }
     __syncthreads();
@@ -2255,8 +2256,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(R == 8 && MV
         if (lane == 0) meta[blockIdx.x] = CandMeta{cut, run};
     }
     __syncthreads();
-    uint32_t *ci = cand_idx + (int64_t)blockIdx.x * kListCap;
-    uint16_t *cv = cand_val + (int64_t)blockIdx.x * kListCap;
+    uint32_t *ci = cand_idx + (int64_t)blockIdx.x * cap;
+    uint16_t *cv = cand_val + (int64_t)blockIdx.x * cap;
 #pragma unroll
     for (int i = 0; i < NB; ++i)
 #pragma unroll
@@ -2268,7 +2269,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(R == 8 && MV
                 uint32_t word = wd[0];
 #pragma unroll
                 for (int k = 1; k < 4; ++k) word = (e >> 1) == k ? wd[k] : word;
-                if (pos < (uint32_t)kListCap) {
+                if (pos < cap) {
                     ci[pos] = (uint32_t)((row0 + i) * g.d) + col[m] + (uint32_t)e;
                     cv[pos] = (uint16_t)((word >> (16 * (e & 1))) & 0xffffu);
                 }
@@ -2312,12 +2313,12 @@ constexpr int kFewLists = 255;         // up to this many lists, a workgroup eac
 constexpr int kListRound = 64 * 8;     // candidates a wave reads at once
 
 // A lane's 8 consecutive candidate values of round k (zeros past the list).
-__device__ __forceinline__ CandVals list_vals(const uint16_t *__restrict__ cand_val, int64_t list, int k, uint32_t n)
+__device__ __forceinline__ CandVals list_vals(const uint16_t *__restrict__ cand_val, int64_t list, uint32_t cap, int k, uint32_t n)
 {
     CandVals r;
     uint4 v = make_uint4(0u, 0u, 0u, 0u);
     const uint32_t e = (uint32_t)(k * kListRound + 8 * (threadIdx.x & 63));
-    if (e < n) v = *reinterpret_cast<const uint4 *>(cand_val + list * kListCap + e);
+    if (e < n) v = *reinterpret_cast<const uint4 *>(cand_val + list * cap + e);
     r.w[0] = v.x; r.w[1] = v.y; r.w[2] = v.z; r.w[3] = v.w;
     return r;
 }
@@ -2357,7 +2358,7 @@ __global__ __launch_bounds__(64 * LW) void k_refine_lists(SaveGeom g, int R, int
                                                                   uint32_t *__restrict__ hist, SelState *__restrict__ state,
                                                                   uint32_t k_full, uint32_t k_last,
                                                                   uint32_t *__restrict__ maxkey, uint32_t *__restrict__ fold,
-                                                                  const uint32_t *__restrict__ coarse,
+                                                                  const uint32_t *__restrict__ coarse, uint32_t cap,
                                                                   const uint16_t *__restrict__ cand_val,
                                                                   const CandMeta *__restrict__ meta)
 {
@@ -2375,9 +2376,9 @@ __global__ __launch_bounds__(64 * LW) void k_refine_lists(SaveGeom g, int R, int
 #pragma unroll
     for (int h = 0; h < HC; ++h) cv[h] = coarse[(chunk * HC + h) * kCoarse + lane];
     const CandMeta mine = meta[has_rows ? list : 0];
-    const uint32_t n = has_rows ? min(mine.count, (uint32_t)kListCap) : 0u;
+    const uint32_t n = has_rows ? min(mine.count, cap) : 0u;
     // the first two rounds go out before the selection's words
-    CandVals v0 = list_vals(cand_val, list, 0, n), v1 = list_vals(cand_val, list, 1, n);
+    CandVals v0 = list_vals(cand_val, list, cap, 0, n), v1 = list_vals(cand_val, list, cap, 1, n);
     if (lane < 16) s_cnt[wave][lane] = 0u;
     const SelState sel = select_level0<HC>(cv, hist + chunk * 3 * HC * kBins, sp);
     if (in && list == chunk * g.wgs_per_chunk && lane == 0) state[chunk * 3 + 0] = sel;
@@ -2388,7 +2389,7 @@ __global__ __launch_bounds__(64 * LW) void k_refine_lists(SaveGeom g, int R, int
         maxkey[0] = m;
     }
     const uint32_t prefix = sel.prefix;  // B0
-    const bool usable = !has_rows || (mine.count <= (uint32_t)kListCap && mine.cut <= prefix);  // (uniform in the wave)
+    const bool usable = !has_rows || (mine.count <= cap && mine.cut <= prefix);  // (uniform in the wave)
     if (lane == 0) s_redo[wave] = usable ? 0u : prefix + 1u;
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the counters are clear before any lane adds
     uint32_t above = 0u;
@@ -2400,7 +2401,7 @@ __global__ __launch_bounds__(64 * LW) void k_refine_lists(SaveGeom g, int R, int
         for (int k = 0; k * kListRound < (int)n; ++k) {
             const CandVals v = v0;
             v0 = v1;
-            v1 = list_vals(cand_val, list, k + 2, n);
+            v1 = list_vals(cand_val, list, cap, k + 2, n);
 #pragma unroll
             for (int j = 0; j < 8; ++j)
                 if ((uint32_t)(k * kListRound + 8 * lane + j) < n) count(bf16_key(v.bits(j)), prefix, wave);
@@ -2447,8 +2448,9 @@ __global__ __launch_bounds__(64 * LW) void k_emit_lists(
     SaveGeom g, int R, int64_t n_lists, const uint16_t *__restrict__ x, const float *__restrict__ qp,
     const uint16_t *__restrict__ coeff, SelState *__restrict__ state, uint32_t chunk_k,
     const uint32_t *__restrict__ maxkey, OutSpec o, float *scale_out, int to_list, const uint32_t *__restrict__ hist,
-    const uint32_t *__restrict__ fold, const uint32_t *__restrict__ cand_idx, const uint16_t *__restrict__ cand_val,
-    const CandMeta *__restrict__ meta, uint32_t *__restrict__ census, uint32_t n_entries)
+    const uint32_t *__restrict__ fold, uint32_t cap, const uint32_t *__restrict__ cand_idx,
+    const uint16_t *__restrict__ cand_val, const CandMeta *__restrict__ meta, uint32_t *__restrict__ census,
+    uint32_t n_entries)
 {
     constexpr int DT = STACR_DTYPE_BF16;
     __shared__ uint32_t s_feat[kBins];
@@ -2468,18 +2470,18 @@ __global__ __launch_bounds__(64 * LW) void k_emit_lists(
         for (int c = 0; c < HC; ++c) hw[c] = h1[c * kBins];
     }
     const CandMeta mine = meta[live ? list : 0];
-    const uint32_t n = min(mine.count, (uint32_t)kListCap);
+    const uint32_t n = min(mine.count, cap);
     struct Round {
         CandVals v;
         uint32_t flat[8];
     };
     auto load_round = [&](int k) {
         Round r;
-        r.v = list_vals(cand_val, list, k, n);
+        r.v = list_vals(cand_val, list, cap, k, n);
         const uint32_t e = (uint32_t)(k * kListRound + 8 * lane);
         uint4 f0 = make_uint4(0u, 0u, 0u, 0u), f1 = f0;
-        if (e < n) f0 = *reinterpret_cast<const uint4 *>(cand_idx + list * kListCap + e);
-        if (e + 4 < n) f1 = *reinterpret_cast<const uint4 *>(cand_idx + list * kListCap + e + 4);
+        if (e < n) f0 = *reinterpret_cast<const uint4 *>(cand_idx + list * cap + e);
+        if (e + 4 < n) f1 = *reinterpret_cast<const uint4 *>(cand_idx + list * cap + e + 4);
         r.flat[0] = f0.x; r.flat[1] = f0.y; r.flat[2] = f0.z; r.flat[3] = f0.w;
         r.flat[4] = f1.x; r.flat[5] = f1.y; r.flat[6] = f1.z; r.flat[7] = f1.w;
         return r;
@@ -2519,7 +2521,7 @@ __global__ __launch_bounds__(64 * LW) void k_emit_lists(
             atomicAdd(&s_feat[f & (kBins - 1)], f >= (uint32_t)kBins ? 0x10000u : 1u);
         }
     };
-    const bool usable = !live || (mine.count <= (uint32_t)kListCap && mine.cut <= (T >> kDigitShift[0]));  // (uniform in the wave)
+    const bool usable = !live || (mine.count <= cap && mine.cut <= (T >> kDigitShift[0]));  // (uniform in the wave)
     if (lane == 0) s_redo[wave] = usable ? 0u : 1u;
     if (live) {
         WgOffset wo;
@@ -2983,6 +2985,7 @@ struct Plan {
     // k_refine_cand, k_emit_cand) with the workgroups' quota
     bool cand;
     uint32_t quota;
+    uint32_t list_cap;  // candidates a list holds (a multiple of 8)
     // bf16 on the batched passes over a stored residual (wide rows, or a quota past the list): the
     // level-1 pass writes the candidate lists (bin B0 and above) and k_emit_cand reads them
     bool cand_rin;
@@ -3090,9 +3093,12 @@ Plan make_plan_wide(const StacrSaveArgs &a)
 }
 
 // The candidate passes take bf16 saves on the batched path and wide rows when a workgroup's
-// quota, four times its mean share of its chunk's k plus 64, is at most 1024 (wide rows: six times, 2048:
-// half the list, as the cut's bin comes in whole): a workgroup then needs more than that many times
-// its share above the chunk's level-0 bin before its list is recomputed.
+// quota, four times its mean share of its chunk's k plus 64, is at most 1024 (wide rows: six times, 2048).
+// A list holds four quotas, at most 2048 candidates (wide rows: 4096) and no more than the workgroup has: at
+// least two, as the cut's bin comes in whole.  Wide rows keep the stored residual where two quotas would take
+// more scratch than it and its own lists do.  (Scratch of a save at 0.005, with lists of 4096 for all and now:
+// 32768 x 768 rank 16 202 and 38 MB, 32768 x 1024 rank 16 202 and 44, 32768 x 768 rank 8 51 and 16, 8192 x 1024
+// rank 8 in chunks of 511 rows 218 and 22; 32768 x 8192 rank 16 204 and 204.)
 Plan make_plan_base(const StacrSaveArgs &a)
 {
     Plan p = make_plan_wide(a);
@@ -3106,7 +3112,14 @@ Plan make_plan_base(const StacrSaveArgs &a)
     double quota = 4.0 * dens * wg_elems + 64.0;
     // (a wide workgroup has few rows, whose shares differ more: half as much again)
     if (p.wide) quota *= 1.5;
-    if (quota > (p.wide ? kListCap : kCandCap) / 2) return p;
+    if (quota > (p.wide ? kListMax : kCandCap) / 2) return p;
+    double cap = hmin<double>(4.0 * quota, p.wide ? kListMax : kCandCap);
+    if (p.wide) {  // the stored residual and the lists of the level-1 pass, a workgroup
+        const double stored = (double)a.rows * (double)a.feats * 2.0 + (double)p.n_wgs * kCandCap * kCandBytes;
+        cap = hmin<double>(cap, stored / ((double)p.n_wgs_w * kCandBytes));
+        if (cap < 2.0 * quota) return p;
+    }
+    p.list_cap = ((uint32_t)hmin<double>(cap, wg_elems) + 7u) & ~7u;
     p.cand = true;
     p.cand_rin = false;
     p.quota = (uint32_t)quota;
@@ -3169,7 +3182,7 @@ size_t layout(const StacrSaveArgs &a, const Plan &p, size_t *off)
     const bool rstore = p.fast && a.dtype != STACR_DTYPE_F32 && a.k_total > 0 && !p.cand;  // (wide rows: p.fast)
     take(WS_R, rstore ? (size_t)a.rows * a.feats * 2 : 0);  // the stored residual (16-bit types)
     const bool lists = p.cand || p.cand_rin;
-    const size_t nc = lists ? (size_t)p.n_wgs * (p.cand ? kListCap : kCandCap) : 0;  // the candidate lists
+    const size_t nc = lists ? (size_t)p.n_wgs * (p.cand ? p.list_cap : kCandCap) : 0;  // the candidate lists
     take(WS_CIDX, nc * sizeof(uint32_t));
     take(WS_CVAL, nc * sizeof(uint16_t));
     take(WS_CMETA, lists ? (size_t)p.n_wgs * sizeof(CandMeta) : 0);
@@ -3230,7 +3243,7 @@ int launch_wide_cand(const StacrSaveArgs &a, const Plan &p, const uint16_t *x, c
         done = true;
         stacr_launch("k_proj_cand_w", s, [&] {
             k_proj_cand_w<R, MV, NT><<<n, NT, 0, s>>>(p.gw, x, qp, coeff, hist, maxkey, coeff_in, coarse, y_out, p.yc,
-                                                      a.energy_part, p.quota, cidx, cval, cmeta);
+                                                      a.energy_part, p.quota, p.list_cap, cidx, cval, cmeta);
         });
     };
     using I1 = std::integral_constant<int, 1>;
@@ -3329,7 +3342,7 @@ int launch_typed(const StacrSaveArgs &a, const Plan &p, char *ws, const size_t *
                 }
             } else if (fast && cand) {
                 if constexpr (kCandOk)
-                    stacr_launch("k_proj_cand", s, [&] { k_proj_cand<R><<<nwg, kBlock, 0, s>>>(p.g, fg, x, qp, coeff_out, hist, maxkey, coeff_in, coarse, p.quota, cidx, cval, cmeta); });
+                    stacr_launch("k_proj_cand", s, [&] { k_proj_cand<R><<<nwg, kBlock, 0, s>>>(p.g, fg, x, qp, coeff_out, hist, maxkey, coeff_in, coarse, p.quota, p.list_cap, cidx, cval, cmeta); });
             } else if (fast) {
                 stacr_launch("k_proj_hist_b", s, [&] { k_proj_hist_b<DT, R, V, kRin><<<nwg, kBlock, 0, s>>>(p.g, fg, x, qp, coeff_out, hist, maxkey, resid ? 1 : 0, coeff_in, rbuf, coarse); });
             }
@@ -3362,7 +3375,7 @@ int launch_typed(const StacrSaveArgs &a, const Plan &p, char *ws, const size_t *
                         stacr_launch("k_refine_lists", s, [&] {
                             const auto k = few ? k_refine_lists<decltype(hc)::value, 1> : k_refine_lists<decltype(hc)::value, kListWaves>;
                             k<<<n_list_wgs, few ? 64 : 64 * kListWaves, 0, s>>>(p.g, p.Rq, p.n_wgs, x, qp, coeff, hist, state, kf, kl,
-                                                                               maxkey, fold, coarse, cval, cmeta);
+                                                                               maxkey, fold, coarse, p.list_cap, cval, cmeta);
                         });
                 };
                 auto refine_lists = [&](auto hc) {
@@ -3417,7 +3430,7 @@ int launch_typed(const StacrSaveArgs &a, const Plan &p, char *ws, const size_t *
                 stacr_launch("k_emit_lists", s, [&] {
                     const auto k = few ? k_emit_lists<decltype(hc)::value, 1> : k_emit_lists<decltype(hc)::value, kListWaves>;
                     k<<<n_list_wgs, few ? 64 : 64 * kListWaves, 0, s>>>(p.g, p.Rq, p.n_wgs, x, qp, coeff, state, kf, maxkey, o, a.scale,
-                                                                        p.trim ? 1 : 0, hist, fold, cidx, cval, cmeta, cen, kt);
+                                                                        p.trim ? 1 : 0, hist, fold, p.list_cap, cidx, cval, cmeta, cen, kt);
                 });
             };
             auto emit_rin = [&](auto hc) {

@@ -94,6 +94,24 @@ def test_workspace_queries_and_error_paths():
     assert rc == 1
 
 
+@pytest.mark.parametrize("rows,feats,rank,mode,budget,chunk,limit", [
+    (32768, 768, 16, 1, 0.005, 512, 76_008_704), (32768, 1024, 16, 1, 0.005, 512, 92_826_880),
+    (131072, 512, 16, 1, 0.005, 512, 185_208_064), (8192, 264, 16, 1, 0.005, 512, 7_736_832),
+    (8192, 2048, 16, 1, 0.03, 512, 47_000_000), (8192, 1024, 16, 1, 0.05, 512, 23_479_552),
+    (32768, 768, 8, 1, 0.005, 512, 25_615_616), (8192, 1024, 8, 0, 0.005, 511, 111_006_208),
+    (8192, 264, 16, 0, 0.005, 511, 115_404_288), (8192, 1024, 8, 1, 0.014, 512, 6_620_416),
+])
+def test_save_workspace_is_no_larger_than_a_stored_residual_needs(rows, feats, rank, mode, budget, chunk, limit):
+    """Scratch of a bf16 save against what the stored residual with lists of 2048 entries (wide rows), or such
+    lists alone (rank 8), take: a list is no larger than its workgroup's share asks for."""
+    _lib()
+    from stacr_amd import _lib as lib
+
+    b = ctypes.c_size_t()
+    assert lib.load().stacr_save_workspace_bytes(rows, feats, rank, 1, mode, budget, chunk, 8, ctypes.byref(b)) == 0
+    assert b.value <= limit
+
+
 def test_python_errors_map_from_status_codes():
     from stacr_amd import _lib as L
 

@@ -1731,6 +1731,24 @@ __device__ __forceinline__ uint32_t bf16_pair(float lo, float hi)
 __device__ __forceinline__ uint32_t bin_lo(uint32_t w) { return __builtin_amdgcn_ubfe(w, 4, 11); }
 __device__ __forceinline__ uint32_t bin_hi(uint32_t w) { return __builtin_amdgcn_ubfe(w, 20, 11); }
 
+// Bit e: element e's |r|, as bits, is at least `low` (0: every element).  Two at a time: a saturating
+// difference to low - 1 is nonzero there.
+__device__ __forceinline__ uint32_t mask_ge(const uint32_t (&w)[4], uint32_t low)
+{
+    typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+    const unsigned short below = (unsigned short)(low - 1u);
+    const u16x2 below2 = {below, below}, one2 = {1, 1};
+    uint32_t k8 = 0u;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        u16x2 t = __builtin_elementwise_sub_sat(__builtin_bit_cast(u16x2, w[k] & 0x7fff7fffu), below2);
+        asm("" : "+v"(t));  // (kept packed: seen through, the two steps become single compares and selects)
+        t = __builtin_elementwise_min(t, one2);
+        k8 |= __builtin_bit_cast(uint32_t, t) << (2 * k);  // elements 2 k at bit 2 k, 2 k + 1 at 16 + 2 k
+    }
+    return low ? (k8 | (k8 >> 15)) & 0xffu : 0xffu;
+}
+
 // A workgroup's cut, by one wave: the highest bin of its histogram where the count from the top reaches
 // the quota (bin 0 when it has fewer keys), from 64 sums of 32 bins and then the chosen 32 bins.  Where
 // that bin's keys do not fit the list (rows of zeros, or any value repeated over the rows, put thousands in one
@@ -2204,28 +2222,16 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(R == 8 && MV
     __syncthreads();
     // ---- the candidates in ascending flat order: (row, vector, wave, lane, element)
     const uint32_t cut = s_cut;
-    // A vector's 8-bit mask of elements in the cut's bin and above: |r|'s bits against the bin's lowest
-    // value, two at a time (a saturating difference is nonzero at or above it).
-    const unsigned short below = (unsigned short)((cut << 4) - 1u);  // (cut 0: every element)
-    const u16x2 below2 = {below, below}, one2 = {1, 1};
+    // a vector's 8-bit mask of elements in the cut's bin and above
     constexpr int NV = NB * MV;
     uint32_t msk[NV];
 #pragma unroll
     for (int i = 0; i < NB; ++i)
 #pragma unroll
         for (int m = 0; m < MV; ++m) {
+            const uint32_t w[4] = {raw[i][m].x, raw[i][m].y, raw[i][m].z, raw[i][m].w};
             uint32_t k8 = 0u;
-            if (col_ok[m] && i < n_rows) {
-                const uint32_t w[4] = {raw[i][m].x, raw[i][m].y, raw[i][m].z, raw[i][m].w};
-#pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    u16x2 t = __builtin_elementwise_sub_sat(__builtin_bit_cast(u16x2, w[k] & 0x7fff7fffu), below2);
-                    asm("" : "+v"(t));  // (kept packed: seen through, the two steps become single compares and selects)
-                    t = __builtin_elementwise_min(t, one2);
-                    k8 |= __builtin_bit_cast(uint32_t, t) << (2 * k);  // elements 2 k at bit 2 k, 2 k + 1 at 16 + 2 k
-                }
-                k8 = cut ? (k8 | (k8 >> 15)) & 0xffu : 0xffu;
-            }
+            if (col_ok[m] && i < n_rows) k8 = mask_ge(w, cut << 4);
             msk[i * MV + m] = k8;
         }
     // their places: prefix sums over the lanes, two vectors' counts (at most 512 a wave) a word, then one
@@ -2305,12 +2311,16 @@ struct CandVals {
 // One wave per list (a projection workgroup's candidates, a few hundred): these passes are a chain of
 // dependent loads and a little arithmetic, so their time is that chain's latency times the rounds of
 // waves the lists take.  A wave a list instead of a workgroup puts every list of 8192 projection workgroups
-// on the chip at once and needs no barrier (8192 lists of about 880: level 1 90 -> 15 us, emission 102 -> 22 us; eight a workgroup 18 and 30 us).
-// A list that is not usable is recomputed by its whole workgroup.
+// on the chip at once and needs no barrier (8192 lists of about 880: level 1 90 -> 15 us, emission 102 -> 22 us;
+// eight a workgroup 18 and 30 us).  A list that is not usable is recomputed by its whole workgroup, and one such
+// list sets the pass's time: up to kFewRefine (kFewEmit) lists, each has a workgroup of its own, so that no
+// workgroup meets two (1024 lists of 8 x 4096, 20 of them not usable: level 1 41 -> 26 us, with none 10.1 and
+// 10.6 us; emission with none 20 us, but 24 at a workgroup a list).
 constexpr int kListWaves = 4;          // lists of a workgroup
-constexpr int kFewLists = 255;         // up to this many lists, a workgroup each: every list a compute unit (measured: 48
-                                       // lists 9.1 -> 8.0 us, but 512 lists 8.6 -> 9.7)
+constexpr int kFewRefine = 1024;
+constexpr int kFewEmit = 512;
 constexpr int kListRound = 64 * 8;     // candidates a wave reads at once
+constexpr int kListC = 256;            // coefficients of a list's rows, padded: 64 x the row slots of a workgroup (at most 4)
 
 // A lane's 8 consecutive candidate values of round k (zeros past the list).
 __device__ __forceinline__ CandVals list_vals(const uint16_t *__restrict__ cand_val, int64_t list, uint32_t cap, int k, uint32_t n)
@@ -2323,107 +2333,253 @@ __device__ __forceinline__ CandVals list_vals(const uint16_t *__restrict__ cand_
     return r;
 }
 
-// The residuals of 8 columns of a row, recomputed from X, the saved C and the basis (the fallback of a list
-// that is not usable): the projection pass's chain, one basis column at a time.
-__device__ __forceinline__ void list_residual(const SaveGeom &g, int R, const uint16_t *__restrict__ x,
-                                              const uint16_t *__restrict__ qph, const uint16_t *__restrict__ coeff,
-                                              int64_t row, int64_t col, float (&r)[8])
+// A list that is not usable: its rows' residuals again from X, the saved C and the basis, by the whole
+// workgroup.  About one list in fifty is such a one where the basis is fitted to X (the rows that an
+// outlier's projection disturbs hold most of the entries), so the few workgroups that meet one set the pass's
+// time: a wave a SIMD, bound by its own instructions and the loads' latency.  Each thread takes two adjacent
+// vectors of 8 columns a round, in flat order, with the next round's X in flight and its basis words loaded
+// together; C is in LDS.  8 x 4096 at rank 8: 16 us a list (the basis words a round ahead as well: the same, and
+// 130 registers).  With four lists a workgroup, where registers decide how many lists are on the chip, one vector
+// a thread and four columns' words at a time (57 registers where the other form has 140; 131072 x 1024, rank 16,
+// in chunks: level 1 30 and 45 us; 32768 x 2048 fitted: 30 and 27 us).
+// s_c holds C as [row of the list][R], zero past the rank; every thread must call both.
+__device__ __forceinline__ void list_stage_c(const SaveGeom &g, int R, const uint16_t *__restrict__ coeff, int64_t row0,
+                                             int64_t row_end, float *__restrict__ s_c)
 {
-    float p[8];
+    __syncthreads();  // (the list before may still be read)
+    for (int e = threadIdx.x; e < (int)(row_end - row0) * R; e += kBlock) {
+        const int i = e / R, j = e - i * R;
+        s_c[e] = j < g.rank ? bf16_bits_to_f(coeff[(row0 + i) * g.rank + j]) : 0.f;
+    }
+    __syncthreads();
+}
+
+// p += the chain of four basis columns over one vector.
+__device__ __forceinline__ void list_chain4(const uint4 &q0, const uint4 &q1, const uint4 &q2, const uint4 &q3, float4 c,
+                                            float (&p)[8])
+{
+    const uint4 q[4] = {q0, q1, q2, q3};
+    const float cs[4] = {c.x, c.y, c.z, c.w};
 #pragma unroll
-    for (int e = 0; e < 8; ++e) p[e] = 0.f;
-#pragma unroll 4  // (R is 4, 8, 16 or 32) four columns' words in flight
-    for (int j = 0; j < R; ++j) {
-        const uint4 v = *reinterpret_cast<const uint4 *>(qph + j * g.d + col);
-        const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-        const float c = j < g.rank ? bf16_bits_to_f(coeff[row * g.rank + j]) : 0.f;
+    for (int j = 0; j < 4; ++j) {
+        const uint32_t qv[4] = {q[j].x, q[j].y, q[j].z, q[j].w};
 #pragma unroll
         for (int e = 0; e < 8; ++e)
-            p[e] = fmaf(c, __uint_as_float(e & 1 ? w[e >> 1] & 0xffff0000u : w[e >> 1] << 16), p[e]);
+            p[e] = fmaf(cs[j], __uint_as_float(e & 1 ? qv[e >> 1] & 0xffff0000u : qv[e >> 1] << 16), p[e]);
     }
-    float xv[8];
-    load_vec<STACR_DTYPE_BF16, 8>(x + row * g.d + col, xv);
-    using A = Act<STACR_DTYPE_BF16>;
+}
+
+// w = the packed residuals of a vector x with projection p.
+__device__ __forceinline__ void list_residual(uint4 x, const float (&p)[8], uint32_t (&w)[4])
+{
+    const uint32_t xw[4] = {x.x, x.y, x.z, x.w};
 #pragma unroll
-    for (int e = 0; e < 8; ++e) r[e] = A::rnd(xv[e] - A::rnd(p[e]));
+    for (int k = 0; k < 4; ++k) {
+        const uint32_t pb = bf16_pair(p[2 * k], p[2 * k + 1]);
+        w[k] = bf16_pair(__uint_as_float(xw[k] << 16) - __uint_as_float(pb << 16),
+                         __uint_as_float(xw[k] & 0xffff0000u) - __uint_as_float(pb & 0xffff0000u));
+    }
+}
+
+// round(v, n_vec, w): the packed residuals of vectors v and v + 1 (of n_vec; those past it hold anything).
+template <int R, typename Round>
+__device__ __forceinline__ void list_rounds_r(const SaveGeom &g, const uint16_t *__restrict__ x,
+                                              const uint16_t *__restrict__ qph, const float *__restrict__ s_c, int64_t row0,
+                                              int64_t row_end, Round &round)
+{
+    const int per_row = (int)(g.d / 8), n_vec = (int)(row_end - row0) * per_row;
+    const uint4 *xs = reinterpret_cast<const uint4 *>(x + row0 * g.d);
+    int v = 2 * (int)threadIdx.x;
+    uint4 nx[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) nx[i] = xs[min(v + i, n_vec - 1)];
+#pragma unroll 1
+    for (int v0 = 0; v0 < n_vec; v0 += 2 * kBlock, v += 2 * kBlock) {
+        const int vc = min(v, n_vec - 1), row = vc / per_row, col = vc - row * per_row;
+        const bool wrap = col + 1 == per_row;  // the second vector begins the next row (past the last row: not used)
+        const uint16_t *q[2] = {qph + 8 * col, qph + (wrap ? 0 : 8 * (col + 1))};
+        const float *c[2] = {s_c + row * R, s_c + min(row + wrap, (int)(row_end - row0) - 1) * R};
+        uint4 qw[2][R], xc[2];
+#pragma unroll
+        for (int j = 0; j < R; ++j)
+#pragma unroll
+            for (int i = 0; i < 2; ++i) qw[i][j] = *reinterpret_cast<const uint4 *>(q[i] + j * g.d);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            xc[i] = nx[i];
+            nx[i] = xs[min(v + 2 * kBlock + i, n_vec - 1)];
+        }
+        float p[2][8] = {};
+        uint32_t w[2][4];
+#pragma unroll
+        for (int j = 0; j < R; j += 4)
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+                list_chain4(qw[i][j], qw[i][j + 1], qw[i][j + 2], qw[i][j + 3], *reinterpret_cast<const float4 *>(c[i] + j), p[i]);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) list_residual(xc[i], p[i], w[i]);
+        round(v, n_vec, w);
+    }
+}
+
+template <typename Round>
+__device__ __forceinline__ void list_rounds(const SaveGeom &g, int R, const uint16_t *__restrict__ x,
+                                            const uint16_t *__restrict__ qph, const float *__restrict__ s_c, int64_t row0,
+                                            int64_t row_end, Round &&round)
+{
+    if (R == 4) list_rounds_r<4>(g, x, qph, s_c, row0, row_end, round);
+    else if (R == 8) list_rounds_r<8>(g, x, qph, s_c, row0, row_end, round);
+    else list_rounds_r<16>(g, x, qph, s_c, row0, row_end, round);
+}
+
+// The same with one vector a thread and four basis columns at a time: round(v, n_vec, w).
+template <typename Round>
+__device__ __forceinline__ void list_rounds_small(const SaveGeom &g, int R, const uint16_t *__restrict__ x,
+                                                  const uint16_t *__restrict__ qph, const float *__restrict__ s_c,
+                                                  int64_t row0, int64_t row_end, Round &&round)
+{
+    const int per_row = (int)(g.d / 8), n_vec = (int)(row_end - row0) * per_row;
+    const uint4 *xs = reinterpret_cast<const uint4 *>(x + row0 * g.d);
+#pragma unroll 1
+    for (int v0 = 0; v0 < n_vec; v0 += kBlock) {
+        const int v = v0 + (int)threadIdx.x, vc = min(v, n_vec - 1), row = vc / per_row;
+        const uint16_t *q = qph + 8 * (vc - row * per_row);
+        const uint4 xc = xs[vc];
+        float p[8] = {};
+#pragma unroll 1
+        for (int j = 0; j < R; j += 4) {
+            uint4 qw[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) qw[k] = *reinterpret_cast<const uint4 *>(q + (j + k) * g.d);
+            list_chain4(qw[0], qw[1], qw[2], qw[3], *reinterpret_cast<const float4 *>(s_c + row * R + j), p);
+        }
+        uint32_t w[4];
+        list_residual(xc, p, w);
+        round(v, n_vec, w);
+    }
+}
+
+// Element e of a packed vector, and of two.  (By value: behind a reference the selects become a load from an
+// array in memory.)
+__device__ __forceinline__ uint32_t list_word(uint4 w, int e)
+{
+    return ((e & 4 ? (e & 2 ? w.w : w.z) : (e & 2 ? w.y : w.x)) >> (16 * (e & 1))) & 0xffffu;
+}
+
+__device__ __forceinline__ uint32_t list_word(uint4 w0, uint4 w1, int e)
+{
+    const uint32_t lo = list_word(w0, e), hi = list_word(w1, e);
+    return e & 8 ? hi : lo;
 }
 
 // Level 1: the level-0 selection, then the 16 live bins of key bits 19..16 inside B0 (bf16: the bits below are
-// zero) and the records of k_refine_hist_b: cum[b] for b = 0..15, and cum[16], the count above B0.
+// zero) and the records of k_refine_hist_b: cum[b] for b = 0..15, and cum[16], the count above B0.  A list that
+// is not usable is recomputed and written anew with B0 as its cut, so that the emission can read it (unless it
+// holds more than the list's slots there).
 template <int HC, int LW>
-__global__ __launch_bounds__(64 * LW) void k_refine_lists(SaveGeom g, int R, int64_t n_lists,
-                                                                  const uint16_t *__restrict__ x,
-                                                                  const float *__restrict__ qp,
-                                                                  const uint16_t *__restrict__ coeff,
-                                                                  uint32_t *__restrict__ hist, SelState *__restrict__ state,
-                                                                  uint32_t k_full, uint32_t k_last,
-                                                                  uint32_t *__restrict__ maxkey, uint32_t *__restrict__ fold,
-                                                                  const uint32_t *__restrict__ coarse, uint32_t cap,
-                                                                  const uint16_t *__restrict__ cand_val,
-                                                                  const CandMeta *__restrict__ meta)
+__global__ __launch_bounds__(kBlock) void k_refine_lists(SaveGeom g, int R, int64_t n_lists,
+                                                         const uint16_t *__restrict__ x, const float *__restrict__ qp,
+                                                         const uint16_t *__restrict__ coeff,
+                                                         uint32_t *__restrict__ hist, SelState *__restrict__ state,
+                                                         uint32_t k_full, uint32_t k_last,
+                                                         uint32_t *__restrict__ maxkey, uint32_t *__restrict__ fold,
+                                                         const uint32_t *__restrict__ coarse, uint32_t cap,
+                                                         uint32_t *__restrict__ cand_idx, uint16_t *__restrict__ cand_val,
+                                                         CandMeta *__restrict__ meta)
 {
     __shared__ uint32_t s_cnt[LW][16];
     __shared__ uint32_t s_above[LW];
     __shared__ uint32_t s_redo[LW];  // the list's B0 + 1 when its workgroup recomputes it, else 0
+    __shared__ uint32_t s_wt[kWaves];
+    __shared__ __align__(16) float s_c[kListC];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int64_t list_raw = (int64_t)blockIdx.x * LW + wave;
     const int64_t list = min(list_raw, n_lists - 1);
     int64_t chunk, row0, row_end;
     wg_rows(g, list, chunk, row0, row_end);
-    const bool in = list_raw < n_lists, has_rows = in && row0 < row_end;
-    const SelState sp = prev_state(0, state, chunk, g.n_chunks, k_full, k_last);
-    uint32_t cv[HC];
-#pragma unroll
-    for (int h = 0; h < HC; ++h) cv[h] = coarse[(chunk * HC + h) * kCoarse + lane];
-    const CandMeta mine = meta[has_rows ? list : 0];
-    const uint32_t n = has_rows ? min(mine.count, cap) : 0u;
-    // the first two rounds go out before the selection's words
-    CandVals v0 = list_vals(cand_val, list, cap, 0, n), v1 = list_vals(cand_val, list, cap, 1, n);
-    if (lane < 16) s_cnt[wave][lane] = 0u;
-    const SelState sel = select_level0<HC>(cv, hist + chunk * 3 * HC * kBins, sp);
-    if (in && list == chunk * g.wgs_per_chunk && lane == 0) state[chunk * 3 + 0] = sel;
-    if (HC > 1 && list_raw == 0 && lane == 0) {  // fold the max key's copies into the first
-        uint32_t m = maxkey[0];
-#pragma unroll
-        for (int c = 1; c < HC; ++c) m = max(m, maxkey[c * kMaxKeyStride]);
-        maxkey[0] = m;
-    }
-    const uint32_t prefix = sel.prefix;  // B0
-    const bool usable = !has_rows || (mine.count <= cap && mine.cut <= prefix);  // (uniform in the wave)
-    if (lane == 0) s_redo[wave] = usable ? 0u : prefix + 1u;
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the counters are clear before any lane adds
+    const bool in = wave < LW && list_raw < n_lists, has_rows = in && row0 < row_end;
     uint32_t above = 0u;
     auto count = [&](uint32_t key, uint32_t b0, int l) {
         if ((key >> kDigitShift[0]) == b0) atomicAdd(&s_cnt[l][(key >> 16) & 15u], 1u);
         above += (key >> kDigitShift[0]) > b0;
     };
-    if (usable) {
-        for (int k = 0; k * kListRound < (int)n; ++k) {
-            const CandVals v = v0;
-            v0 = v1;
-            v1 = list_vals(cand_val, list, cap, k + 2, n);
+    if (wave < LW) {
+        const SelState sp = prev_state(0, state, chunk, g.n_chunks, k_full, k_last);
+        uint32_t cv[HC];
 #pragma unroll
-            for (int j = 0; j < 8; ++j)
-                if ((uint32_t)(k * kListRound + 8 * lane + j) < n) count(bf16_key(v.bits(j)), prefix, wave);
+        for (int h = 0; h < HC; ++h) cv[h] = coarse[(chunk * HC + h) * kCoarse + lane];
+        const CandMeta mine = has_rows ? meta[list] : CandMeta{0u, 0u};
+        const uint32_t n = min(mine.count, cap);
+        // the first two rounds go out before the selection's words
+        CandVals v0 = list_vals(cand_val, list, cap, 0, n), v1 = list_vals(cand_val, list, cap, 1, n);
+        if (lane < 16) s_cnt[wave][lane] = 0u;
+        const SelState sel = select_level0<HC>(cv, hist + chunk * 3 * HC * kBins, sp);
+        if (in && list == chunk * g.wgs_per_chunk && lane == 0) state[chunk * 3 + 0] = sel;
+        if (HC > 1 && list_raw == 0 && lane == 0) {  // fold the max key's copies into the first
+            uint32_t m = maxkey[0];
+#pragma unroll
+            for (int c = 1; c < HC; ++c) m = max(m, maxkey[c * kMaxKeyStride]);
+            maxkey[0] = m;
         }
+        const uint32_t prefix = sel.prefix;  // B0
+        const bool usable = !has_rows || (mine.count <= cap && mine.cut <= prefix);  // (uniform in the wave)
+        if (lane == 0) s_redo[wave] = usable ? 0u : prefix + 1u;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the counters are clear before any lane adds
+        if (usable) {
+            for (int k = 0; k * kListRound < (int)n; ++k) {
+                const CandVals v = v0;
+                v0 = v1;
+                v1 = list_vals(cand_val, list, cap, k + 2, n);
+#pragma unroll
+                for (int j = 0; j < 8; ++j)
+                    if ((uint32_t)(k * kListRound + 8 * lane + j) < n) count(bf16_key(v.bits(j)), prefix, wave);
+            }
+        }
+        above = (uint32_t)__shfl((int)wave_inclusive_scan(above), 63, 64);
+        if (lane == 0) s_above[wave] = above;
     }
-    above = (uint32_t)__shfl((int)wave_inclusive_scan(above), 63, 64);
-    if (lane == 0) s_above[wave] = above;
     __syncthreads();
     for (int l = 0; l < LW; ++l) {
         if (s_redo[l] == 0u) continue;  // (uniform)
+        const int64_t list2 = (int64_t)blockIdx.x * LW + l;
+        const uint32_t b0 = s_redo[l] - 1u;
         int64_t c2, r0, r1;
-        wg_rows(g, (int64_t)blockIdx.x * LW + l, c2, r0, r1);
+        wg_rows(g, list2, c2, r0, r1);
+        list_stage_c(g, R, coeff, r0, r1, s_c);
         above = 0u;
-        const int per_row = (int)(g.d / 8), n_vec = (int)(r1 - r0) * per_row;
-        for (int v = threadIdx.x; v < n_vec; v += 64 * LW) {
-            float r[8];
-            list_residual(g, R, x, reinterpret_cast<const uint16_t *>(qp + 2 * g.d * R), coeff, r0 + v / per_row,
-                          8 * (v % per_row), r);
-#pragma unroll
-            for (int e = 0; e < 8; ++e) count(__float_as_uint(r[e]) & 0x7fffffffu, s_redo[l] - 1u, l);
-        }
+        uint32_t *ci = cand_idx + list2 * cap;
+        uint16_t *cv = cand_val + list2 * cap;
+        uint32_t before = 0u;  // candidates of the earlier rounds
+        // the candidates of vectors v .. v + U - 1 from their packed residuals (those past n_vec masked)
+        auto take = [&](int v, uint32_t m, auto word) {
+            uint32_t tot;
+            uint32_t pos = before + block_exclusive_scan((uint32_t)__popc(m), s_wt, &tot);
+            for (uint32_t k = m; k != 0u; k &= k - 1u, ++pos) {  // (only the elements of bin B0 and above, one by one)
+                const int e = __builtin_ctz(k);
+                const uint32_t val = word(e);
+                count(bf16_key(val), b0, l);
+                if (pos < cap) {
+                    ci[pos] = (uint32_t)(r0 * g.d) + 8u * (uint32_t)v + (uint32_t)e;
+                    cv[pos] = (uint16_t)val;
+                }
+            }
+            before += tot;
+        };
+        const uint16_t *qph = reinterpret_cast<const uint16_t *>(qp + 2 * g.d * R);
+        const uint32_t low = b0 << 4;
+        if constexpr (LW == 1)
+            list_rounds(g, R, x, qph, s_c, r0, r1, [&](int v, int n_vec, const uint32_t (&w)[2][4]) {
+                const uint4 w0 = make_uint4(w[0][0], w[0][1], w[0][2], w[0][3]), w1 = make_uint4(w[1][0], w[1][1], w[1][2], w[1][3]);
+                take(v, (mask_ge(w[0], low) | mask_ge(w[1], low) << 8) & (v + 1 < n_vec ? 0xffffu : v < n_vec ? 0xffu : 0u),
+                     [&](int e) { return list_word(w0, w1, e); });
+            });
+        else
+            list_rounds_small(g, R, x, qph, s_c, r0, r1, [&](int v, int n_vec, const uint32_t (&w)[4]) {
+                const uint4 w0 = make_uint4(w[0], w[1], w[2], w[3]);
+                take(v, mask_ge(w, low) & (v < n_vec ? 0xffu : 0u), [&](int e) { return list_word(w0, e); });
+            });
         if (above) atomicAdd(&s_above[l], above);
+        if (threadIdx.x == 0) meta[list2] = CandMeta{b0, before};
     }
     __syncthreads();
     if (!in) return;
@@ -2444,7 +2600,7 @@ __global__ __launch_bounds__(64 * LW) void k_refine_lists(SaveGeom g, int R, int
 // per feature in LDS first: two 16-bit counts a word (features f and f + 2048; a feature has at most one entry
 // a row, so no half overflows), rows of at most 4096 features.
 template <int HC, int LW>
-__global__ __launch_bounds__(64 * LW) void k_emit_lists(
+__global__ __launch_bounds__(kBlock) void k_emit_lists(
     SaveGeom g, int R, int64_t n_lists, const uint16_t *__restrict__ x, const float *__restrict__ qp,
     const uint16_t *__restrict__ coeff, SelState *__restrict__ state, uint32_t chunk_k,
     const uint32_t *__restrict__ maxkey, OutSpec o, float *scale_out, int to_list, const uint32_t *__restrict__ hist,
@@ -2455,21 +2611,22 @@ __global__ __launch_bounds__(64 * LW) void k_emit_lists(
     constexpr int DT = STACR_DTYPE_BF16;
     __shared__ uint32_t s_feat[kBins];
     __shared__ uint32_t s_redo[LW], s_T[LW], s_off[LW], s_take[LW];
-    __shared__ uint32_t s_wt[LW];
+    __shared__ uint32_t s_wt[kWaves];
+    __shared__ __align__(16) float s_c[kListC];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int64_t list_raw = (int64_t)blockIdx.x * LW + wave;
     const int64_t list = min(list_raw, n_lists - 1);
     int64_t chunk, row0, row_end;
     wg_rows(g, list, chunk, row0, row_end);
     const int64_t w = list - chunk * g.wgs_per_chunk, wg0 = chunk * g.wgs_per_chunk;
-    const bool live = list_raw < n_lists && row0 < row_end;  // (a trailing list with no rows writes nothing)
+    const bool live = wave < LW && list_raw < n_lists && row0 < row_end;  // (a trailing list with no rows writes nothing)
     uint32_t hw[HC];
     {
         const uint32_t *h1 = hist + (chunk * 3 + 1) * HC * kBins + ((lane & 15) << 7);
 #pragma unroll
         for (int c = 0; c < HC; ++c) hw[c] = h1[c * kBins];
     }
-    const CandMeta mine = meta[live ? list : 0];
+    const CandMeta mine = live ? meta[list] : CandMeta{0u, 0u};
     const uint32_t n = min(mine.count, cap);
     struct Round {
         CandVals v;
@@ -2504,7 +2661,7 @@ __global__ __launch_bounds__(64 * LW) void k_emit_lists(
     const uint32_t cfeat = (uint32_t)g.d, dmask = (cfeat & (cfeat - 1)) == 0 ? cfeat - 1u : 0u;
     const uint32_t cwords = min(cfeat, (uint32_t)kBins);
     if (census) {
-        for (uint32_t f = threadIdx.x; f < cwords; f += 64 * LW) s_feat[f] = 0u;
+        for (uint32_t f = threadIdx.x; f < cwords; f += kBlock) s_feat[f] = 0u;
         __syncthreads();
     }
     auto put = [&](uint32_t pos, uint32_t fl, float rv) {
@@ -2522,7 +2679,7 @@ __global__ __launch_bounds__(64 * LW) void k_emit_lists(
         }
     };
     const bool usable = !live || (mine.count <= cap && mine.cut <= (T >> kDigitShift[0]));  // (uniform in the wave)
-    if (lane == 0) s_redo[wave] = usable ? 0u : 1u;
+    if (wave < LW && lane == 0) s_redo[wave] = usable ? 0u : 1u;
     if (live) {
         WgOffset wo;
         {
@@ -2584,40 +2741,36 @@ __global__ __launch_bounds__(64 * LW) void k_emit_lists(
         if (s_redo[l] == 0u) continue;  // (uniform)
         int64_t c2, r0, r1;
         wg_rows(g, (int64_t)blockIdx.x * LW + l, c2, r0, r1);
+        list_stage_c(g, R, coeff, r0, r1, s_c);
         const uint32_t Tl = s_T[l], off = s_off[l], take = s_take[l];
-        const int per_row = (int)(g.d / 8), n_vec = (int)(r1 - r0) * per_row;
         uint32_t gt_before = 0u, eq_before = 0u;
-        for (int v0 = 0; v0 < n_vec; v0 += 64 * LW) {
-            const int v = v0 + (int)threadIdx.x, vc = min(v, n_vec - 1);
-            const int64_t row = r0 + vc / per_row, col = 8 * (vc % per_row);
-            float r[8];
-            list_residual(g, R, x, reinterpret_cast<const uint16_t *>(qp + 2 * g.d * R), coeff, row, col, r);
-            uint32_t m = 0u;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const uint32_t key = __float_as_uint(r[e]) & 0x7fffffffu;
-                m |= v < n_vec && key > Tl ? 1u << e : 0u;
-                m |= v < n_vec && key == Tl ? 0x100u << e : 0u;
-            }
-            const uint32_t c = (uint32_t)__popc(m & 0xffu) | ((uint32_t)__popc(m >> 8) << 16);
+        // (the lists that level 1 could not write anew, so seldom any)
+        list_rounds_small(g, R, x, reinterpret_cast<const uint16_t *>(qp + 2 * g.d * R), s_c, r0, r1,
+                          [&](int v, int n_vec, const uint32_t (&w)[4]) {
+            const uint32_t live8 = v < n_vec ? 0xffu : 0u, low = Tl >> 16;  // (a bf16 key has no bits below 16)
+            const uint32_t ge = mask_ge(w, low) & live8, gt = mask_ge(w, low + 1u) & live8;
+            const uint32_t c = (uint32_t)__popc(gt) | ((uint32_t)__popc(ge ^ gt) << 16);
             uint32_t tot;
-            const uint32_t ex = block_exclusive_scan<64 * LW>(c, s_wt, &tot);  // (at most 4096 of each)
+            const uint32_t ex = block_exclusive_scan(c, s_wt, &tot);  // (at most 2048 of each)
             uint32_t gb = gt_before + (ex & 0xffffu), eb = eq_before + (ex >> 16);
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const bool is_gt = (m >> e) & 1u, is_eq = (m >> (8 + e)) & 1u;
-                if (is_gt || (is_eq && eb < take)) put(off + gb + min(eb, take), (uint32_t)(row * g.d + col + e), r[e]);
+            const uint4 w0 = make_uint4(w[0], w[1], w[2], w[3]);
+            for (uint32_t k = ge; k != 0u; k &= k - 1u) {
+                const int e = __builtin_ctz(k);
+                const bool is_gt = (gt >> e) & 1u;
+                if (is_gt || eb < take)
+                    put(off + gb + min(eb, take), (uint32_t)(r0 * g.d) + 8u * (uint32_t)v + (uint32_t)e,
+                        bf16_bits_to_f(list_word(w0, e)));
                 gb += is_gt;
-                eb += is_eq;
+                eb += !is_gt;
             }
             gt_before += tot & 0xffffu;
             eq_before += tot >> 16;
-        }
+        });
     }
     if (census) {  // the entries per feature
         __syncthreads();
         uint32_t *counts = census + (int64_t)(blockIdx.x % kCensusCopies) * cfeat;
-        for (uint32_t f = threadIdx.x; f < cwords; f += 64 * LW) {
+        for (uint32_t f = threadIdx.x; f < cwords; f += kBlock) {
             const uint32_t v = s_feat[f];
             if (v & 0xffffu) atomicAdd(&counts[f], v & 0xffffu);
             if (v >> 16) atomicAdd(&counts[f + kBins], v >> 16);
@@ -3280,8 +3433,8 @@ int launch_typed(const StacrSaveArgs &a, const Plan &p, char *ws, const size_t *
     WgCount *counts = carve<WgCount>(ws, off[WS_COUNTS]);
     const bool resid = a.k_total > 0;
     const int nwg = (int)p.n_wgs;
-    const bool few = p.n_wgs <= kFewLists;
-    const unsigned n_list_wgs = (unsigned)(few ? p.n_wgs : (p.n_wgs + kListWaves - 1) / kListWaves);
+    const bool few_refine = p.n_wgs <= kFewRefine, few_emit = p.n_wgs <= kFewEmit;
+    auto list_wgs = [&](bool few) { return (unsigned)(few ? p.n_wgs : (p.n_wgs + kListWaves - 1) / kListWaves); };
 
     // padded basis; histograms and max key (contiguous in the layout) cleared in the same launch
     const int64_t n_zero = resid ? (int64_t)((off[WS_MAXKEY] + (size_t)p.g.hcopies * kMaxKeyStride * sizeof(uint32_t) -
@@ -3373,9 +3526,9 @@ int launch_typed(const StacrSaveArgs &a, const Plan &p, char *ws, const size_t *
                 auto refine_cand = [&](auto hc) {
                     if constexpr (kCandOk)
                         stacr_launch("k_refine_lists", s, [&] {
-                            const auto k = few ? k_refine_lists<decltype(hc)::value, 1> : k_refine_lists<decltype(hc)::value, kListWaves>;
-                            k<<<n_list_wgs, few ? 64 : 64 * kListWaves, 0, s>>>(p.g, p.Rq, p.n_wgs, x, qp, coeff, hist, state, kf, kl,
-                                                                               maxkey, fold, coarse, p.list_cap, cval, cmeta);
+                            const auto k = few_refine ? k_refine_lists<decltype(hc)::value, 1> : k_refine_lists<decltype(hc)::value, kListWaves>;
+                            k<<<list_wgs(few_refine), kBlock, 0, s>>>(p.g, p.Rq, p.n_wgs, x, qp, coeff, hist, state, kf, kl,
+                                                                               maxkey, fold, coarse, p.list_cap, cidx, cval, cmeta);
                         });
                 };
                 auto refine_lists = [&](auto hc) {
@@ -3428,8 +3581,8 @@ int launch_typed(const StacrSaveArgs &a, const Plan &p, char *ws, const size_t *
             const uint32_t kt = (uint32_t)a.k_sum;  // the entries emitted (no trim: the chunks' k summed)
             auto emit = [&](auto hc) {
                 stacr_launch("k_emit_lists", s, [&] {
-                    const auto k = few ? k_emit_lists<decltype(hc)::value, 1> : k_emit_lists<decltype(hc)::value, kListWaves>;
-                    k<<<n_list_wgs, few ? 64 : 64 * kListWaves, 0, s>>>(p.g, p.Rq, p.n_wgs, x, qp, coeff, state, kf, maxkey, o, a.scale,
+                    const auto k = few_emit ? k_emit_lists<decltype(hc)::value, 1> : k_emit_lists<decltype(hc)::value, kListWaves>;
+                    k<<<list_wgs(few_emit), kBlock, 0, s>>>(p.g, p.Rq, p.n_wgs, x, qp, coeff, state, kf, maxkey, o, a.scale,
                                                                         p.trim ? 1 : 0, hist, fold, p.list_cap, cidx, cval, cmeta, cen, kt);
                 });
             };

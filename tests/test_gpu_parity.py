@@ -1043,3 +1043,43 @@ def test_rows_of_zeros_leave_the_lists_usable(dev, rows, d, rank):
     x.view(8, rows // 8, d)[:, rows * 3 // 32:] = 0.0  # eight sequences, the last quarter of each padding
     padded = _list_passes_us(x, qd)
     assert padded <= 2.5 * whole, f"{padded:.1f} us with a quarter of the rows zero, {whole:.1f} us without"
+
+
+@pytest.mark.parametrize("kind,rows,d,rank,mode,budget,chunk,bits", [
+    # 'outlier_rows': lists that hold more than their slots above the chunk's bin (both passes recompute them);
+    # 'outlier_single': lists whose cut lies above it (level 1 writes them anew); 'tie_block': one bin floods lists
+    ("outlier_rows", 1024, 1024, 16, "global_topk", 0.005, 512, 8),
+    ("outlier_single", 1024, 1024, 16, "global_topk", 0.005, 512, 8),
+    ("outlier_single", 4200, 264, 16, "global_topk", 0.005, 512, 4),     # 1050 lists: four a workgroup
+    ("outlier_rows", 4200, 264, 13, "chunk_topk", 0.005, 100, 0),
+    ("outlier_single", 2064, 2048, 16, "chunk_topk", 0.005, 512, 8),
+    ("outlier_single", 600, 8192, 16, "global_topk", 0.005, 512, 8),
+    ("tie_block", 512, 8192, 16, "global_topk", 0.005, 512, 0),
+    ("outlier_single", 1030, 1024, 4, "global_topk", 0.005, 512, 8),
+    ("outlier_single", 1100, 1024, 8, "chunk_topk", 0.005, 11, 8),       # 1100 lists of one row
+    ("outlier_single", 3000, 2064, 8, "global_topk", 0.005, 512, 8),     # vector pairs across rows of 258 vectors
+    ("outlier_rows", 515, 2328, 7, "global_topk", 0.004, 512, 8),        # 291 vectors a row, a partial last list
+])
+def test_save_unusable_lists_match_oracle(dev, kind, rows, d, rank, mode, budget, chunk, bits):
+    announce("save unusable lists", kind, rows, d, rank, mode, budget, chunk, bits)
+    x = _crafted_activation("outlier_rows" if kind == "outlier_single" else kind, rows, d)
+    if kind == "outlier_single":
+        x[32:48] /= 1000.0
+        x[33::100] *= 300.0
+    q = torch.zeros(d, rank) if kind == "tie_block" else make_basis(d, rank)
+    names = _check_save_against_oracle(x.to(dev, torch.bfloat16), q.to(dev, torch.bfloat16), mode, budget, chunk, bits)
+    assert {"k_refine_lists", "k_emit_lists"} <= names
+
+
+@pytest.mark.parametrize("rows,d,rank", [(1024, 1024, 8), (8192, 1024, 8), (8192, 4096, 8)])
+def test_a_fitted_basis_keeps_the_list_passes_fast(dev, rows, d, rank):
+    """With a basis fitted to X about one list in fifty is not usable: the entries gather in the rows that an
+    outlier's projection disturbs.  (Lists recomputed a row of loads at a time, by one wave for up to 255 lists,
+    made these passes 3 to 7 times as long as with a random basis.)"""
+    announce("fitted basis, list passes", rows, d, rank)
+    x = make_activation(rows, d, lognormal=True)
+    _, v = torch.linalg.eigh(x.t().double() @ x.double())
+    xd = x.to(dev, torch.bfloat16)
+    fitted = _list_passes_us(xd, v[:, -rank:].contiguous().to(dev, torch.bfloat16))
+    random = _list_passes_us(xd, make_basis(d, rank).to(dev, torch.bfloat16))
+    assert fitted <= 2.3 * random, f"{fitted:.1f} us with a fitted basis, {random:.1f} us with a random one"

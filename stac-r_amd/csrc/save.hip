@@ -2312,13 +2312,13 @@ struct CandVals {
 // dependent loads and a little arithmetic, so their time is that chain's latency times the rounds of
 // waves the lists take.  A wave a list instead of a workgroup puts every list of 8192 projection workgroups
 // on the chip at once and needs no barrier (8192 lists of about 880: level 1 90 -> 15 us, emission 102 -> 22 us;
-// eight a workgroup 18 and 30 us).  A list that is not usable is recomputed by its whole workgroup, and one such
-// list sets the pass's time: up to kFewRefine (kFewEmit) lists, each has a workgroup of its own, so that no
-// workgroup meets two (1024 lists of 8 x 4096, 20 of them not usable: level 1 41 -> 26 us, with none 10.1 and
-// 10.6 us; emission with none 20 us, but 24 at a workgroup a list).
+// eight a workgroup 18 and 30 us).  Up to kFewLists lists, each has a workgroup of its own: a list that is not
+// usable is recomputed by its whole workgroup and sets the pass's time, so none should meet two, and in the
+// emission the four waves share the earlier lists' records and a long list's rounds (1024 lists of 8 x 4096, 20 of
+// them not usable: level 1 41 -> 26 us, emission 25 -> 19, with none 10.1 and 10.4, 19.3 and 17.3; 128 lists of
+// 16 x 1024: emission 13 -> 10.5 us; 2048 lists of 4 x 1024: 15.3 us, 22.2 at a workgroup a list).
 constexpr int kListWaves = 4;          // lists of a workgroup
-constexpr int kFewRefine = 1024;
-constexpr int kFewEmit = 512;
+constexpr int kFewLists = 1024;
 constexpr int kListRound = 64 * 8;     // candidates a wave reads at once
 constexpr int kListC = 256;            // coefficients of a list's rows, padded: 64 x the row slots of a workgroup (at most 4)
 
@@ -2609,17 +2609,19 @@ __global__ __launch_bounds__(kBlock) void k_emit_lists(
     uint32_t n_entries)
 {
     constexpr int DT = STACR_DTYPE_BF16;
+    constexpr int TW = kWaves / LW;  // waves of a list: its candidates are taken TW rounds at a time, one a wave
     __shared__ uint32_t s_feat[kBins];
     __shared__ uint32_t s_redo[LW], s_T[LW], s_off[LW], s_take[LW];
-    __shared__ uint32_t s_wt[kWaves];
+    __shared__ uint32_t s_wt[kWaves], s_sum[2 * kWaves];
     __shared__ __align__(16) float s_c[kListC];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int64_t list_raw = (int64_t)blockIdx.x * LW + wave;
+    const int slot = wave / TW, tw = wave % TW;
+    const int64_t list_raw = (int64_t)blockIdx.x * LW + slot;
     const int64_t list = min(list_raw, n_lists - 1);
     int64_t chunk, row0, row_end;
     wg_rows(g, list, chunk, row0, row_end);
     const int64_t w = list - chunk * g.wgs_per_chunk, wg0 = chunk * g.wgs_per_chunk;
-    const bool live = wave < LW && list_raw < n_lists && row0 < row_end;  // (a trailing list with no rows writes nothing)
+    const bool live = list_raw < n_lists && row0 < row_end;  // (a trailing list with no rows writes nothing)
     uint32_t hw[HC];
     {
         const uint32_t *h1 = hist + (chunk * 3 + 1) * HC * kBins + ((lane & 15) << 7);
@@ -2643,10 +2645,10 @@ __global__ __launch_bounds__(kBlock) void k_emit_lists(
         r.flat[4] = f1.x; r.flat[5] = f1.y; r.flat[6] = f1.z; r.flat[7] = f1.w;
         return r;
     };
-    Round cur = load_round(0);  // (before the selection's and the offsets' words)
+    Round cur = load_round(tw);  // (before the selection's and the offsets' words)
     SelState sel1;
     const SelState st = fold_select<HC>(hw, state[chunk * 3 + 0], &sel1);
-    if (live && w == 0 && lane == 0) {
+    if (live && w == 0 && lane == 0 && tw == 0) {
         state[chunk * 3 + 1] = sel1;
         state[chunk * 3 + 2] = st;
     }
@@ -2657,7 +2659,7 @@ __global__ __launch_bounds__(kBlock) void k_emit_lists(
     const uint32_t T = st.prefix;
     const float amax = Act<DT>::rnd(__uint_as_float(mk));
     const float scale = o.bits ? quant_scale(mk, o.bits, amax) : 1.f;
-    if (!to_list && list_raw == 0 && lane == 0 && scale_out) *scale_out = scale;
+    if (!to_list && list_raw == 0 && lane == 0 && tw == 0 && scale_out) *scale_out = scale;
     const uint32_t cfeat = (uint32_t)g.d, dmask = (cfeat & (cfeat - 1)) == 0 ? cfeat - 1u : 0u;
     const uint32_t cwords = min(cfeat, (uint32_t)kBins);
     if (census) {
@@ -2678,21 +2680,28 @@ __global__ __launch_bounds__(kBlock) void k_emit_lists(
             atomicAdd(&s_feat[f & (kBins - 1)], f >= (uint32_t)kBins ? 0x10000u : 1u);
         }
     };
-    const bool usable = !live || (mine.count <= cap && mine.cut <= (T >> kDigitShift[0]));  // (uniform in the wave)
-    if (wave < LW && lane == 0) s_redo[wave] = usable ? 0u : 1u;
-    if (live) {
+    const bool usable = !live || (mine.count <= cap && mine.cut <= (T >> kDigitShift[0]));  // (uniform over the list's waves)
+    if (tw == 0 && lane == 0) s_redo[slot] = usable ? 0u : 1u;
+    if (live) {  // (a workgroup of one list: uniform, so the barriers below are met by all)
         WgOffset wo;
         {
             uint32_t gt = 0u, eq = 0u;
 #pragma unroll 4
-            for (int64_t v = lane; v < w; v += 64) {
+            for (int64_t v = 64 * tw + lane; v < w; v += 64 * TW) {
                 const uint32_t hi = fhi[v], lo = flo[v];
                 gt += hi;
                 eq += lo - hi;
             }
             const uint32_t my_eq = flo[w] - fhi[w];
-            const uint32_t gt_before = (uint32_t)__shfl((int)wave_inclusive_scan(gt), 63, 64);
-            const uint32_t eq_before = (uint32_t)__shfl((int)wave_inclusive_scan(eq), 63, 64);
+            uint32_t gt_before = (uint32_t)__shfl((int)wave_inclusive_scan(gt), 63, 64);
+            uint32_t eq_before = (uint32_t)__shfl((int)wave_inclusive_scan(eq), 63, 64);
+            if constexpr (TW > 1) {
+                if (lane == 0) s_sum[2 * wave] = gt_before, s_sum[2 * wave + 1] = eq_before;
+                __syncthreads();
+                gt_before = eq_before = 0u;
+#pragma unroll
+                for (int t = 0; t < TW; ++t) gt_before += s_sum[2 * t], eq_before += s_sum[2 * t + 1];
+            }
             // (opaque: written as take = eq_before >= need ? 0 : ..., off = ... + min(need, eq_before), this
             // compiler drops the min here, in its middle end, and later lists' offsets come out too large)
             uint32_t eq_taken = min(st.need, eq_before);
@@ -2701,20 +2710,26 @@ __global__ __launch_bounds__(kBlock) void k_emit_lists(
         }
         uint32_t before = 0u;  // survivors of the earlier rounds: above T, and equal to it in the upper half
         if (usable) {
-            for (int k = 0; k * kListRound < (int)n; ++k) {
+            for (int k = 0; k * TW * kListRound < (int)n; ++k) {
                 const Round r = cur;
-                if ((k + 1) * kListRound < (int)n) cur = load_round(k + 1);
+                if ((k + 1) * TW * kListRound < (int)n) cur = load_round((k + 1) * TW + tw);
                 uint32_t m = 0u;  // bits 0..7 above T, 8..15 equal to it
 #pragma unroll
                 for (int j = 0; j < 8; ++j) {
-                    const bool in = (uint32_t)(k * kListRound + 8 * lane + j) < n;
+                    const bool in = (uint32_t)((k * TW + tw) * kListRound + 8 * lane + j) < n;
                     const uint32_t key = bf16_key(r.v.bits(j));
                     m |= in && key > T ? 1u << j : 0u;
                     m |= in && key == T ? 0x100u << j : 0u;
                 }
                 const uint32_t c = (uint32_t)__popc(m & 0xffu) | ((uint32_t)__popc(m >> 8) << 16);
-                const uint32_t incl = wave_inclusive_scan(c);
-                const uint32_t ex = before + incl - c;
+                uint32_t ex, tot;
+                if constexpr (TW > 1) {
+                    ex = before + block_exclusive_scan(c, s_wt, &tot);
+                } else {
+                    const uint32_t incl = wave_inclusive_scan(c);
+                    ex = before + incl - c;
+                    tot = (uint32_t)__shfl((int)incl, 63, 64);
+                }
                 uint32_t gb = ex & 0xffffu, eb = ex >> 16;
 #pragma unroll
                 for (int j = 0; j < 8; ++j) {
@@ -2723,14 +2738,14 @@ __global__ __launch_bounds__(kBlock) void k_emit_lists(
                     gb += is_gt;
                     eb += is_eq;
                 }
-                before += (uint32_t)__shfl((int)incl, 63, 64);
+                before += tot;
             }
-        } else if (lane == 0) {
-            s_T[wave] = T;
-            s_off[wave] = wo.off;
-            s_take[wave] = wo.take;
+        } else if (tw == 0 && lane == 0) {
+            s_T[slot] = T;
+            s_off[slot] = wo.off;
+            s_take[slot] = wo.take;
         }
-        if (census && lane == 0) {
+        if (census && tw == 0 && lane == 0) {
             uint32_t *bstart = census + (int64_t)kCensusCopies * cfeat;
             if (row0 % kCensusRows == 0) bstart[row0 / kCensusRows] = wo.off;
             if (list == 0) bstart[(g.rows + kCensusRows - 1) / kCensusRows] = n_entries;
@@ -3433,8 +3448,8 @@ int launch_typed(const StacrSaveArgs &a, const Plan &p, char *ws, const size_t *
     WgCount *counts = carve<WgCount>(ws, off[WS_COUNTS]);
     const bool resid = a.k_total > 0;
     const int nwg = (int)p.n_wgs;
-    const bool few_refine = p.n_wgs <= kFewRefine, few_emit = p.n_wgs <= kFewEmit;
-    auto list_wgs = [&](bool few) { return (unsigned)(few ? p.n_wgs : (p.n_wgs + kListWaves - 1) / kListWaves); };
+    const bool few = p.n_wgs <= kFewLists;
+    const unsigned n_list_wgs = (unsigned)(few ? p.n_wgs : (p.n_wgs + kListWaves - 1) / kListWaves);
 
     // padded basis; histograms and max key (contiguous in the layout) cleared in the same launch
     const int64_t n_zero = resid ? (int64_t)((off[WS_MAXKEY] + (size_t)p.g.hcopies * kMaxKeyStride * sizeof(uint32_t) -
@@ -3526,8 +3541,8 @@ int launch_typed(const StacrSaveArgs &a, const Plan &p, char *ws, const size_t *
                 auto refine_cand = [&](auto hc) {
                     if constexpr (kCandOk)
                         stacr_launch("k_refine_lists", s, [&] {
-                            const auto k = few_refine ? k_refine_lists<decltype(hc)::value, 1> : k_refine_lists<decltype(hc)::value, kListWaves>;
-                            k<<<list_wgs(few_refine), kBlock, 0, s>>>(p.g, p.Rq, p.n_wgs, x, qp, coeff, hist, state, kf, kl,
+                            const auto k = few ? k_refine_lists<decltype(hc)::value, 1> : k_refine_lists<decltype(hc)::value, kListWaves>;
+                            k<<<n_list_wgs, kBlock, 0, s>>>(p.g, p.Rq, p.n_wgs, x, qp, coeff, hist, state, kf, kl,
                                                                                maxkey, fold, coarse, p.list_cap, cidx, cval, cmeta);
                         });
                 };
@@ -3581,8 +3596,8 @@ int launch_typed(const StacrSaveArgs &a, const Plan &p, char *ws, const size_t *
             const uint32_t kt = (uint32_t)a.k_sum;  // the entries emitted (no trim: the chunks' k summed)
             auto emit = [&](auto hc) {
                 stacr_launch("k_emit_lists", s, [&] {
-                    const auto k = few_emit ? k_emit_lists<decltype(hc)::value, 1> : k_emit_lists<decltype(hc)::value, kListWaves>;
-                    k<<<list_wgs(few_emit), kBlock, 0, s>>>(p.g, p.Rq, p.n_wgs, x, qp, coeff, state, kf, maxkey, o, a.scale,
+                    const auto k = few ? k_emit_lists<decltype(hc)::value, 1> : k_emit_lists<decltype(hc)::value, kListWaves>;
+                    k<<<n_list_wgs, kBlock, 0, s>>>(p.g, p.Rq, p.n_wgs, x, qp, coeff, state, kf, maxkey, o, a.scale,
                                                                         p.trim ? 1 : 0, hist, fold, p.list_cap, cidx, cval, cmeta, cen, kt);
                 });
             };

@@ -1083,3 +1083,15 @@ def test_a_fitted_basis_keeps_the_list_passes_fast(dev, rows, d, rank):
     fitted = _list_passes_us(xd, v[:, -rank:].contiguous().to(dev, torch.bfloat16))
     random = _list_passes_us(xd, make_basis(d, rank).to(dev, torch.bfloat16))
     assert fitted <= 2.3 * random, f"{fitted:.1f} us with a fitted basis, {random:.1f} us with a random one"
+
+
+@pytest.mark.parametrize("rows,d,rank,budget", [
+    (300, 4096, 8, 0.009),     # a workgroup a list, lists past its 2048 candidates a round
+    (4100, 2048, 16, 0.01),    # four lists a workgroup, lists past a wave's 512
+    (8192, 2048, 8, 0.005), (8200, 2048, 8, 0.005),  # 1024 and 1025 lists: the last with their own workgroup, and past it
+])
+def test_save_long_lists_match_oracle(dev, rows, d, rank, budget):
+    announce("save long lists", rows, d, rank, budget)
+    xd = make_activation(rows, d).to(dev, torch.bfloat16)
+    assert "k_emit_lists" in _check_save_against_oracle(xd, make_basis(d, rank).to(dev, torch.bfloat16), "global_topk",
+                                                        budget, 512, 8)

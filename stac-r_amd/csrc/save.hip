@@ -2319,6 +2319,8 @@ struct CandVals {
 // 16 x 1024: emission 13 -> 10.5 us; 2048 lists of 4 x 1024: 15.3 us, 22.2 at a workgroup a list).
 constexpr int kListWaves = 4;          // lists of a workgroup
 constexpr int kFewLists = 1024;
+constexpr int kListGroup = kBlock;     // lists of a group, and
+constexpr int kGroupedLists = 4096;    // the lists of a chunk past which their records are summed by groups first
 constexpr int kListRound = 64 * 8;     // candidates a wave reads at once
 constexpr int kListC = 256;            // coefficients of a list's rows, padded: 64 x the row slots of a workgroup (at most 4)
 
@@ -2595,6 +2597,32 @@ __global__ __launch_bounds__(kBlock) void k_refine_lists(SaveGeom g, int R, int6
     if (mine16) atomicAdd(&hist[((chunk * 3 + 1) * HC + (int)(list % HC)) * kBins + (lane << 7)], mine16);
 }
 
+// The lists' records summed by groups of kListGroup (one workgroup a group), for the emission of chunks with more
+// than kGroupedLists lists: there every list would sum all earlier ones' itself, the square of the lists in all.
+// (Global top-k, save with and without: 32768 lists of 4 x 512 474 and 576 us, 8192 of 4 x 2048 175 and 180, 4096 of
+// 32 x 512 137 and 137, 2048 of 4 x 1024 56 and 54.)
+template <int HC>
+__global__ __launch_bounds__(kBlock) void k_list_groups(SaveGeom g, int64_t n_lists, int64_t groups,
+                                                        const SelState *__restrict__ state,
+                                                        const uint32_t *__restrict__ hist,
+                                                        const uint32_t *__restrict__ fold, WgCount *__restrict__ group_sums)
+{
+    __shared__ uint32_t s_wt[kWaves];
+    const int64_t chunk = blockIdx.x / groups, v = (blockIdx.x % groups) * kListGroup + threadIdx.x;
+    uint32_t hw[HC];
+    const uint32_t *h1 = hist + (chunk * 3 + 1) * HC * kBins + ((threadIdx.x & 15) << 7);
+#pragma unroll
+    for (int c = 0; c < HC; ++c) hw[c] = h1[c * kBins];
+    SelState sel1;
+    const SelState st = fold_select<HC>(hw, state[chunk * 3 + 0], &sel1);
+    const uint32_t b1 = (st.prefix >> 16) & 15u;
+    const uint32_t *flo = fold + (int64_t)b1 * n_lists + chunk * g.wgs_per_chunk, *fhi = flo + n_lists;
+    uint32_t hi = 0u, lo = 0u;
+    if (v < g.wgs_per_chunk) hi = fhi[v], lo = flo[v];
+    const uint32_t gt = block_sum(hi, s_wt), eq = block_sum(lo - hi, s_wt);
+    if (threadIdx.x == 0) group_sums[blockIdx.x] = WgCount{gt, eq};
+}
+
 // Emission: the final selection and the list's offset and tie budget (the earlier lists' records), then its
 // survivors quantized and written in ascending flat order.  With a census the workgroup counts its lists' entries
 // per feature in LDS first: two 16-bit counts a word (features f and f + 2048; a feature has at most one entry
@@ -2604,8 +2632,8 @@ __global__ __launch_bounds__(kBlock) void k_emit_lists(
     SaveGeom g, int R, int64_t n_lists, const uint16_t *__restrict__ x, const float *__restrict__ qp,
     const uint16_t *__restrict__ coeff, SelState *__restrict__ state, uint32_t chunk_k,
     const uint32_t *__restrict__ maxkey, OutSpec o, float *scale_out, int to_list, const uint32_t *__restrict__ hist,
-    const uint32_t *__restrict__ fold, uint32_t cap, const uint32_t *__restrict__ cand_idx,
-    const uint16_t *__restrict__ cand_val, const CandMeta *__restrict__ meta, uint32_t *__restrict__ census,
+    const uint32_t *__restrict__ fold, const WgCount *__restrict__ group_sums, int64_t groups, uint32_t cap,
+    const uint32_t *__restrict__ cand_idx, const uint16_t *__restrict__ cand_val, const CandMeta *__restrict__ meta, uint32_t *__restrict__ census,
     uint32_t n_entries)
 {
     constexpr int DT = STACR_DTYPE_BF16;
@@ -2686,8 +2714,18 @@ __global__ __launch_bounds__(kBlock) void k_emit_lists(
         WgOffset wo;
         {
             uint32_t gt = 0u, eq = 0u;
+            int64_t first = 0;
+            if (LW > 1 && groups) {  // (uniform) the groups before this list's
+                const int64_t before = w / kListGroup;
+                first = before * kListGroup;
+                for (int64_t v = lane; v < before; v += 64) {
+                    const WgCount c = group_sums[chunk * groups + v];
+                    gt += c.gt;
+                    eq += c.eq;
+                }
+            }
 #pragma unroll 4
-            for (int64_t v = 64 * tw + lane; v < w; v += 64 * TW) {
+            for (int64_t v = first + 64 * tw + lane; v < w; v += 64 * TW) {
                 const uint32_t hi = fhi[v], lo = flo[v];
                 gt += hi;
                 eq += lo - hi;
@@ -3321,10 +3359,16 @@ Plan make_plan(const StacrSaveArgs &a)
     return p;
 }
 
+// Groups of lists a chunk (0: its lists are few enough that each sums the earlier ones' records).
+int64_t list_groups(const Plan &p)
+{
+    return p.cand && p.g.wgs_per_chunk > kGroupedLists ? (p.g.wgs_per_chunk + kListGroup - 1) / kListGroup : 0;
+}
+
 template <typename T> T *carve(char *base, size_t off) { return reinterpret_cast<T *>(base + off); }
 
 enum { WS_QP, WS_HIST, WS_COARSE, WS_STATE, WS_MAXKEY, WS_COUNTS, WS_OFFS, WS_LRBITS, WS_LIDX, WS_THIST, WS_TSTATE,
-       WS_LCOUNTS, WS_LOFFS, WS_Q4, WS_FOLD, WS_R, WS_CIDX, WS_CVAL, WS_CMETA, WS_N };
+       WS_LCOUNTS, WS_LOFFS, WS_Q4, WS_FOLD, WS_GROUPS, WS_R, WS_CIDX, WS_CVAL, WS_CMETA, WS_N };
 
 size_t layout(const StacrSaveArgs &a, const Plan &p, size_t *off)
 {
@@ -3347,6 +3391,7 @@ size_t layout(const StacrSaveArgs &a, const Plan &p, size_t *off)
     take(WS_LOFFS, nb * sizeof(WgOffset));
     take(WS_Q4, a.bits == 4 ? (size_t)a.k_total : 0);
     take(WS_FOLD, p.fold ? (size_t)17 * p.n_wgs * sizeof(uint32_t) : 0);  // cum[0..16][workgroup]
+    take(WS_GROUPS, (size_t)list_groups(p) * p.g.n_chunks * sizeof(WgCount));
     const bool rstore = p.fast && a.dtype != STACR_DTYPE_F32 && a.k_total > 0 && !p.cand;  // (wide rows: p.fast)
     take(WS_R, rstore ? (size_t)a.rows * a.feats * 2 : 0);  // the stored residual (16-bit types)
     const bool lists = p.cand || p.cand_rin;
@@ -3595,10 +3640,17 @@ int launch_typed(const StacrSaveArgs &a, const Plan &p, char *ws, const size_t *
             uint32_t *cen = census ? a.census : nullptr;
             const uint32_t kt = (uint32_t)a.k_sum;  // the entries emitted (no trim: the chunks' k summed)
             auto emit = [&](auto hc) {
+                const int64_t groups = list_groups(p);
+                WgCount *gsums = carve<WgCount>(ws, off[WS_GROUPS]);
+                if (groups)
+                    stacr_launch("k_list_groups", s, [&] {
+                        k_list_groups<decltype(hc)::value><<<(unsigned)(groups * p.g.n_chunks), kBlock, 0, s>>>(p.g, p.n_wgs, groups, state,
+                                                                                                             hist, fold, gsums);
+                    });
                 stacr_launch("k_emit_lists", s, [&] {
                     const auto k = few ? k_emit_lists<decltype(hc)::value, 1> : k_emit_lists<decltype(hc)::value, kListWaves>;
                     k<<<n_list_wgs, kBlock, 0, s>>>(p.g, p.Rq, p.n_wgs, x, qp, coeff, state, kf, maxkey, o, a.scale,
-                                                                        p.trim ? 1 : 0, hist, fold, p.list_cap, cidx, cval, cmeta, cen, kt);
+                                                                        p.trim ? 1 : 0, hist, fold, gsums, groups, p.list_cap, cidx, cval, cmeta, cen, kt);
                 });
             };
             auto emit_rin = [&](auto hc) {

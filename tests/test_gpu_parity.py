@@ -1095,3 +1095,42 @@ def test_save_long_lists_match_oracle(dev, rows, d, rank, budget):
     xd = make_activation(rows, d).to(dev, torch.bfloat16)
     assert "k_emit_lists" in _check_save_against_oracle(xd, make_basis(d, rank).to(dev, torch.bfloat16), "global_topk",
                                                         budget, 512, 8)
+
+
+@pytest.mark.parametrize("rows,d,rank,mode,chunk,kind", [
+    (16700, 264, 16, "global_topk", 512, "plain"),      # 4175 lists: 17 groups of their records, the last partly filled
+    (16700, 264, 16, "global_topk", 512, "ties"),       # the threshold's ties run out in a later group
+    (33000, 264, 16, "chunk_topk", 16400, "plain"),     # 4100 lists a chunk, a last chunk of 50 and empty groups
+])
+def test_save_grouped_list_records_match_oracle(dev, rows, d, rank, mode, chunk, kind):
+    from stacr_amd import kernels
+
+    announce("save grouped records", rows, d, rank, mode, chunk, kind)
+    x, q = make_activation(rows, d), make_basis(d, rank)
+    if kind == "ties":
+        q.zero_()
+        x = 0.01 * x
+        x[::3, ::40] = torch.where(x[::3, ::40] < 0, -1.0, 1.0)  # 39 k equal entries, k of 22 k
+    xd, qd = x.to(dev, torch.bfloat16), q.to(dev, torch.bfloat16)
+    assert "k_list_groups" in _check_save_against_oracle(xd, qd, mode, 0.005, chunk, 8)
+    if kind == "plain" and mode == "global_topk":
+        _, idx, _, _, census = kernels.save_with_census(xd, qd, mode=mode, budget=0.005, chunk_rows=chunk, bits=8)
+        cen = census.cpu().numpy().view(np.uint32).astype(np.int64)
+        pos = idx.cpu().numpy().astype(np.int64)
+        assert np.array_equal(cen[: 8 * d].reshape(8, d).sum(0), np.bincount(pos % d, minlength=d))
+        assert np.array_equal(cen[8 * d:], np.searchsorted(pos, np.minimum(np.arange(cen.size - 8 * d) * 512, rows) * d))
+
+
+def test_emission_of_many_lists_stays_a_small_part_of_the_save(dev):
+    """Each list's offset is a sum over the lists before it: with 32768 lists that had grown to half the
+    projection pass's time."""
+    from stacr_amd import _lib, kernels
+
+    announce("emission of many lists")
+    xd = make_activation(4096, 512).to(dev, torch.bfloat16).repeat(32, 1)
+    qd = make_basis(512, 16).to(dev, torch.bfloat16)
+    with _lib.KernelTimer(max_launches=256) as timer:
+        for _ in range(6):
+            kernels.save(xd, qd, mode="global_topk", budget=0.005, chunk_rows=512, bits=8)
+        torch.cuda.synchronize()
+    assert timer.results["k_emit_lists"][0] <= 0.3 * timer.results["k_proj_cand_w"][0]

@@ -3320,8 +3320,9 @@ Plan make_plan_base(const StacrSaveArgs &a)
     if (p.wide) quota *= 1.5;
     if (quota > (p.wide ? kListMax : kCandCap) / 2) return p;
     double cap = hmin<double>(4.0 * quota, p.wide ? kListMax : kCandCap);
-    if (p.wide) {  // the stored residual and the lists of the level-1 pass, a workgroup
-        const double stored = (double)a.rows * (double)a.feats * 2.0 + (double)p.n_wgs * kCandCap * kCandBytes;
+    // what the stored residual and the lists of the level-1 pass would take
+    const double stored = (double)a.rows * (double)a.feats * 2.0 + (double)p.n_wgs * kCandCap * kCandBytes;
+    if (p.wide) {
         cap = hmin<double>(cap, stored / ((double)p.n_wgs_w * kCandBytes));
         if (cap < 2.0 * quota) return p;
     }
@@ -3331,7 +3332,14 @@ Plan make_plan_base(const StacrSaveArgs &a)
     p.quota = (uint32_t)quota;
     if (p.wide) {
         p.wcand = true;
-        p.gw.hcopies = p.gw.wgs_per_chunk >= 256 ? kHistCopies : 1;
+        // Histogram copies where many workgroups add to one chunk's.  From 128 a chunk on they take a fifth off the
+        // projection, but cost the later passes a little a list, and scratch a chunk: only for few lists, within
+        // what the lists leave of `stored` (chunks of 512 rows, rank 16, save: 8192 x 1024 59 -> 52 us,
+        // 131072 x 1024 521 -> 532, which stays without).
+        const double copies = (double)p.gw.n_chunks * 3.0 * (kHistCopies - 1) * kBins * sizeof(uint32_t);
+        const bool few_many = p.gw.wgs_per_chunk >= 128 && p.n_wgs_w <= 4096 &&
+                              (double)p.n_wgs_w * p.list_cap * kCandBytes + copies <= stored;
+        p.gw.hcopies = p.gw.wgs_per_chunk >= 256 || few_many ? kHistCopies : 1;
         p.g = p.gw;
         p.n_wgs = p.n_wgs_w;
     }

@@ -1134,3 +1134,23 @@ def test_emission_of_many_lists_stays_a_small_part_of_the_save(dev):
             kernels.save(xd, qd, mode="global_topk", budget=0.005, chunk_rows=512, bits=8)
         torch.cuda.synchronize()
     assert timer.results["k_emit_lists"][0] <= 0.3 * timer.results["k_proj_cand_w"][0]
+
+
+def test_chunks_of_many_workgroups_do_not_slow_the_wide_projection(dev):
+    """128 workgroups a chunk that add to one histogram made the projection a quarter longer than 2048 workgroups
+    that add to eight copies."""
+    from stacr_amd import _lib, kernels
+
+    announce("wide projection in chunks")
+    xd = make_activation(8192, 1024).to(dev, torch.bfloat16)
+    qd = make_basis(1024, 16).to(dev, torch.bfloat16)
+    us = {}
+    for mode in ("global_topk", "chunk_topk"):
+        us[mode] = float("inf")
+        for _ in range(5):
+            with _lib.KernelTimer(max_launches=256) as timer:
+                for _ in range(6):
+                    kernels.save(xd, qd, mode=mode, budget=0.005, chunk_rows=512, bits=8)
+                torch.cuda.synchronize()
+            us[mode] = min(us[mode], timer.results["k_proj_cand_w"][0] / 6 * 1e3)
+    assert us["chunk_topk"] <= 1.15 * us["global_topk"], us

@@ -271,6 +271,18 @@ __global__ __launch_bounds__(kBlock) void k_select_step(int lvl, const uint32_t 
     chunk_select(lvl, hist, state, blockIdx.x, n_chunks, k_full, k_last, true, s_tot, &s_res);
 }
 
+// An output offset and tie budget from the keys above (gt_before) and equal to (eq_before) the threshold in what
+// comes earlier in the chunk: ties go first come, `need` of them in all.  (The earlier ties that are taken first,
+// then what they leave.  Written as eq_before >= need ? 0 : min(mine, need - eq_before) for the budget and
+// min(need, eq_before) in the offset, the compiler speculates the difference as one that cannot wrap, its
+// constraint elimination takes that for a fact, and in straight-line code drops the min of the offset.)
+__device__ __forceinline__ WgOffset tie_offset(uint32_t need, uint32_t gt_before, uint32_t eq_before, uint32_t mine_eq,
+                                               uint32_t base)
+{
+    const uint32_t taken = min(need, eq_before);
+    return WgOffset{base + gt_before + taken, min(mine_eq, need - taken)};
+}
+
 // A workgroup's output offset and tie budget: its chunk's earlier workgroups in order, ties handed
 // out first come (the per-workgroup form of k_offsets).
 __device__ WgOffset wg_offset(const WgCount *__restrict__ counts, int64_t chunk, int64_t w, int64_t wgs_per_chunk,
@@ -285,8 +297,7 @@ __device__ WgOffset wg_offset(const WgCount *__restrict__ counts, int64_t chunk,
     const uint32_t gt_before = block_sum(gt, s_tot);
     const uint32_t eq_before = block_sum(eq, s_tot);
     const WgCount mine = counts[chunk * wgs_per_chunk + w];
-    const uint32_t take = eq_before >= need_eq ? 0u : min(mine.eq, need_eq - eq_before);
-    return WgOffset{(uint32_t)chunk * chunk_k + gt_before + min(need_eq, eq_before), take};
+    return tie_offset(need_eq, gt_before, eq_before, mine.eq, (uint32_t)chunk * chunk_k);
 }
 
 // Pass 1: coefficients, first-digit histogram, max key.
@@ -477,7 +488,7 @@ __global__ __launch_bounds__(kBlock) void k_offsets(const WgCount *__restrict__ 
         const WgCount c = w < wgs_per_chunk ? counts[chunk * wgs_per_chunk + w] : WgCount{0u, 0u};
         uint32_t tot_eq, tot_sel;
         const uint32_t eq_before = carry_eq + block_exclusive_scan(c.eq, s_tot, &tot_eq);
-        const uint32_t take = eq_before >= need_eq ? 0u : min(c.eq, need_eq - eq_before);
+        const uint32_t take = tie_offset(need_eq, 0u, eq_before, c.eq, 0u).take;
         const uint32_t sel = c.gt + take;
         const uint32_t sel_before = carry_sel + block_exclusive_scan(sel, s_tot, &tot_sel);
         if (w < wgs_per_chunk) offs[chunk * wgs_per_chunk + w] = WgOffset{base + sel_before, take};
@@ -1628,9 +1639,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
         const uint32_t gt_before = block_sum(gt, s_off);
         const uint32_t eq_before = block_sum(eq, s_off);
         const WgCount mine = kFold ? WgCount{fhi[w], flo[w] - fhi[w]} : counts[wg0 + w];
-        const uint32_t take = eq_before >= st.need ? 0u : min(mine.eq, st.need - eq_before);
-        wo = WgOffset{(uint32_t)chunk * chunk_k + gt_before + min(st.need, eq_before), take};
-        n_out = mine.gt + take;
+        wo = tie_offset(st.need, gt_before, eq_before, mine.eq, (uint32_t)chunk * chunk_k);
+        n_out = mine.gt + wo.take;
     }
     const bool staged = n_out <= (uint32_t)kEmitStage;  // uniform
     uint32_t cnt[NB], incl[NB];
@@ -2740,11 +2750,7 @@ __global__ __launch_bounds__(kBlock) void k_emit_lists(
 #pragma unroll
                 for (int t = 0; t < TW; ++t) gt_before += s_sum[2 * t], eq_before += s_sum[2 * t + 1];
             }
-            // (opaque: written as take = eq_before >= need ? 0 : ..., off = ... + min(need, eq_before), this
-            // compiler drops the min here, in its middle end, and later lists' offsets come out too large)
-            uint32_t eq_taken = min(st.need, eq_before);
-            asm volatile("" : "+v"(eq_taken));
-            wo = WgOffset{(uint32_t)chunk * chunk_k + gt_before + eq_taken, min(my_eq, st.need - eq_taken)};
+            wo = tie_offset(st.need, gt_before, eq_before, my_eq, (uint32_t)chunk * chunk_k);
         }
         uint32_t before = 0u;  // survivors of the earlier rounds: above T, and equal to it in the upper half
         if (usable) {
@@ -2968,8 +2974,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
         const uint32_t gt_before = block_sum(gt, s_off);
         const uint32_t eq_before = block_sum(eq, s_off);
         const uint32_t my_eq = flo[w] - fhi[w];
-        const uint32_t take = eq_before >= st.need ? 0u : min(my_eq, st.need - eq_before);
-        wo = WgOffset{(uint32_t)chunk * chunk_k + gt_before + min(st.need, eq_before), take};
+        wo = tie_offset(st.need, gt_before, eq_before, my_eq, (uint32_t)chunk * chunk_k);
     }
     auto put = [&](uint32_t pos, uint32_t fl, float rv) {
         if (pos >= o.cap) {

@@ -982,13 +982,14 @@ def test_weight_grad_wide_tiles_at_their_edges(dev, rows, d_in, d_out, rank, dty
 
 
 def _check_save_against_oracle(xd, qd, mode, budget, chunk, bits, coeff=None):
-    """One bf16 save, its entries bit for bit against the oracle on the kernel's own coefficients; the
+    """One save, its entries bit for bit against the oracle on the kernel's own coefficients; the
     names of the kernels that ran."""
     from stacr_amd import kernels
 
     with _kernel_names() as names:
         c, idx, data, scale = kernels.save(xd, qd, mode=mode, budget=budget, chunk_rows=chunk, bits=bits, coeff=coeff)
-    _, oidx, odata, oscale = orc.save(_np(xd), _np(qd), "bf16", mode, budget, chunk, bits, coeff=_np(c))
+    dtype = next(k for k, v in DT.items() if v == xd.dtype)
+    _, oidx, odata, oscale = orc.save(_np(xd), _np(qd), dtype, mode, budget, chunk, bits, coeff=_np(c))
     assert np.array_equal(idx.cpu().numpy().astype(np.int64), oidx)
     if bits == 0:
         assert np.array_equal(_np(data), odata)
@@ -1154,3 +1155,25 @@ def test_chunks_of_many_workgroups_do_not_slow_the_wide_projection(dev):
                 torch.cuda.synchronize()
             us[mode] = min(us[mode], timer.results["k_proj_cand_w"][0] / 6 * 1e3)
     assert us["chunk_topk"] <= 1.15 * us["global_topk"], us
+
+
+@pytest.mark.parametrize("kernel,rows,d,rank,dtype,mode,budget,chunk", [
+    ("k_emit_lists", 2048, 1024, 8, "bf16", "global_topk", 0.004, 512),    # a workgroup a list
+    ("k_emit_lists", 5000, 264, 16, "bf16", "global_topk", 0.004, 512),    # four lists a workgroup
+    ("k_emit_cand", 1024, 1024, 8, "bf16", "global_topk", 0.02, 512),
+    ("k_emit_b", 1024, 1024, 8, "f16", "chunk_topk", 0.004, 256),
+    ("k_emit", 900, 30, 4, "f32", "global_topk", 0.02, 512),
+    ("k_list_emit", 1000, 1024, 8, "bf16", "chunk_topk", 0.0041, 100),     # trimmed: the list's own ties
+])
+def test_ties_run_out_between_workgroups(dev, kernel, rows, d, rank, dtype, mode, budget, chunk):
+    """More entries equal to the threshold than are taken, spread over all rows: the workgroups up to the one
+    where they run out take ties, the later ones none, and the entries above follow both."""
+    announce("ties run out", kernel, rows, d, dtype, mode)
+    g = torch.Generator().manual_seed(11)
+    x = 0.01 * torch.randn(rows, d, generator=g)
+    u = torch.rand(rows, d, generator=g)
+    x[u < 2 * budget] = 1.0
+    x[u < 0.25 * budget] = 3.0
+    x = torch.where(torch.rand(rows, d, generator=g) < 0.5, -x, x)
+    names = _check_save_against_oracle(x.to(dev, DT[dtype]), torch.zeros(d, rank).to(dev, DT[dtype]), mode, budget, chunk, 8)
+    assert kernel in names

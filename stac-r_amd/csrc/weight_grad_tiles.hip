@@ -1573,6 +1573,10 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4))
 #pragma unroll
             for (int h = 0; h < L::per_wave; ++h) issue_g(blk + 1, h, B2);
         }
+        // The wait at the end counts on the order of the copies and the record loads after them: no load may
+        // move up past this, nor down past the wait.
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
         // one chunk: A = the G rows of slots k1 (.. + 3 over the group) and k1 + 4, per 16 outputs;
         // B = the values at (feature in the tile, slot) of the zeroed scratch, cleared again after the
         // read; one product per 16 outputs.  Every lane stores unconditionally: a lane past the tile's
@@ -1634,7 +1638,10 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4))
                 __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
             }
         }
-        // the copies have landed: the eight record loads above are younger
+        // the copies have landed: the eight record loads above are younger (kept so by the two statements after
+        // the copies and the two here; a test counts them in the compiled code)
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
         __builtin_amdgcn_s_waitcnt(0x0078);  // vmcnt(8) lgkmcnt(0)
         return x;
     };

@@ -180,6 +180,29 @@ def test_adaptive_save_y_matches_oracle(name, rows, d, qc, r):
     np.testing.assert_allclose(e[3:3 + r], per_rank, rtol=1e-5, atol=1e-7)
 
 
+@pytest.mark.parametrize("rows,d,qc,r", [(1024, 1024, 16, 5), (600, 8192, 16, 9), (4200, 264, 12, 3)])
+@pytest.mark.parametrize("heavy", ["rows_apart", "rows_together"])
+def test_adaptive_save_y_recomputes_lists_without_the_columns_past_the_rank(heavy, rows, d, qc, r):
+    """Rows far above the others leave candidate lists that the later passes recompute from X and C: with Y
+    asked for, the padded basis holds q_cols columns, of which the residual takes the first `rank` only."""
+    from stacr_amd import adaptive as ad
+
+    dev = _dev()
+    print(f"CASE save_y recomputed {heavy} {rows} {d} {qc} {r}", flush=True)
+    x = make_activation(rows, d)
+    if heavy == "rows_apart":
+        x[33::100] *= 300.0
+    else:
+        x[32:48] *= 1000.0
+    x, q = x.to(torch.bfloat16), make_basis(d, qc).to(torch.bfloat16)
+    coeff, idx, values, _, y = ad.save_y(x.to(dev), q.to(dev), r, 0.005, 512)
+    assert y is not None and torch.equal(coeff.cpu(), y[:, :r].cpu().to(torch.bfloat16))
+    _, idx_ref, val_ref = orc.adaptive_save(x.float().numpy(), q.float().numpy()[:, :r], "bf16", 0.005, 512,
+                                            coeff=coeff.float().cpu().numpy())
+    assert np.array_equal(idx.cpu().numpy().astype(np.int64), idx_ref.astype(np.int64))
+    assert np.array_equal(values.float().cpu().numpy(), val_ref)
+
+
 # ---------------------------------------------------------------- the adaptive Function
 FUNC_CONFIGS = [
     dict(residual_mode="topk", residual_budget=0.005, quantize_coefficients=True, quantize_residuals=True,

@@ -202,11 +202,17 @@ def _crafted_activation(kind, rows, d):
     ("tie_block", 512, 1024, "global_topk", 0.005, 512, 0),
     ("tie_block", 1024, 1024, "chunk_topk", 0.01, 128, 8),
     ("outlier_scattered", 4096, 1024, "global_topk", 0.005, 512, 8),
-    # wide rows (the level-1 pass writes the lists from the stored residual; overflowing lists
-    # fall back to the stored residual)
+    # wide rows
     ("tie_block", 512, 4096, "global_topk", 0.005, 512, 0),
     ("outlier_rows", 1024, 4096, "chunk_topk", 0.005, 256, 8),
     ("outlier_scattered", 2048, 4096, "global_topk", 0.005, 512, 8),
+    # a quota past the projection pass's lists: the level-1 pass writes the lists from the stored residual, and
+    # overflowing ones fall back to it
+    ("tie_block", 512, 1024, "global_topk", 0.02, 512, 0),
+    ("outlier_rows", 1024, 1024, "chunk_topk", 0.02, 256, 8),
+    ("tie_block", 512, 4096, "global_topk", 0.02, 512, 8),
+    ("outlier_rows", 1024, 8192, "global_topk", 0.005, 512, 8),
+    ("outlier_scattered", 600, 8192, "chunk_topk", 0.005, 200, 0),
 ])
 def test_save_candidate_fallback_matches_oracle(dev, kind, rows, d, mode, budget, chunk, bits):
     """bf16 saves keep per-workgroup candidate lists (kept by the projection pass, or by the level-1
@@ -220,8 +226,10 @@ def test_save_candidate_fallback_matches_oracle(dev, kind, rows, d, mode, budget
     x = _crafted_activation(kind, rows, d)
     q = torch.zeros(d, rank) if kind == "tie_block" else make_basis(d, rank)
     xd, qd = x.to(dev, torch.bfloat16), q.to(dev, torch.bfloat16)
-    coeff, idx, data, scale = kernels.save(xd, qd, mode=mode, budget=budget, chunk_rows=chunk, bits=bits)
-    torch.cuda.synchronize()
+    with _kernel_names() as names:
+        coeff, idx, data, scale = kernels.save(xd, qd, mode=mode, budget=budget, chunk_rows=chunk, bits=bits)
+    stored = budget > 0.01 or d == 8192
+    assert ("k_emit_cand" if stored else "k_emit_lists") in names
     xf, qf, cf = _np(xd), _np(qd), _np(coeff)
     _, oidx, odata, oscale = orc.save(xf, qf, "bf16", mode, budget, chunk, bits, coeff=cf)
     assert np.array_equal(idx.cpu().numpy().astype(np.int64), oidx)
@@ -1177,3 +1185,42 @@ def test_ties_run_out_between_workgroups(dev, kernel, rows, d, rank, dtype, mode
     x = torch.where(torch.rand(rows, d, generator=g) < 0.5, -x, x)
     names = _check_save_against_oracle(x.to(dev, DT[dtype]), torch.zeros(d, rank).to(dev, DT[dtype]), mode, budget, chunk, 8)
     assert kernel in names
+
+
+@pytest.mark.parametrize("rows,d,rank", [(96, 1024, 16), (96, 2064, 8), (64, 4096, 13), (40, 8192, 16)])
+@pytest.mark.parametrize("values", ["subnormal", "infinite", "nan"])
+def test_residual_chain_is_the_same_on_the_matrix_cores_and_off_them(dev, values, rows, d, rank):
+    """The wide projection forms sum_j c_j q_j on v_mfma_f32_4x4x1, a recomputed list and the per-row kernels by
+    fmaf: the same bits, also for subnormal, infinite and NaN operands.  An activation off the 16-byte
+    alignment takes the per-row kernels; a few heavy rows make lists that are recomputed."""
+    from stacr_amd import kernels
+
+    announce("residual chain", values, rows, d, rank)
+    g = torch.Generator().manual_seed(23)
+    x = torch.randn(rows, d, generator=g)
+    q = make_basis(d, rank)
+    c = torch.randn(rows, rank, generator=g)
+    x[5::16] *= 300.0
+    if values == "subnormal":  # bf16 values, products and sums below 2^-126
+        x, c = x * 2.0**-128, c * 2.0**-118
+        q = q * 2.0**-8
+    else:
+        c[1, rank - 1] = c[rows - 3, 0] = float("inf") if values == "infinite" else float("nan")
+        q[d // 3, 2] = -float("inf") if values == "infinite" else float("nan")
+        x[7, 9] = float("inf")
+    xd, qd, cd = (t.to(dev, torch.bfloat16) for t in (x, q, c))
+    off = torch.empty(rows * d + 1, dtype=torch.bfloat16, device=dev)[1:].view(rows, d)
+    off.copy_(xd)
+    out = []
+    for a in (xd, off):
+        with _kernel_names() as names:
+            _, idx, data, _ = kernels.save(a, qd, mode="global_topk", budget=0.005, chunk_rows=512, bits=0, coeff=cd)
+        out.append((idx.cpu(), data.cpu().view(torch.int16), names))
+    assert "k_emit_lists" in out[0][2] and "k_emit" in out[1][2]
+    assert torch.equal(out[0][0], out[1][0])
+    a, b = out[0][1], out[1][1]
+    if values == "nan":  # (a NaN's sign is the conversion's own)
+        nan = (a & 0x7fff) > 0x7f80
+        assert torch.equal(nan, (b & 0x7fff) > 0x7f80)
+        a, b = a.masked_fill(nan, 0), b.masked_fill(nan, 0)
+    assert torch.equal(a, b)

@@ -1718,9 +1718,9 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
 // its share of the chunk's k), in ascending flat order, with their residuals; the residual is not
 // stored.  The chunk's level-0 bin B0 is known after the pass.  A workgroup whose cut is at or
 // below B0, and whose candidates fit its list, holds every element of bin B0 and above among its
-// candidates, so the level-1 pass and the emission work on those lists; any other workgroup
-// recomputes its residuals from X, C and the basis there (the same values, rarely needed).  The
-// selection is the same as the full passes'.
+// candidates, so the level-1 pass and the emission work on those lists; the residuals of any other
+// workgroup are recomputed from X, C and the basis (the same values).  The selection is the same as
+// the full passes'.
 
 __device__ __forceinline__ uint32_t bf16_key(uint32_t bits16)
 {
@@ -2908,7 +2908,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
     __shared__ uint32_t s_off[kWaves];
     __shared__ uint32_t s_wt[kWaves];
     // with a census: this workgroup's entries per feature of the layer, two 16-bit counts a word
-    // (features f and f + 2048; a workgroup emits at most kCandCap entries, so no half overflows):
+    // (features f and f + 2048; a feature has at most one entry a row, so no half overflows):
     // census_feats <= 4096
     __shared__ uint32_t s_feat[kBins];
     int64_t chunk, row0, row_end;
@@ -3192,13 +3192,13 @@ struct Plan {
     // (bf16 wide rows with a residual and a quota inside the list) the projection pass keeps the lists
     // (k_proj_cand_w): no stored residual, and g is the projection pass's geometry
     bool wcand;
-    // bf16 on the batched path with a residual and not wide: the candidate passes (k_proj_cand,
-    // k_refine_cand, k_emit_cand) with the workgroups' quota
+    // bf16 on the batched path or wide, with a residual and a quota inside the list: the projection pass keeps
+    // the lists (k_proj_cand, or k_proj_cand_w with wcand), read by k_refine_lists and k_emit_lists
     bool cand;
     uint32_t quota;
     uint32_t list_cap;  // candidates a list holds (a multiple of 8)
-    // bf16 on the batched passes over a stored residual (wide rows, or a quota past the list): the
-    // level-1 pass writes the candidate lists (bin B0 and above) and k_emit_cand reads them
+    // bf16 on the batched passes over a stored residual (a quota past the list): the level-1 pass
+    // writes the candidate lists (bin B0 and above) and k_emit_cand reads them
     bool cand_rin;
     bool trim;
     int64_t n_list_blocks;
@@ -3251,7 +3251,8 @@ Plan make_plan_rows(const StacrSaveArgs &a)
 // ntw threads with mvw vectors each and stores the residual; the later passes run on the batched
 // kernels over that residual viewed as f * rows rows of d / f <= 2048 columns (row-major, so the
 // flat indices are the same; chunks are f * chunk_rows such rows, so the chunks are the same) at
-// rank 8 (they read neither the basis nor C).
+// rank 8 (they read neither the basis nor C).  (bf16 with a residual and a quota inside the lists:
+// k_proj_cand_w in its place, and the later passes on its lists, see make_plan_base.)
 Plan make_plan_wide(const StacrSaveArgs &a)
 {
     Plan p = make_plan_rows(a);
@@ -3514,7 +3515,8 @@ int launch_typed(const StacrSaveArgs &a, const Plan &p, char *ws, const size_t *
                                               off[WS_HIST]) / sizeof(uint32_t)) : 0;
     // the entry census (bf16 candidate passes without a trim, blocks of whole workgroups): its
     // counts are cleared here and filled by the emission pass.  Lists from X: rows of <= 2048
-    // features; lists from the stored residual: also rows split into segments (<= 4096 features)
+    // features, wide rows of <= 4096; lists from the stored residual: also rows split into segments
+    // (<= 4096 features)
     const int64_t csegs = p.g.d > 0 && a.feats % p.g.d == 0 ? a.feats / p.g.d : 0;
     const bool census = a.census && (p.cand || p.cand_rin) && !p.trim && csegs >= 1 &&
                         (kCensusRows * csegs) % p.g.rows_per_wg == 0 && p.g.rows % csegs == 0 &&
@@ -3560,8 +3562,8 @@ int launch_typed(const StacrSaveArgs &a, const Plan &p, char *ws, const size_t *
                 }
                 if constexpr (kRin) {
                     if (!p.wcand) {
-                    const int rc = launch_wide_pass1<DT>(a, p, x, qp, coeff_out, hist, maxkey, resid ? 1 : 0, coeff_in, rbuf, coarse);
-                    if (rc) return rc;
+                        const int rc = launch_wide_pass1<DT>(a, p, x, qp, coeff_out, hist, maxkey, resid ? 1 : 0, coeff_in, rbuf, coarse);
+                        if (rc) return rc;
                     }
                 } else {
                     return stacr_fail(STACR_ERR_INVALID, "stacr_save: wide rows outside 16-bit activations");
@@ -3596,7 +3598,7 @@ int launch_typed(const StacrSaveArgs &a, const Plan &p, char *ws, const size_t *
                 using L2 = std::integral_constant<int, 2>;
                 using H8 = std::integral_constant<int, kHistCopies>;
                 using H1 = std::integral_constant<int, 1>;
-                auto refine_cand = [&](auto hc) {
+                auto refine_lists = [&](auto hc) {
                     if constexpr (kCandOk)
                         stacr_launch("k_refine_lists", s, [&] {
                             const auto k = few ? k_refine_lists<decltype(hc)::value, 1> : k_refine_lists<decltype(hc)::value, kListWaves>;
@@ -3604,7 +3606,7 @@ int launch_typed(const StacrSaveArgs &a, const Plan &p, char *ws, const size_t *
                                                                                maxkey, fold, coarse, p.list_cap, cidx, cval, cmeta);
                         });
                 };
-                auto refine_lists = [&](auto hc) {
+                auto refine_stored = [&](auto hc) {
                     if constexpr (kCandOk && kRin)
                         stacr_launch("k_refine_hist_b", s, [&] {
                             k_refine_hist_b<DT, R, V, decltype(hc)::value, true, 1, true><<<nwg, kBlock, 0, s>>>(
@@ -3613,11 +3615,11 @@ int launch_typed(const StacrSaveArgs &a, const Plan &p, char *ws, const size_t *
                         });
                 };
                 if (lvl == 1 && cand) {
-                    if (hc8) refine_cand(H8{});
-                    else refine_cand(H1{});
-                } else if (lvl == 1 && cand_rin) {
                     if (hc8) refine_lists(H8{});
                     else refine_lists(H1{});
+                } else if (lvl == 1 && cand_rin) {
+                    if (hc8) refine_stored(H8{});
+                    else refine_stored(H1{});
                 } else if (lvl == 1) {
                     if (hc8) refine(H8{}, L1{});
                     else refine(H1{}, L1{});

@@ -2355,11 +2355,12 @@ __device__ __forceinline__ CandVals list_vals(const uint16_t *__restrict__ cand_
 // a thread and four columns' words at a time (57 registers where the other form has 140; 131072 x 1024, rank 16,
 // in chunks: level 1 30 and 45 us; 32768 x 2048 fitted: 30 and 27 us).
 // s_c holds C as [row of the list][R], zero past the rank; every thread must call both.
+template <int NT>
 __device__ __forceinline__ void list_stage_c(const SaveGeom &g, int R, const uint16_t *__restrict__ coeff, int64_t row0,
                                              int64_t row_end, float *__restrict__ s_c)
 {
     __syncthreads();  // (the list before may still be read)
-    for (int e = threadIdx.x; e < (int)(row_end - row0) * R; e += kBlock) {
+    for (int e = threadIdx.x; e < (int)(row_end - row0) * R; e += NT) {
         const int i = e / R, j = e - i * R;
         s_c[e] = j < g.rank ? bf16_bits_to_f(coeff[(row0 + i) * g.rank + j]) : 0.f;
     }
@@ -2394,7 +2395,7 @@ __device__ __forceinline__ void list_residual(uint4 x, const float (&p)[8], uint
 }
 
 // round(v, n_vec, w): the packed residuals of vectors v and v + 1 (of n_vec; those past it hold anything).
-template <int R, typename Round>
+template <int R, int NT, typename Round>
 __device__ __forceinline__ void list_rounds_r(const SaveGeom &g, const uint16_t *__restrict__ x,
                                               const uint16_t *__restrict__ qph, const float *__restrict__ s_c, int64_t row0,
                                               int64_t row_end, Round &round)
@@ -2406,7 +2407,7 @@ __device__ __forceinline__ void list_rounds_r(const SaveGeom &g, const uint16_t 
 #pragma unroll
     for (int i = 0; i < 2; ++i) nx[i] = xs[min(v + i, n_vec - 1)];
 #pragma unroll 1
-    for (int v0 = 0; v0 < n_vec; v0 += 2 * kBlock, v += 2 * kBlock) {
+    for (int v0 = 0; v0 < n_vec; v0 += 2 * NT, v += 2 * NT) {
         const int vc = min(v, n_vec - 1), row = vc / per_row, col = vc - row * per_row;
         const bool wrap = col + 1 == per_row;  // the second vector begins the next row (past the last row: not used)
         const uint16_t *q[2] = {qph + 8 * col, qph + (wrap ? 0 : 8 * (col + 1))};
@@ -2419,7 +2420,7 @@ __device__ __forceinline__ void list_rounds_r(const SaveGeom &g, const uint16_t 
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
             xc[i] = nx[i];
-            nx[i] = xs[min(v + 2 * kBlock + i, n_vec - 1)];
+            nx[i] = xs[min(v + 2 * NT + i, n_vec - 1)];
         }
         float p[2][8] = {};
         uint32_t w[2][4];
@@ -2434,14 +2435,14 @@ __device__ __forceinline__ void list_rounds_r(const SaveGeom &g, const uint16_t 
     }
 }
 
-template <typename Round>
+template <int NT, typename Round>
 __device__ __forceinline__ void list_rounds(const SaveGeom &g, int R, const uint16_t *__restrict__ x,
                                             const uint16_t *__restrict__ qph, const float *__restrict__ s_c, int64_t row0,
                                             int64_t row_end, Round &&round)
 {
-    if (R == 4) list_rounds_r<4>(g, x, qph, s_c, row0, row_end, round);
-    else if (R == 8) list_rounds_r<8>(g, x, qph, s_c, row0, row_end, round);
-    else list_rounds_r<16>(g, x, qph, s_c, row0, row_end, round);
+    if (R == 4) list_rounds_r<4, NT>(g, x, qph, s_c, row0, row_end, round);
+    else if (R == 8) list_rounds_r<8, NT>(g, x, qph, s_c, row0, row_end, round);
+    else list_rounds_r<16, NT>(g, x, qph, s_c, row0, row_end, round);
 }
 
 // The same with one vector a thread and four basis columns at a time: round(v, n_vec, w).
@@ -2488,8 +2489,8 @@ __device__ __forceinline__ uint32_t list_word(uint4 w0, uint4 w1, int e)
 // zero) and the records of k_refine_hist_b: cum[b] for b = 0..15, and cum[16], the count above B0.  A list that
 // is not usable is recomputed and written anew with B0 as its cut, so that the emission can read it (unless it
 // holds more than the list's slots there).
-template <int HC, int LW>
-__global__ __launch_bounds__(kBlock) void k_refine_lists(SaveGeom g, int R, int64_t n_lists,
+template <int HC, int LW, int NT>
+__global__ __launch_bounds__(NT) void k_refine_lists(SaveGeom g, int R, int64_t n_lists,
                                                          const uint16_t *__restrict__ x, const float *__restrict__ qp,
                                                          const uint16_t *__restrict__ coeff,
                                                          uint32_t *__restrict__ hist, SelState *__restrict__ state,
@@ -2502,7 +2503,7 @@ __global__ __launch_bounds__(kBlock) void k_refine_lists(SaveGeom g, int R, int6
     __shared__ uint32_t s_cnt[LW][16];
     __shared__ uint32_t s_above[LW];
     __shared__ uint32_t s_redo[LW];  // the list's B0 + 1 when its workgroup recomputes it, else 0
-    __shared__ uint32_t s_wt[kWaves];
+    __shared__ uint32_t s_wt[NT / 64];
     __shared__ __align__(16) float s_c[kListC];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int64_t list_raw = (int64_t)blockIdx.x * LW + wave;
@@ -2557,7 +2558,7 @@ __global__ __launch_bounds__(kBlock) void k_refine_lists(SaveGeom g, int R, int6
         const uint32_t b0 = s_redo[l] - 1u;
         int64_t c2, r0, r1;
         wg_rows(g, list2, c2, r0, r1);
-        list_stage_c(g, R, coeff, r0, r1, s_c);
+        list_stage_c<NT>(g, R, coeff, r0, r1, s_c);
         above = 0u;
         uint32_t *ci = cand_idx + list2 * cap;
         uint16_t *cv = cand_val + list2 * cap;
@@ -2565,7 +2566,7 @@ __global__ __launch_bounds__(kBlock) void k_refine_lists(SaveGeom g, int R, int6
         // the candidates of vectors v .. v + U - 1 from their packed residuals (those past n_vec masked)
         auto take = [&](int v, uint32_t m, auto word) {
             uint32_t tot;
-            uint32_t pos = before + block_exclusive_scan((uint32_t)__popc(m), s_wt, &tot);
+            uint32_t pos = before + block_exclusive_scan<NT>((uint32_t)__popc(m), s_wt, &tot);
             for (uint32_t k = m; k != 0u; k &= k - 1u, ++pos) {  // (only the elements of bin B0 and above, one by one)
                 const int e = __builtin_ctz(k);
                 const uint32_t val = word(e);
@@ -2580,7 +2581,7 @@ __global__ __launch_bounds__(kBlock) void k_refine_lists(SaveGeom g, int R, int6
         const uint16_t *qph = reinterpret_cast<const uint16_t *>(qp + 2 * g.d * R);
         const uint32_t low = b0 << 4;
         if constexpr (LW == 1)
-            list_rounds(g, R, x, qph, s_c, r0, r1, [&](int v, int n_vec, const uint32_t (&w)[2][4]) {
+            list_rounds<NT>(g, R, x, qph, s_c, r0, r1, [&](int v, int n_vec, const uint32_t (&w)[2][4]) {
                 const uint4 w0 = make_uint4(w[0][0], w[0][1], w[0][2], w[0][3]), w1 = make_uint4(w[1][0], w[1][1], w[1][2], w[1][3]);
                 take(v, (mask_ge(w[0], low) | mask_ge(w[1], low) << 8) & (v + 1 < n_vec ? 0xffffu : v < n_vec ? 0xffu : 0u),
                      [&](int e) { return list_word(w0, w1, e); });
@@ -2800,7 +2801,7 @@ __global__ __launch_bounds__(kBlock) void k_emit_lists(
         if (s_redo[l] == 0u) continue;  // (uniform)
         int64_t c2, r0, r1;
         wg_rows(g, (int64_t)blockIdx.x * LW + l, c2, r0, r1);
-        list_stage_c(g, R, coeff, r0, r1, s_c);
+        list_stage_c<kBlock>(g, R, coeff, r0, r1, s_c);
         const uint32_t Tl = s_T[l], off = s_off[l], take = s_take[l];
         uint32_t gt_before = 0u, eq_before = 0u;
         // (the lists that level 1 could not write anew, so seldom any)
@@ -3508,6 +3509,10 @@ int launch_typed(const StacrSaveArgs &a, const Plan &p, char *ws, const size_t *
     const bool resid = a.k_total > 0;
     const int nwg = (int)p.n_wgs;
     const bool few = p.n_wgs <= kFewLists;
+    // a recomputed list in half the rounds, where it has more than one and the chip holds the workgroups (fitted
+    // basis, save: 1024 x 4096 rank 8 53.5 -> 49.7 us, 2048 x 8192 rank 16 74.1 -> 68.6, with a random basis the
+    // same; at 1024 threads 48.4 and 67.9, but 55.8 for 52.4 with a random one)
+    const bool twice = p.n_wgs <= kFewLists / 2 && p.g.rows_per_wg * p.g.d > 2 * 8 * kBlock;
     const unsigned n_list_wgs = (unsigned)(few ? p.n_wgs : (p.n_wgs + kListWaves - 1) / kListWaves);
 
     // padded basis; histograms and max key (contiguous in the layout) cleared in the same launch
@@ -3601,8 +3606,10 @@ int launch_typed(const StacrSaveArgs &a, const Plan &p, char *ws, const size_t *
                 auto refine_lists = [&](auto hc) {
                     if constexpr (kCandOk)
                         stacr_launch("k_refine_lists", s, [&] {
-                            const auto k = few ? k_refine_lists<decltype(hc)::value, 1> : k_refine_lists<decltype(hc)::value, kListWaves>;
-                            k<<<n_list_wgs, kBlock, 0, s>>>(p.g, p.Rq, p.n_wgs, x, qp, coeff, hist, state, kf, kl,
+                            constexpr int HC = decltype(hc)::value;
+                            const auto k = twice ? k_refine_lists<HC, 1, 2 * kBlock>
+                                           : few ? k_refine_lists<HC, 1, kBlock> : k_refine_lists<HC, kListWaves, kBlock>;
+                            k<<<n_list_wgs, twice ? 2 * kBlock : kBlock, 0, s>>>(p.g, p.Rq, p.n_wgs, x, qp, coeff, hist, state, kf, kl,
                                                                                maxkey, fold, coarse, p.list_cap, cidx, cval, cmeta);
                         });
                 };

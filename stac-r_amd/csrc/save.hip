@@ -2321,8 +2321,8 @@ struct CandVals {
 // One wave per list (a projection workgroup's candidates, a few hundred): these passes are a chain of
 // dependent loads and a little arithmetic, so their time is that chain's latency times the rounds of
 // waves the lists take.  A wave a list instead of a workgroup puts every list of 8192 projection workgroups
-// on the chip at once and needs no barrier (8192 lists of about 880: level 1 90 -> 15 us, emission 102 -> 22 us;
-// eight a workgroup 18 and 30 us).  Up to kFewLists lists, each has a workgroup of its own: a list that is not
+// on the chip at once and needs no barrier (the same 8192 lists of about 880 entries, a workgroup and a wave each:
+// level 1 90 and 15 us, emission 102 and 22 us; eight lists a workgroup 18 and 30 us).  Up to kFewLists lists, each has a workgroup of its own: a list that is not
 // usable is recomputed by its whole workgroup and sets the pass's time, so none should meet two, and in the
 // emission the four waves share the earlier lists' records and a long list's rounds (1024 lists of 8 x 4096, 20 of
 // them not usable: level 1 41 -> 26 us, emission 25 -> 19, with none 10.1 and 10.4, 19.3 and 17.3; 128 lists of
